@@ -570,12 +570,16 @@ static bool enqueue_step(Handle* h, hipStream_t st, Recorder* rec = nullptr) {
     }
   }
   if (h->out_mode == OUT_GEMM) {  // output layer wider than one tile: stand-alone loss head
+    LossHead lh;
+    lh.scalars = h->scalars;
+    lh.bc_table = h->bc_table;
+    lh.bc_len = h->bc_len;
+    lh.partials = h->loss_partials;
+    lh.counter = h->counters + h->n_counters - 1;
     if (s.loss == VOLTA_LOSS_MSE)
-      VOLTA_CHECK(launch_loss_mse(h->act[n], static_cast<const float*>(h->target), h->delta[n - 1], B * Ln,
-                                  h->scalars, h->bc_table, h->bc_len, st));
+      VOLTA_CHECK(launch_loss_mse(h->act[n], static_cast<const float*>(h->target), h->delta[n - 1], B, Ln, lh, st));
     else
-      VOLTA_CHECK(launch_loss_ce(h->act[n], static_cast<const int32_t*>(h->target), h->delta[n - 1], B, Ln,
-                                 h->scalars, h->bc_table, h->bc_len, st));
+      VOLTA_CHECK(launch_loss_ce(h->act[n], static_cast<const int32_t*>(h->target), h->delta[n - 1], B, Ln, lh, st));
     VOLTA_CHECK(mark(rec, "loss", 0.0, 12.0 * B * Ln));
   }
   // Backward (:819-993).  dX_i reads W_i before dW_i updates it in place,
@@ -1053,7 +1057,8 @@ static bool build(Handle* h) {
   if (ws_floats) req((void**)&h->gemm_ws, ws_floats * 4);
   req((void**)&h->counters, (size_t)h->n_counters * sizeof(unsigned));
   req((void**)&h->loss_partials,
-      (size_t)std::max({(B + 63) / 64, out_layer_blocks(B), out_layer_dx_blocks(B)}) * 4);
+      (size_t)std::max({(B + 63) / 64, out_layer_blocks(B), out_layer_dx_blocks(B),
+                        h->out_mode == OUT_GEMM ? loss_head_blocks(s.loss, B, Ln) : 1}) * 4);
   size_t total = 0;
   for (auto& r : reqs) total += r.bytes;
   h->arena_bytes = total;

@@ -21,10 +21,24 @@ struct SegTable {
   float wd[kMaxSegments];       // weight decay applied to this segment
 };
 
-hipError_t launch_loss_mse(const float* yhat, const float* y, float* delta, int nt, DevScalars* sc,
-                           const float2* bc_table, int bc_len, hipStream_t st);
-hipError_t launch_loss_ce(const float* z, const int32_t* labels, float* delta, int B, int C,
-                          DevScalars* sc, const float2* bc_table, int bc_len, hipStream_t st);
+// What a stand-alone loss head needs beside its operands: where the step's
+// loss goes, and for more than one block their partial sums (one float per
+// block, loss_head_blocks of them) and an arrival counter (zero between
+// launches).
+struct LossHead {
+  DevScalars* scalars = nullptr;
+  const float2* bc_table = nullptr;  // Adam bias-correction table (null without Adam)
+  int bc_len = 0;
+  float* partials = nullptr;
+  unsigned* counter = nullptr;
+};
+constexpr int kLossMaxBlocks = 1024;
+int loss_head_blocks(int loss, int B, int C);
+// delta [B x C] and the step's loss from z / yhat [B x C].
+hipError_t launch_loss_mse(const float* yhat, const float* y, float* delta, int B, int C, const LossHead& h,
+                           hipStream_t st);
+hipError_t launch_loss_ce(const float* z, const int32_t* labels, float* delta, int B, int C, const LossHead& h,
+                          hipStream_t st);
 hipError_t launch_adam(float* w, float* m, float* v, const float* g, const SegTable& segs,
                        int64_t total, const DevScalars* sc, float b1, float b2, float eps,
                        hipStream_t st);

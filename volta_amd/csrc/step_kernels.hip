@@ -5,39 +5,86 @@
 // association order and no floating-point atomics.
 #include "step_kernels.h"
 
+#include <algorithm>
+
 namespace volta {
 
+// The stand-alone loss heads: the output layer's logits are in memory, the
+// rows (CE) or elements (MSE) are spread over the chip, and the step's loss is
+// formed by whichever block finishes last.
+//
+// A block leaves its loss sum in partials[block] and takes the ticket; the
+// block that arrives last adds the partials (thread t: blocks t, t + 256, ...
+// in order, then a fixed butterfly and the waves in order), so the sum does
+// not depend on the arrival order.  The partials are stored and read at agent
+// scope, past the XCDs' L2s, and a store has completed (vmcnt 0) before its
+// block takes the ticket: only the partials cross between blocks, so nothing
+// else of the L2s is written back or invalidated (an agent-scope fence per
+// block would do that).
+constexpr int kLossThreads = 256;
+constexpr int kLossWaves = kLossThreads / kWave;
+
 // Block-wide sum with a fixed order: butterfly inside each wave, then wave
-// partials added in wave order by thread 0.  Result valid in thread 0.
-template <int THREADS>
+// partials added in wave order.  Result valid in thread 0.
 __device__ __forceinline__ float block_sum_fixed(float v, float* lds) {
   v = wave_sum(v);
   const int wave = threadIdx.x >> 6;
+  __syncthreads();  // earlier readers of lds are done
   if ((threadIdx.x & 63) == 0) lds[wave] = v;
   __syncthreads();
-  float s = 0.0f;
-  if (threadIdx.x == 0) {
-    s = lds[0];
-    for (int w = 1; w < THREADS / kWave; ++w) s = s + lds[w];
-  }
+  float s = lds[0];
+#pragma unroll
+  for (int w = 1; w < kLossWaves; ++w) s = s + lds[w];
   return s;
 }
 
+// The block's sum `s` (thread 0) into the step's loss: sum / denom.
+__device__ __forceinline__ void loss_finish(float s, float denom, const LossHead& h, float* lds) {
+  if (gridDim.x == 1) {
+    if (threadIdx.x == 0) step_epilogue(h.scalars, h.bc_table, h.bc_len, s / denom);
+    return;
+  }
+  __shared__ unsigned last;
+  if (threadIdx.x == 0) {
+    __hip_atomic_store(h.partials + blockIdx.x, s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    last = __hip_atomic_fetch_add(h.counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1u;
+  }
+  __syncthreads();
+  if (!last) return;  // block-uniform
+  float t = 0.0f;
+  for (unsigned b = threadIdx.x; b < gridDim.x; b += kLossThreads)
+    t = t + __hip_atomic_load(h.partials + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  t = block_sum_fixed(t, lds);
+  if (threadIdx.x == 0) {
+    step_epilogue(h.scalars, h.bc_table, h.bc_len, t / denom);
+    *h.counter = 0u;  // for the next step's launch
+  }
+}
+
 // MSE head (mlp_train_rust_codegen.rs:792-798): d = yhat - y,
-// loss = sum(d^2)/nt, delta = 2*d/nt with nt = B*Ln.
-__global__ void __launch_bounds__(1024)
-loss_mse_kernel(const float* __restrict__ yhat, const float* __restrict__ y, float* __restrict__ delta,
-                int nt, DevScalars* sc, const float2* bc_table, int bc_len) {
-  __shared__ float lds[1024 / kWave];
+// loss = sum(d^2)/nt, delta = 2*d/nt with nt = B*Ln.  Block b takes elements
+// [b * per, (b + 1) * per).
+__global__ void __launch_bounds__(kLossThreads)
+loss_mse_kernel(const float* __restrict__ yhat, const float* __restrict__ y, float* __restrict__ delta, int nt,
+                int per, LossHead h) {
+  __shared__ float lds[kLossWaves];
   const float ntf = (float)nt;
+  const int64_t lo = (int64_t)blockIdx.x * per;
+  const int64_t hi = lo + per < nt ? lo + per : nt;
   float acc = 0.0f;
-  for (int k = threadIdx.x; k < nt; k += 1024) {
+  for (int64_t k = lo + threadIdx.x; k < hi; k += kLossThreads) {
     const float d = yhat[k] - y[k];
     acc = acc + d * d;
     delta[k] = 2.0f * d / ntf;
   }
-  const float s = block_sum_fixed<1024>(acc, lds);
-  if (threadIdx.x == 0) step_epilogue(sc, bc_table, bc_len, s / ntf);
+  loss_finish(block_sum_fixed(acc, lds), ntf, h, lds);
+}
+
+__device__ __forceinline__ float wave_max(float v) {
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, kWave));
+  return v;
 }
 
 // Softmax cross-entropy head with integer labels.
@@ -45,40 +92,73 @@ loss_mse_kernel(const float* __restrict__ yhat, const float* __restrict__ y, flo
 // lse = max + ln(sum), sample loss -(z_label - lse); mean over B.
 // Gradient (autograd.rs:467-534): (softmax(z) - onehot) / B with
 // softmax = exp(z - max) / sum (kernels/reduce.rs:203-213).
-// One thread per row; an out-of-range label raises BAD_ARGUMENT and makes
+// One wave per row, rows_per_wave of them in turn: lane l takes columns l,
+// l + 64, ... (a row of up to 64 * PER columns stays in registers with its
+// exponentials; PER = 0 reads it again from the cache), the row's maximum and
+// exp sum by butterflies.  An out-of-range label raises BAD_ARGUMENT and makes
 // that row's loss NaN (it is never used as an index).
-__global__ void __launch_bounds__(1024)
-loss_ce_kernel(const float* __restrict__ z, const int32_t* __restrict__ labels,
-               float* __restrict__ delta, int B, int C, DevScalars* sc, const float2* bc_table,
-               int bc_len) {
-  __shared__ float lds[1024 / kWave];
+// Latency bound: one load round, two butterflies and one store per row.  One
+// thread per row in a single block took 452 us of the 2961 us step of
+// 1500-3000-3000-1000-100 at B=2000 (2505 us a step with this), and 42 us of
+// the 61 us step of 800-384-100 at B=1 (24 us).
+template <int PER>
+__global__ void __launch_bounds__(kLossThreads)
+loss_ce_kernel(const float* __restrict__ z, const int32_t* __restrict__ labels, float* __restrict__ delta, int B,
+               int C, int rows_per_wave, LossHead h) {
+  __shared__ float lds[kLossWaves];
+  constexpr int R = PER > 0 ? PER : 1;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const float bf = (float)B;
-  float acc = 0.0f;
+  float acc = 0.0f;  // lane 0: the wave's row losses in row order
   bool bad = false;
-  for (int b = threadIdx.x; b < B; b += 1024) {
+  const int row0 = (blockIdx.x * kLossWaves + wave) * rows_per_wave;
+  for (int b = row0; b < min(B, row0 + rows_per_wave); ++b) {  // wave-uniform
     const float* zr = z + (size_t)b * C;
     float* dr = delta + (size_t)b * C;
     const int lab = labels[b];
-    float mx = -INFINITY;
-    for (int j = 0; j < C; ++j) mx = fmaxf(mx, zr[j]);
-    float sum = 0.0f;
-    for (int j = 0; j < C; ++j) sum = sum + expf(zr[j] - mx);
-    const float lse = mx + logf(sum);
-    float sample = __builtin_nanf("");
-    for (int j = 0; j < C; ++j) {
-      const bool on = j == lab;
-      if (on) sample = -(zr[j] - lse);
-      dr[j] = (expf(zr[j] - mx) / sum - (on ? 1.0f : 0.0f)) / bf;
+    const bool ok = lab >= 0 && lab < C;
+    const float zl = zr[ok ? lab : 0];
+    float v[R];
+    float mx = -INFINITY, sum = 0.0f;
+    if constexpr (PER > 0) {
+#pragma unroll
+      for (int i = 0; i < R; ++i) v[i] = zr[min(lane + 64 * i, C - 1)];
+#pragma unroll
+      for (int i = 0; i < R; ++i) mx = fmaxf(mx, v[i]);  // a repeated last column changes no maximum
+    } else {
+      for (int j = lane; j < C; j += 64) mx = fmaxf(mx, zr[j]);
     }
-    bad |= lab < 0 || lab >= C;
-    acc = acc + sample;
+    mx = wave_max(mx);
+    if constexpr (PER > 0) {
+#pragma unroll
+      for (int i = 0; i < R; ++i) {
+        v[i] = expf(v[i] - mx);
+        sum = lane + 64 * i < C ? sum + v[i] : sum;
+      }
+    } else {
+      for (int j = lane; j < C; j += 64) sum = sum + expf(zr[j] - mx);
+    }
+    sum = wave_sum(sum);
+    auto grad = [&](int j, float e) { dr[j] = (e / sum - (j == lab ? 1.0f : 0.0f)) / bf; };
+    if constexpr (PER > 0) {
+#pragma unroll
+      for (int i = 0; i < R; ++i)
+        if (lane + 64 * i < C) grad(lane + 64 * i, v[i]);
+    } else {
+      for (int j = lane; j < C; j += 64) grad(j, expf(zr[j] - mx));
+    }
+    acc = acc + (ok ? -(zl - (mx + logf(sum))) : __builtin_nanf(""));
+    bad |= !ok;
   }
-  const int any_bad = __syncthreads_or(bad ? 1 : 0);
-  const float s = block_sum_fixed<1024>(acc, lds);
-  if (threadIdx.x == 0) {
-    if (any_bad) atomicOr(&sc->flags, (uint32_t)VOLTA_STATUS_BAD_ARGUMENT);
-    step_epilogue(sc, bc_table, bc_len, s / bf);
-  }
+  if (bad && lane == 0) atomicOr(&h.scalars->flags, (uint32_t)VOLTA_STATUS_BAD_ARGUMENT);
+  __syncthreads();
+  if (lane == 0) lds[wave] = acc;
+  __syncthreads();
+  float s = lds[0];
+#pragma unroll
+  for (int w = 1; w < kLossWaves; ++w) s = s + lds[w];
+  __syncthreads();
+  loss_finish(s, bf, h, lds);
 }
 
 // Find the segment holding flat element `base` (segments are padded to
@@ -128,17 +208,46 @@ adagrad_kernel(float* __restrict__ w, float* __restrict__ G, const float* __rest
 }
 
 // ---------------------------------------------------------------------------
-hipError_t launch_loss_mse(const float* yhat, const float* y, float* delta, int nt, DevScalars* sc,
-                           const float2* bc_table, int bc_len, hipStream_t st) {
-  hipLaunchKernelGGL(loss_mse_kernel, dim3(1), dim3(1024), 0, st, yhat, y, delta, nt, sc, bc_table,
-                     bc_len);
+// Elements a block of the MSE head takes: four per thread, and more once that
+// is over kLossMaxBlocks blocks.
+static int mse_per_block(int64_t nt) {
+  const int64_t per = std::max<int64_t>(4 * kLossThreads, (nt + kLossMaxBlocks - 1) / kLossMaxBlocks);
+  return (int)((per + kLossThreads - 1) / kLossThreads * kLossThreads);
+}
+// Rows a wave of the CE head takes in turn: one, until that is over
+// kLossMaxBlocks blocks.
+static int ce_rows_per_wave(int B) {
+  return std::max(1, (B + kLossMaxBlocks * kLossWaves - 1) / (kLossMaxBlocks * kLossWaves));
+}
+
+int loss_head_blocks(int loss, int B, int C) {
+  if (loss == VOLTA_LOSS_MSE) {
+    const int per = mse_per_block((int64_t)B * C);
+    return (int)(((int64_t)B * C + per - 1) / per);
+  }
+  const int rows = kLossWaves * ce_rows_per_wave(B);
+  return (B + rows - 1) / rows;
+}
+
+hipError_t launch_loss_mse(const float* yhat, const float* y, float* delta, int B, int C, const LossHead& h,
+                           hipStream_t st) {
+  const int blocks = loss_head_blocks(VOLTA_LOSS_MSE, B, C);
+  if (blocks > 1 && (!h.partials || !h.counter)) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(loss_mse_kernel, dim3(blocks), dim3(kLossThreads), 0, st, yhat, y, delta, B * C,
+                     mse_per_block((int64_t)B * C), h);
   return hipGetLastError();
 }
 
-hipError_t launch_loss_ce(const float* z, const int32_t* labels, float* delta, int B, int C,
-                          DevScalars* sc, const float2* bc_table, int bc_len, hipStream_t st) {
-  hipLaunchKernelGGL(loss_ce_kernel, dim3(1), dim3(1024), 0, st, z, labels, delta, B, C, sc, bc_table,
-                     bc_len);
+hipError_t launch_loss_ce(const float* z, const int32_t* labels, float* delta, int B, int C, const LossHead& h,
+                          hipStream_t st) {
+  const int blocks = loss_head_blocks(VOLTA_LOSS_SOFTMAX_CE, B, C), rows = ce_rows_per_wave(B);
+  if (blocks > 1 && (!h.partials || !h.counter)) return hipErrorInvalidValue;
+  const dim3 grid(blocks), block(kLossThreads);
+  if (C <= 64) hipLaunchKernelGGL(loss_ce_kernel<1>, grid, block, 0, st, z, labels, delta, B, C, rows, h);
+  else if (C <= 128) hipLaunchKernelGGL(loss_ce_kernel<2>, grid, block, 0, st, z, labels, delta, B, C, rows, h);
+  else if (C <= 256) hipLaunchKernelGGL(loss_ce_kernel<4>, grid, block, 0, st, z, labels, delta, B, C, rows, h);
+  else if (C <= 1024) hipLaunchKernelGGL(loss_ce_kernel<16>, grid, block, 0, st, z, labels, delta, B, C, rows, h);
+  else hipLaunchKernelGGL(loss_ce_kernel<0>, grid, block, 0, st, z, labels, delta, B, C, rows, h);
   return hipGetLastError();
 }
 
