@@ -66,3 +66,47 @@ def test_wide_loss_head_special_values():
     assert np.isnan(t.loss()) and t.status() == STATUS_NONFINITE_LOSS
     np.testing.assert_array_equal(np.delete(t.debug_buffer(1, 0).reshape(B, C), 2, 0), np.delete(d0, 2, 0))
     t.close()
+
+
+# The step's inputs: a host-fed step reads them from a ring of pinned slots (or
+# one slot and a copy engine above 1 MiB), a device-fed one from any 4-byte
+# aligned address.  Both leave the resident batch and the training as a step on
+# the resident batch does, over more steps than the ring has slots.
+@pytest.mark.parametrize("L0,B,Ln,loss", [(5, 3, 3, "mse"), (1, 1, 1, "mse"), (7, 33, 10, "ce"), (64, 64, 70, "mse"),
+                                          (400, 650, 5, "ce"), (400, 700, 5, "ce"), (401, 701, 1, "mse")])
+def test_step_inputs(L0, B, Ln, loss):
+    say(f"step inputs L0={L0} B={B} {loss}")
+    lib, steps = load_hip(), 7
+    spec = MlpSpec([L0, 8, Ln], "tanh", "sgd", loss)
+    ws, bs = data.he_uniform(3, spec.sizes)
+    batches = [data.batch(40 + s, spec.sizes, B, loss) for s in range(steps)]
+    X = np.concatenate([np.zeros(1, np.float32)] + [b[0].ravel() for b in batches])  # every step's X is misaligned
+    Y = np.concatenate([np.zeros(1, batches[0][1].dtype)] + [b[1].ravel() for b in batches])
+    dx, dy = DeviceArray(X), DeviceArray(Y)
+    got = []
+    for feed in ("host", "device", "resident"):
+        t = Trainer(lib, spec, B)
+        t.set_all_params(ws, bs)
+        xb, yb = t.batch_buffers()
+        for s, (x, y) in enumerate(batches):
+            px, py = dx.ptr + 4 + 4 * s * x.size, dy.ptr + 4 + 4 * s * y.size
+            if feed == "host":
+                x, y = x.copy(), y.copy()
+                t.step(x, y, 0.05)
+                x.fill(np.nan)  # the caller's arrays are its own again
+                y.fill(0)
+            elif feed == "device":
+                assert t.step_device(px, py, 0.05) == 0
+            else:
+                assert t.sync() == 0
+                assert lib.lib.volta_hip_copy(xb, px, 4 * x.size, 3) == 0
+                assert lib.lib.volta_hip_copy(yb, py, 4 * y.size, 3) == 0
+                assert t.step_device(xb, yb, 0.05) == 0
+        np.testing.assert_array_equal(t.debug_buffer(0, 0), batches[-1][0].ravel())
+        got.append((t.loss(), *t.get_params()))
+        assert t.status() == 0
+        t.close()
+    for other in got[1:]:
+        assert got[0][0] == other[0]
+        for a, b in zip(got[0][1] + got[0][2], other[1] + other[2]):
+            np.testing.assert_array_equal(a, b)

@@ -162,10 +162,16 @@ struct Handle {
 
   // --- host side -------------------------------------------------------------
   float* h_params = nullptr;  // pinned mirror returned by get_params
-  float* h_stage_x = nullptr;   // pinned [X | gap | Y] (one allocation)
-  void* h_stage_y = nullptr;    // its Y part, stage_y_off bytes in
-  size_t stage_y_off = 0;
-  hipEvent_t stage_free = nullptr;  // staging buffers may be overwritten
+  // Pinned staging of host-fed steps, slots of [X | gap | Y]: a ring read by
+  // the step's input launch, which reports the number of the step whose slot
+  // it has read in *stage_done; or, for large inputs, one slot read by a copy
+  // engine (stage_free: it may be overwritten).
+  char* h_stage = nullptr;
+  size_t stage_bytes = 0, stage_y_off = 0;  // of one slot; of Y in it
+  int stage_slots = 1;
+  uint32_t stage_seq = 0;               // host-fed steps staged so far
+  uint32_t* stage_done = nullptr;       // pinned; written by the device
+  hipEvent_t stage_free = nullptr;
   static constexpr int kLrSlots = 64;
   float* h_lr = nullptr;
   hipEvent_t lr_ev[kLrSlots] = {};
@@ -187,7 +193,7 @@ Handle::~Handle() {
     if (e) (void)hipEventDestroy(e);
   if (stage_free) (void)hipEventDestroy(stage_free);
   if (h_params) (void)hipHostFree(h_params);
-  if (h_stage_x) (void)hipHostFree(h_stage_x);
+  if (h_stage) (void)hipHostFree(h_stage);
   if (h_lr) (void)hipHostFree(h_lr);
   if (bc_table) (void)hipFree(bc_table);
   if (infer_x) (void)hipFree(infer_x);
@@ -871,6 +877,8 @@ static float* scratch_address(int dev) {
   return g_scratch_dev[dev];
 }
 
+constexpr size_t kStageRingMax = (size_t)1 << 20;  // largest staging slot of the ring
+
 static bool build(Handle* h) {
   const volta_mlp_spec& s = h->spec;
   const int n = h->n, B = h->B;
@@ -1055,7 +1063,7 @@ static bool build(Handle* h) {
   if (h->ext_clip) req((void**)&h->clip_partials, kClipBlocks * 4);
   for (int i = 0; i < n; ++i) req((void**)&h->delta[i], (size_t)B * h->L[i + 1] * 4);
   if (ws_floats) req((void**)&h->gemm_ws, ws_floats * 4);
-  req((void**)&h->counters, (size_t)h->n_counters * sizeof(unsigned));
+  req((void**)&h->counters, (size_t)(h->n_counters + 1) * sizeof(unsigned));  // + the input launch's
   req((void**)&h->loss_partials,
       (size_t)std::max({(B + 63) / 64, out_layer_blocks(B), out_layer_dx_blocks(B),
                         h->out_mode == OUT_GEMM ? loss_head_blocks(s.loss, B, Ln) : 1}) * 4);
@@ -1073,13 +1081,17 @@ static bool build(Handle* h) {
 
   // Host side: pinned parameter mirror, input staging, lr slots.
   VOLTA_CHECK(hipHostMalloc((void**)&h->h_params, (size_t)h->flat * 4, hipHostMallocDefault));
-  // [X | gap | Y], laid out as act_0 and the targets are in the arena
+  // Staging slots [X | gap | Y], laid out as act_0 and the targets are in the
+  // arena.  Up to 1 MiB a ring that the input launch reads (four slots while
+  // they fit 256 KiB, else two): the host runs ahead of the GPU, and no copy engine has to be handed the stream and
+  // hand it back (256-512-512-256-1 at B=64: 47.4 -> 34.1 us a step,
+  // 300-1655-200-17 at B=629, 0.8 MB a step: 205 -> 196).  Past that one slot
+  // for a copy engine, whose 57 GB/s a kernel's reads of host memory do not
+  // reach (33 MB a step: 1790 us against 1920).
   h->stage_y_off = align_up((size_t)B * h->L[0] * 4, 256);
-  VOLTA_CHECK(hipHostMalloc((void**)&h->h_stage_x, h->stage_y_off + (size_t)B * std::max(h->L[n], 1) * 4,
-                            hipHostMallocDefault));
-  h->h_stage_y = reinterpret_cast<char*>(h->h_stage_x) + h->stage_y_off;
+  h->stage_bytes = align_up(h->stage_y_off + (size_t)B * std::max(h->L[n], 1) * 4, 256);
+  h->stage_slots = h->stage_bytes > kStageRingMax ? 1 : 4 * h->stage_bytes <= kStageRingMax / 4 ? 4 : 2;
   VOLTA_CHECK(hipHostMalloc((void**)&h->h_lr, Handle::kLrSlots * sizeof(float), hipHostMallocDefault));
-  VOLTA_CHECK(hipEventCreateWithFlags(&h->stage_free, hipEventDisableTiming));
   for (auto& e : h->lr_ev) VOLTA_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
 
   // Reference init: LCG Xavier-uniform W from one stream seeded 42, b = 0.
@@ -1204,17 +1216,98 @@ static bool launch_step(Handle* h) {
   return enqueue_step(h, h->stream);
 }
 
+// Wait until the device has read the staging slot of host-fed step `seq`.
+static bool stage_wait(Handle* h, uint32_t seq) {
+  for (int spin = 0; (int32_t)(__atomic_load_n(h->stage_done, __ATOMIC_ACQUIRE) - seq) < 0; ++spin) {
+    if (spin % 4096 != 4095) continue;
+    // an idle stream has run every launch; an error ends the wait
+    const hipError_t e = hipStreamQuery(h->stream);
+    if (e == hipSuccess) return true;
+    if (e != hipErrorNotReady) {
+      set_last_error(hip_msg("hipStreamQuery", e));
+      return false;
+    }
+  }
+  return true;
+}
+
+// The staging slots, on the handle's first host-fed step (a program whose
+// inputs are on the device never pins them).
+static bool stage_alloc(Handle* h) {
+  VOLTA_CHECK(hipEventCreateWithFlags(&h->stage_free, hipEventDisableTiming));
+  VOLTA_CHECK(hipHostMalloc((void**)&h->h_stage, h->stage_slots * h->stage_bytes + 256,
+                            hipHostMallocMapped | hipHostMallocCoherent));
+  h->stage_done = reinterpret_cast<uint32_t*>(h->h_stage + h->stage_slots * h->stage_bytes);
+  *h->stage_done = 0;
+  return true;
+}
+
+static InputCopy input_copy(const Handle* h, const void* X, const void* Y, size_t ybytes) {
+  InputCopy c;
+  c.x = static_cast<const uint32_t*>(X);
+  c.x_dst = reinterpret_cast<uint32_t*>(h->act[0]);
+  c.nx = X ? (size_t)h->B * h->L[0] : 0;
+  c.y = static_cast<const uint32_t*>(Y);
+  c.y_dst = static_cast<uint32_t*>(h->target);
+  c.ny = Y ? ybytes / 4 : 0;
+  return c;
+}
+
 // Stage host inputs through pinned memory so the caller may reuse X/Y at once.
 static bool stage_inputs(Handle* h, const float* X, const void* Y, size_t ybytes) {
   const size_t xbytes = (size_t)h->B * h->L[0] * 4;
-  VOLTA_CHECK(hipEventSynchronize(h->stage_free));
-  std::memcpy(h->h_stage_x, X, xbytes);
-  std::memcpy(h->h_stage_y, Y, ybytes);
-  // act_0 and the targets are adjacent in the arena as in the staging buffer
-  // (the gap is copied too): one host-to-device transfer per step
-  if (static_cast<char*>(h->target) != reinterpret_cast<char*>(h->act[0]) + h->stage_y_off) return false;
-  VOLTA_CHECK(hipMemcpyAsync(h->act[0], h->h_stage_x, h->stage_y_off + ybytes, hipMemcpyHostToDevice, h->stream));
-  VOLTA_CHECK(hipEventRecord(h->stage_free, h->stream));
+  if (!h->h_stage && !stage_alloc(h)) return false;
+  if (h->stage_slots == 1) {
+    VOLTA_CHECK(hipEventSynchronize(h->stage_free));
+    std::memcpy(h->h_stage, X, xbytes);
+    std::memcpy(h->h_stage + h->stage_y_off, Y, ybytes);
+    // act_0 and the targets are adjacent in the arena as in the slot (the gap
+    // is copied too): one transfer
+    if (static_cast<char*>(h->target) != reinterpret_cast<char*>(h->act[0]) + h->stage_y_off) return false;
+    VOLTA_CHECK(hipMemcpyAsync(h->act[0], h->h_stage, h->stage_y_off + ybytes, hipMemcpyHostToDevice, h->stream));
+    VOLTA_CHECK(hipEventRecord(h->stage_free, h->stream));
+    return true;
+  }
+  const uint32_t seq = h->stage_seq + 1;
+  // the slot's previous user, stage_slots steps ago
+  if (!stage_wait(h, seq - (uint32_t)h->stage_slots)) return false;
+  char* slot = h->h_stage + (seq % (uint32_t)h->stage_slots) * h->stage_bytes;
+  std::memcpy(slot, X, xbytes);
+  std::memcpy(slot + h->stage_y_off, Y, ybytes);
+  InputCopy c = input_copy(h, slot, slot + h->stage_y_off, ybytes);
+  c.done = h->stage_done;
+  c.seq = seq;
+  c.ticket = h->counters + h->n_counters;
+  VOLTA_CHECK(launch_input_copy(c, h->stream));
+  h->stage_seq = seq;
+  return true;
+}
+
+// Whether [p, p + bytes) lies in one allocation of this device's memory, so
+// that a kernel may read it (anything else goes through hipMemcpyAsync, which
+// checks what it is given).
+static bool device_range(const Handle* h, const void* p, size_t bytes) {
+  hipPointerAttribute_t at{};
+  hipDeviceptr_t base = nullptr;
+  size_t size = 0;
+  if (hipPointerGetAttributes(&at, p) != hipSuccess || at.type != hipMemoryTypeDevice || at.device != h->device ||
+      hipMemGetAddressRange(&base, &size, const_cast<void*>(p)) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  const char *b = static_cast<const char*>(base), *q = static_cast<const char*>(p);
+  return ((uintptr_t)p & 3) == 0 && q >= b && bytes <= size && (size_t)(q - b) <= size - bytes;
+}
+
+// Copy device inputs into the resident batch (null: already there).
+static bool load_inputs(Handle* h, const float* X, const void* Y, size_t ybytes) {
+  const size_t xbytes = (size_t)h->B * h->L[0] * 4;
+  if ((!X || device_range(h, X, xbytes)) && (!Y || device_range(h, Y, ybytes))) {
+    VOLTA_CHECK(launch_input_copy(input_copy(h, X, Y, ybytes), h->stream));
+    return true;
+  }
+  if (X) VOLTA_CHECK(hipMemcpyAsync(h->act[0], X, xbytes, hipMemcpyDeviceToDevice, h->stream));
+  if (Y) VOLTA_CHECK(hipMemcpyAsync(h->target, Y, ybytes, hipMemcpyDeviceToDevice, h->stream));
   return true;
 }
 
@@ -1304,13 +1397,8 @@ int32_t volta_train_step_device(VoltaTrainHandle* vh, const float* X, const void
     return -1;
   }
   const size_t ybytes = h->spec.loss == VOLTA_LOSS_MSE ? (size_t)h->B * h->L[h->n] * 4 : (size_t)h->B * 4;
-  bool ok = true;
-  if (X != h->act[0])
-    ok = ok && hipMemcpyAsync(h->act[0], X, (size_t)h->B * h->L[0] * 4, hipMemcpyDeviceToDevice, h->stream) ==
-                   hipSuccess;
-  if (Y != h->target)
-    ok = ok && hipMemcpyAsync(h->target, Y, ybytes, hipMemcpyDeviceToDevice, h->stream) == hipSuccess;
-  ok = ok && volta::set_lr(h, lr) && volta::launch_step(h);
+  const bool ok = volta::load_inputs(h, X != h->act[0] ? X : nullptr, Y != h->target ? Y : nullptr, ybytes) &&
+                  volta::set_lr(h, lr) && volta::launch_step(h);
   if (!ok) {
     h->status |= VOLTA_STATUS_DEVICE_ERROR;
     return -1;

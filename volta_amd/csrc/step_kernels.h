@@ -39,6 +39,24 @@ hipError_t launch_loss_mse(const float* yhat, const float* y, float* delta, int 
                            hipStream_t st);
 hipError_t launch_loss_ce(const float* z, const int32_t* labels, float* delta, int B, int C, const LossHead& h,
                           hipStream_t st);
+// A step's inputs into the resident batch by one launch: nx words of x and ny
+// words of y (either count 0: not copied), from device memory or from pinned
+// host memory.  With `done` set (pinned host memory), the launch stores `seq`
+// there once every source word has been read; `ticket` (device, zero between
+// launches) counts the blocks.
+struct InputCopy {
+  const uint32_t* x = nullptr;
+  uint32_t* x_dst = nullptr;
+  size_t nx = 0;
+  const uint32_t* y = nullptr;
+  uint32_t* y_dst = nullptr;
+  size_t ny = 0;
+  uint32_t* done = nullptr;
+  uint32_t seq = 0;
+  unsigned* ticket = nullptr;
+};
+hipError_t launch_input_copy(const InputCopy& c, hipStream_t st);
+
 hipError_t launch_adam(float* w, float* m, float* v, const float* g, const SegTable& segs,
                        int64_t total, const DevScalars* sc, float b1, float b2, float eps,
                        hipStream_t st);

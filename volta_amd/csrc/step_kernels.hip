@@ -161,6 +161,58 @@ loss_ce_kernel(const float* __restrict__ z, const int32_t* __restrict__ labels, 
   loss_finish(s, bf, h, lds);
 }
 
+// A step's inputs into the resident batch.  Blocks [0, xb) copy x, the rest y:
+// 16-byte accesses where source and destination allow them, 4-byte ones
+// otherwise and for the last words; a block's loads are all issued before its
+// first store.  One launch of a few blocks: 2 us on the queue, where a
+// hipMemcpyAsync each for x and y took 4 us of a 52 us step on the device and
+// 14 us of host time, and one from pinned host memory, on a copy engine, 20 us
+// of a 28 us step.
+template <int U>
+__device__ __forceinline__ void copy_words(const uint32_t* src, uint32_t* dst, size_t n, unsigned block,
+                                           unsigned blocks) {
+  const size_t t = (size_t)block * blockDim.x + threadIdx.x, all = (size_t)blocks * blockDim.x;
+  size_t head = 0;  // words copied four at a time
+  if ((((uintptr_t)src | (uintptr_t)dst) & 15) == 0) {
+    const size_t n4 = n / 4;
+    const uint4* s4 = reinterpret_cast<const uint4*>(src);
+    uint4* d4 = reinterpret_cast<uint4*>(dst);
+    for (size_t i = t; i < n4; i += U * all) {
+      uint4 v[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) v[u] = s4[i + u * all < n4 ? i + u * all : i];
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (i + u * all < n4) d4[i + u * all] = v[u];
+    }
+    head = n4 * 4;
+  }
+  for (size_t i = head + t; i < n; i += 4 * all) {
+    uint32_t v[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) v[u] = src[i + u * all < n ? i + u * all : i];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (i + u * all < n) dst[i + u * all] = v[u];
+  }
+}
+
+template <int U>
+__global__ void __launch_bounds__(256) input_copy_kernel(InputCopy c, int xb) {
+  if ((int)blockIdx.x < xb) copy_words<U>(c.x, c.x_dst, c.nx, blockIdx.x, xb);
+  else copy_words<U>(c.y, c.y_dst, c.ny, blockIdx.x - xb, gridDim.x - xb);
+  if (!c.done) return;
+  // every load of the block has returned (its stores took the values) once
+  // its memory counter is at zero
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  if (__hip_atomic_fetch_add(c.ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1u) {
+    __hip_atomic_store(c.ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(c.done, c.seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+}
+
 // Find the segment holding flat element `base` (segments are padded to
 // kSegAlign floats, so a whole block lies in one segment).
 __device__ __forceinline__ int find_segment(const SegTable& t, int64_t base) {
@@ -248,6 +300,20 @@ hipError_t launch_loss_ce(const float* z, const int32_t* labels, float* delta, i
   else if (C <= 256) hipLaunchKernelGGL(loss_ce_kernel<4>, grid, block, 0, st, z, labels, delta, B, C, rows, h);
   else if (C <= 1024) hipLaunchKernelGGL(loss_ce_kernel<16>, grid, block, 0, st, z, labels, delta, B, C, rows, h);
   else hipLaunchKernelGGL(loss_ce_kernel<0>, grid, block, 0, st, z, labels, delta, B, C, rows, h);
+  return hipGetLastError();
+}
+
+hipError_t launch_input_copy(const InputCopy& c, hipStream_t st) {
+  if (!c.nx && !c.ny) return hipSuccess;
+  if ((c.nx && (!c.x || !c.x_dst)) || (c.ny && (!c.y || !c.y_dst)) || (c.done && !c.ticket))
+    return hipErrorInvalidValue;
+  // four words per thread; from a megaword on 16, over at most 2048 blocks
+  const bool big = c.nx + c.ny > ((size_t)1 << 20);
+  const size_t per = big ? 256 * 16 : 256 * 4;
+  auto blocks = [&](size_t n) { return (int)std::min<size_t>((n + per - 1) / per, 2048); };
+  const int xb = blocks(c.nx), yb = blocks(c.ny);
+  if (big) hipLaunchKernelGGL(input_copy_kernel<4>, dim3(xb + yb), dim3(256), 0, st, c, xb);
+  else hipLaunchKernelGGL(input_copy_kernel<1>, dim3(xb + yb), dim3(256), 0, st, c, xb);
   return hipGetLastError();
 }
 
