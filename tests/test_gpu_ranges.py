@@ -110,3 +110,17 @@ def test_step_inputs(L0, B, Ln, loss):
         assert got[0][0] == other[0]
         for a, b in zip(got[0][1] + got[0][2], other[1] + other[2]):
             np.testing.assert_array_equal(a, b)
+
+
+# The output layer of up to 64 columns on 16-row strips (one, two and four
+# column tiles; strips, K ranges and dX columns with remainders; the strips'
+# loss by ticket, by the dW group and by the outer-product dX launch).
+@pytest.mark.parametrize("loss,K,N,B", [("ce", 19, 10, 1), ("mse", 1, 2, 17), ("mse", 130, 4, 16), ("ce", 1088, 16, 33),
+                                        ("ce", 300, 17, 5), ("mse", 64, 33, 40), ("ce", 129, 64, 256),
+                                        ("ce", 3100, 10, 256), ("mse", 50, 3, 257), ("ce", 67, 16, 1025),
+                                        ("ce", 48, 40, 513), ("mse", 36, 1, 300)])
+@pytest.mark.parametrize("extras", [False, True])
+def test_output_strips(loss, K, N, B, extras):
+    say(f"output strips {loss} K={K} N={N} B={B} extras={extras}")
+    kw = dict(layernorm=True, clip_grad=0.5) if extras else {}
+    against_oracle(MlpSpec([8, K, N], "tanh", "sgd", loss, **kw), B)

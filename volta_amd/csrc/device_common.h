@@ -183,6 +183,23 @@ __device__ __forceinline__ void step_finish(DevScalars* sc, const StepNext& s, b
   }
 }
 
+// A block's partial sum handed to whichever block of the launch finishes last
+// (one thread per block calls it, once): stores it in partials[block] and
+// takes the ticket; true in the last block.  The partials are stored and read
+// at agent scope, past the XCDs' L2s, and a store has completed (vmcnt 0)
+// before its block takes the ticket: only the partials cross between blocks,
+// so nothing else of the L2s is written back or invalidated, as an agent-scope
+// fence per block would.
+__device__ __forceinline__ bool publish_partial(float* partials, unsigned* counter, unsigned block, unsigned blocks,
+                                                float s) {
+  __hip_atomic_store(partials + block, s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  return __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == blocks - 1u;
+}
+__device__ __forceinline__ float published_partial(const float* partials, unsigned block) {
+  return __hip_atomic_load(partials + block, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // Fixed-order wavefront sum (butterfly over 64 lanes).  Every lane ends with
 // the same value and the association order depends only on lane indices,
 // so results are bit-identical run to run.

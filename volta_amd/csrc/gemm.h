@@ -22,8 +22,6 @@ enum EpiKind {
   EPI_BIAS_ACT = 1,  // pre = acc + bias; out = f(pre)     (f = identity for the output layer)
   EPI_DX_ACT = 2,    // out = acc * f'(aux_pre, aux_act)
   EPI_DW_OPT = 3,    // acc is dW: optimizer update of W (and of b from the fused column sums)
-  EPI_LOSS = 4,      // output layer + loss head: out = acc + bias, delta, loss
-  EPI_ROWS = 5,      // small-M tile only: acc + bias into the workgroup's LDS rows (the output head)
 };
 
 struct EpiArgs {
@@ -32,7 +30,7 @@ struct EpiArgs {
   int ldc;
   float* out;               // result; for EPI_DW_OPT the weights W_i (updated in place)
   float* pre;               // EPI_BIAS_ACT: where to keep the pre-activation (may be null)
-  const float* bias;        // EPI_BIAS_ACT / EPI_LOSS
+  const float* bias;        // EPI_BIAS_ACT
   const float* aux_act;     // EPI_DX_ACT: activation output of the layer below
   const float* aux_pre;     // EPI_DX_ACT: its pre-activation (null when not kept)
   DevScalars* scalars;      // lr, bias corrections, loss, flags
@@ -49,17 +47,6 @@ struct EpiArgs {
   float* bm;                // state for b_i
   float* bv;
   float* bgrad;             // optional copy of db_i, may be null
-
-  // EPI_LOSS
-  int loss;                 // enum volta_loss
-  const float* y;           // MSE targets [M x N]
-  const int32_t* labels;    // CE labels [M]
-  float* delta;             // seed gradient [M x N]
-  float* loss_partials;     // one float per M-tile
-  unsigned* loss_counter;   // arrival counter (zero between launches)
-  int loss_tiles;           // number of M-tiles
-  const float2* bc_table;   // Adam bias-correction table (null without Adam)
-  int bc_len;
 };
 
 struct GemmArgs {
@@ -144,16 +131,6 @@ bool khalves_supported(const GemmPlan& p, const GemmArgs& a, int k_half);
 hipError_t launch_smallm_khalves(const GemmPlan& p, const GemmArgs& a, float* planes, int k_half, hipStream_t st);
 bool planes_supported(const GemmPlan& p, const GemmArgs& a, const PlaneArgs& pa);
 hipError_t launch_smallm_planes(const GemmPlan& p, const GemmArgs& a, const PlaneArgs& pa, hipStream_t st);
-// The narrow output layer of a large batch (L_n <= 16, more rows than the
-// one-launch output kernels take) on 16-wave small-M tiles, one per 16-row
-// strip: z = act_{n-1} W + b on MFMA, then the loss head per row
-// (head_row: z, delta_{n-1}, the row loss); each workgroup stores its rows'
-// loss sum in row order to o.partials[strip], block 0 advances the step
-// counter, and a later launch adds the partials (the outer-product dX_{n-1}
-// launch, LossDefer).  `a` carries A = act_{n-1}, B = W, M = B, N = L_n,
-// K = L_{n-1} and the bias (a.epi.bias).
-bool out_head_gemm_supported(const GemmArgs& a, const OutLayerArgs& o);
-hipError_t launch_smallm_out_head(const GemmArgs& a, const OutLayerArgs& o, hipStream_t st);
 bool tail_supported(const GemmPlan& p, const GemmArgs& a, const OutLayerArgs& o);
 hipError_t launch_smallm_tail(const GemmPlan& p, const GemmArgs& a, const OutLayerArgs& o, hipStream_t st);
 bool fwd_head_supported(const GemmPlan& p, const GemmArgs& a, const OutLayerArgs& o, int n_counters);

@@ -1,7 +1,7 @@
 // fp32 GEMM family on CDNA4 fp32 MFMA (v_mfma_f32_32x32x2_f32), with the
 // step's other work fused into the epilogue: bias + activation (forward),
 // activation derivative (dX), bias-gradient column sums + optimizer update
-// (dW), and the loss head (output layer).
+// (dW).
 //
 //   C[M x N] = sum_k A(m,k) * B(k,n)
 //
@@ -458,75 +458,6 @@ __device__ __forceinline__ void apply_bias_update(const EpiArgs& e, int n, int N
   }
 }
 
-// Output layer + loss head on a staged tile (z[mm][nn] = acc + bias, one
-// thread per row).  MSE (:792-798): d = z - y, loss += d^2, delta = 2d/nt.
-// Softmax-CE (interpreter.rs:762-812, autograd.rs:467-534): row max,
-// sum exp(z - max), lse, sample loss -(z_label - lse), delta = (p - onehot)/B.
-// Returns the row's loss contribution; raises BAD_ARGUMENT for a label
-// outside [0, N) (it is never used as an index).
-__device__ __forceinline__ float loss_row(const EpiArgs& e, const float* z, int m, int N, int M) {
-  float* out = e.out + (size_t)m * N;
-  float* d = e.delta + (size_t)m * N;
-  for (int j = 0; j < N; ++j) out[j] = z[j];
-  if (e.loss == VOLTA_LOSS_MSE) {
-    const float nt = (float)(M * N);
-    const float* y = e.y + (size_t)m * N;
-    float acc = 0.0f;
-    for (int j = 0; j < N; ++j) {
-      const float dj = z[j] - y[j];
-      acc = acc + dj * dj;
-      d[j] = 2.0f * dj / nt;
-    }
-    return acc;
-  }
-  const float bf = (float)M;
-  const int lab = e.labels[m];
-  float mx = -INFINITY;
-  for (int j = 0; j < N; ++j) mx = fmaxf(mx, z[j]);
-  float sum = 0.0f;
-  for (int j = 0; j < N; ++j) sum = sum + expf(z[j] - mx);
-  const float lse = mx + logf(sum);
-  float sample = __builtin_nanf("");
-  for (int j = 0; j < N; ++j) {
-    const bool on = j == lab;
-    if (on) sample = -(z[j] - lse);
-    d[j] = (expf(z[j] - mx) / sum - (on ? 1.0f : 0.0f)) / bf;
-  }
-  if (lab < 0 || lab >= N) atomicOr(&e.scalars->flags, (uint32_t)VOLTA_STATUS_BAD_ARGUMENT);
-  return sample;
-}
-
-// Loss head for one output-layer tile staged in LDS (z[mm*ZS + nn] =
-// acc + bias, rows m0.. of the batch).  One thread per row; the tile's sum
-// goes to loss_partials[tm]; with one tile it is the total, otherwise the
-// last tile to finish adds the partials in tile order.
-template <int BM>
-__device__ __forceinline__ void loss_tile(const EpiArgs& e, const float* z, int ZS, int m0, int tm, int M, int N,
-                                          float* lds_rows) {
-  const int tid = threadIdx.x;
-  if (tid < BM) lds_rows[tid] = m0 + tid < M ? loss_row(e, z + tid * ZS, m0 + tid, N, M) : 0.0f;
-  __syncthreads();
-  if (tid == 0) {
-    float s = 0.0f;
-    for (int r = 0; r < BM && m0 + r < M; ++r) s = s + lds_rows[r];
-    const float denom = e.loss == VOLTA_LOSS_MSE ? (float)(M * N) : (float)M;
-    if (e.loss_tiles == 1) {
-      step_epilogue(e.scalars, e.bc_table, e.bc_len, s / denom);
-    } else {
-      e.loss_partials[tm] = s;
-      __threadfence();
-      const unsigned ticket = atomicAdd(e.loss_counter, 1u);
-      if (ticket == (unsigned)e.loss_tiles - 1u) {
-        __threadfence();
-        float total = 0.0f;
-        for (int t = 0; t < e.loss_tiles; ++t) total = total + e.loss_partials[t];
-        step_epilogue(e.scalars, e.bc_table, e.bc_len, total / denom);
-        *e.loss_counter = 0u;
-      }
-    }
-  }
-}
-
 // Split-K planes whose loads the last slice of a tile issues together.
 constexpr int kInkPlanes = 4;
 
@@ -554,7 +485,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& args, int bx, int by, 
   constexpr int THREADS = T::kThreads;
   using LA = LdsTile<BM, BK, A_KC>;
   using LB = LdsTile<BN, BK, B_KC>;
-  static_assert(KG == 1 || (EPI != EPI_LOSS && !INK), "K groups finish whole tiles in their own epilogue");
+  static_assert(KG == 1 || !INK, "K groups finish whole tiles in their own epilogue");
   const int grp = KG > 1 ? (int)threadIdx.x / THREADS : 0;  // workgroup-uniform per wave
   float* const lds_x = lds_a0;  // the K groups' exchange area (all operand buffers)
   auto lds_a = [&](int i) { return lds_a0 + (grp * 2 + i) * LA::kFloats; };
@@ -826,27 +757,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& args, int bx, int by, 
   }
 
   const EpiArgs& e = args.epi;
-  if constexpr (EPI == EPI_LOSS) {
-    // Output layer (N <= BN): stage z = acc + bias for the whole tile in the
-    // (now free) A buffers, then the per-row loss head.
-    static_assert(BM * (BN + 1) <= 2 * LA::kFloats, "loss staging does not fit");
-    float* z = lds_a(0);
-    constexpr int ZS = BN + 1;
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < T::TM; ++i)
-#pragma unroll
-      for (int j = 0; j < T::TN; ++j) {
-        const int nn = wn * WN + j * 32 + l32;
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const int mm = wm * WM + i * 32 + 8 * (v >> 2) + 4 * h + (v & 3);
-          if (nn < N) z[mm * ZS + nn] = acc[i][j][v] + e.bias[nn];
-        }
-      }
-    __syncthreads();
-    loss_tile<BM>(e, z, ZS, m0, tm, M, N, lds_small);
-  } else {
+  {
     // Blocks in (i, j) order, unrolled at compile time: a loop the unroller
     // gives up on (it did for 4x4 blocks of 32x32) would index the
     // accumulators at run time and put them in scratch memory.
@@ -1428,7 +1339,6 @@ struct SmallHead {
   float* dx_out = nullptr;     // delta_{n-2} [M x lda] (AH == 3: the previous layer's output), or null
   float* pre_out = nullptr;    // AH == 3: the previous layer's pre-activation [M x lda], or null
   int act = 0;                 // activation of layer n-2 (AH == 3: of the previous layer)
-  float* zrows = nullptr;      // EPI_ROWS: the tile's 16 rows of acc + bias (LDS, row stride 17)
 };
 struct SmallNoop {
   __device__ void operator()() const {}
@@ -1529,7 +1439,7 @@ __device__ __forceinline__ void smallm_tile(const GemmArgs& args, int blk, float
   const bool eok = tid < 256 && em < M && en < N;
   const size_t eidx = eok ? (size_t)em * ep.ldc + en : 0;
   float e_y = 0.0f, e_p = 0.0f;
-  if constexpr (EPI == EPI_BIAS_ACT || EPI == EPI_ROWS) e_y = ep.bias[eok ? en : 0];
+  if constexpr (EPI == EPI_BIAS_ACT) e_y = ep.bias[eok ? en : 0];
   if constexpr (EPI == EPI_DX_ACT) {
     e_y = ep.aux_act[eidx];
     e_p = ep.aux_pre ? ep.aux_pre[eidx] : e_y;
@@ -1696,8 +1606,6 @@ __device__ __forceinline__ void smallm_tile(const GemmArgs& args, int blk, float
       ep.out[eidx] = act_forward(ep.act, v);  // (:725-743)
     } else if constexpr (EPI == EPI_DX_ACT) {
       ep.out[eidx] = sum * act_derivative(ep.act, e_p, e_y);  // (:893-929)
-    } else if constexpr (EPI == EPI_ROWS) {
-      hd.zrows[i * 17 + j] = sum + e_y;  // z = act_{n-1} W + b (:792-798)
     } else {
       apply_epilogue<EPI>(ep, m, n, sum);
     }
@@ -1729,54 +1637,6 @@ gemm_smallm_stg(GemmArgs args) {
 static int smallm_stage_width(int K) {
   const int kq = (K + 255) / 256 * 16;
   return kq >= 48 ? 64 : kq == 32 ? 32 : 0;
-}
-
-// The narrow output layer of a large batch on the small-M tile (one 16-row
-// strip per workgroup, the strip's z rows in LDS), then the loss head of
-// each row by one thread (head_row: the same per-row code as the
-// wave-dot-product output kernels), the strip's loss sum in row order into
-// partials[strip], and the step counter advanced by block 0.  The loss
-// itself is formed by a later launch of the step from the partials.
-template <bool VEC>
-__global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4)))
-gemm_smallm_out_head(GemmArgs args, OutLayerArgs p) {
-  __shared__ float lds[SmallLds<16>::kFloats];
-  __shared__ float zrows[16 * 17];
-  __shared__ float row_loss[16];
-  StepNext next{};
-  if (threadIdx.x == 0 && blockIdx.x == 0) next = step_prefetch(p.scalars, p.bc_table, p.bc_len);
-  const int tid = threadIdx.x, m0 = blockIdx.x * 16;  // tiles_n == 1: workgroup b owns strip b
-  // the row's targets or label, loaded before the product
-  const int rm = min(m0 + tid, p.B - 1);
-  float y[16];
-  int lab = 0;
-  if (tid < 16) {
-#pragma unroll
-    for (int j = 0; j < 16; ++j) y[j] = p.loss == VOLTA_LOSS_MSE ? p.y[(size_t)rm * p.N + min(j, p.N - 1)] : 0.0f;
-    if (p.loss != VOLTA_LOSS_MSE) lab = p.labels[rm];
-  }
-  SmallHead hd;
-  hd.zrows = zrows;
-  smallm_tile<false, VEC, EPI_ROWS, 16>(args, blockIdx.x, lds, hd);
-  __syncthreads();
-  if (tid < 16) {
-    float z[16];
-#pragma unroll
-    for (int j = 0; j < 16; ++j) z[j] = zrows[tid * 17 + min(j, p.N - 1)];
-    row_loss[tid] = m0 + tid < p.B ? head_row<16>(p, z, y, lab, m0 + tid) : 0.0f;
-  }
-  __syncthreads();
-  if (tid == 0) {
-    const int rows = min(16, p.B - m0);
-    float s = row_loss[0];
-    for (int r = 1; r < rows; ++r) s = s + row_loss[r];
-    p.partials[blockIdx.x] = s;
-    if (blockIdx.x == 0 && p.bc_table) {
-      p.scalars->t = next.t;
-      p.scalars->bc1 = next.bc.x;
-      p.scalars->bc2 = next.bc.y;
-    }
-  }
 }
 
 // A forward product over two halves of its K (a grid of at most half a
@@ -1865,8 +1725,8 @@ gemm_smallm_head(GemmArgs args, OutLayerArgs p, unsigned* strip_counters) {
     strip_counters[tm] = 0u;
     next = step_prefetch(p.scalars, p.bc_table, p.bc_len);
   }
-  const float l0 = out_dx_row<1, false>(p, nullptr, 16 * tm + wave);
-  const float l1 = out_dx_row<1, false>(p, nullptr, 16 * tm + 8 + wave);
+  const float l0 = out_dx_row(p, 16 * tm + wave);
+  const float l1 = out_dx_row(p, 16 * tm + 8 + wave);
   if (lane == 0) {
     row_loss[wave] = l0;
     row_loss[8 + wave] = l1;
@@ -2530,7 +2390,7 @@ static hipError_t launch_epi(const GemmArgs& a, bool vec, int splits, bool ink, 
   using T = Tile<BM, BN, BK, WM, WN>;
   // K groups where their operand LDS fits the CU's 160 KB
   constexpr int kStageFloats = LdsTile<BM, BK, A_KC>::kFloats + LdsTile<BN, BK, B_KC>::kFloats;
-  if constexpr (EPI != EPI_LOSS && BK == 32) {
+  if constexpr (BK == 32) {
     if constexpr (2 * 2 * kStageFloats * 4 <= 160 * 1024) {
       if (kg == 2) return launch_kg<BM, BN, BK, WM, WN, A_KC, B_KC, EPI, 2>(a, vec, st);
     }
@@ -2564,10 +2424,6 @@ static hipError_t launch_cfg(const GemmArgs& a, int layout, bool vec, int splits
       if (k == EPI_BIAS_ACT)
         return launch_epi<BM, BN, BK, WM, WN, true, false, EPI_BIAS_ACT>(a, vec, splits, ink, st, kg);
       if (k == EPI_STORE) return launch_epi<BM, BN, BK, WM, WN, true, false, EPI_STORE>(a, vec, splits, ink, st, kg);
-      if constexpr (BM * (BN + 1) <= 2 * LdsTile<BM, BK, true>::kFloats) {
-        if (k == EPI_LOSS && kg == 1)
-          return launch_epi<BM, BN, BK, WM, WN, true, false, EPI_LOSS>(a, vec, splits, true, st);
-      }
       break;
     case GEMM_NT:
       if (k == EPI_DX_ACT) return launch_epi<BM, BN, BK, WM, WN, true, true, EPI_DX_ACT>(a, vec, splits, ink, st, kg);
@@ -2714,20 +2570,6 @@ hipError_t launch_smallm_tail(const GemmPlan& p, const GemmArgs& args_in, const 
   return hipGetLastError();
 }
 
-bool out_head_gemm_supported(const GemmArgs& a, const OutLayerArgs& o) {
-  return o.N >= 1 && o.N <= 16 && o.B == a.M && o.N == a.N && o.K == a.K && a.M > 0 && o.partials && o.scalars &&
-         o.out && o.delta && a.epi.bias && (o.loss == VOLTA_LOSS_MSE ? o.y != nullptr : o.labels != nullptr) &&
-         a.ldb == o.N && a.lda == o.K;
-}
-
-hipError_t launch_smallm_out_head(const GemmArgs& a, const OutLayerArgs& o, hipStream_t st) {
-  if (!out_head_gemm_supported(a, o)) return hipErrorInvalidValue;
-  const dim3 grid((a.M + 15) / 16);
-  if (smallm_vec_ok(a, GEMM_NN)) hipLaunchKernelGGL(gemm_smallm_out_head<true>, grid, dim3(1024), 0, st, a, o);
-  else hipLaunchKernelGGL(gemm_smallm_out_head<false>, grid, dim3(1024), 0, st, a, o);
-  return hipGetLastError();
-}
-
 bool khalves_supported(const GemmPlan& p, const GemmArgs& a, int k_half) {
   return p.tile == TILE_SMALLM && p.layout == GEMM_NN && p.splits == 1 && p.vec && a.M > 0 && a.N > 0 &&
          k_half > 0 && k_half < a.K && k_half % 16 == 0 && a.ldb % 4 == 0 && smallm_vec_ok(a, GEMM_NN);
@@ -2812,12 +2654,10 @@ hipError_t gemm_launch(const GemmPlan& p, const GemmArgs& args_in, hipStream_t s
   GemmArgs a = args_in;
   a.k_per_split = p.k_per_split;
   if (p.splits > 1 && (!a.partial || !a.counters)) return hipErrorInvalidValue;
-  if (a.epi.kind == EPI_LOSS && (p.tile == TILE_128x128 || a.N > 64)) return hipErrorInvalidValue;
   if (a.colsum_b && p.layout != GEMM_TN) return hipErrorInvalidValue;
   // the optimizer epilogue indexes W_i with 32-bit element offsets
   if (a.epi.kind == EPI_DW_OPT && (size_t)a.M * a.epi.ldc >= ((size_t)1 << 30)) return hipErrorInvalidValue;
-  // The loss head always reduces in-kernel (it needs whole rows).
-  const bool ink = p.inkernel_reduce || a.epi.kind == EPI_LOSS;
+  const bool ink = p.inkernel_reduce;
   hipError_t err;
   if (p.tile == TILE_SMALLM) {
     if (p.splits != 1) return hipErrorInvalidValue;
@@ -2870,7 +2710,7 @@ hipError_t gemm_launch(const GemmPlan& p, const GemmArgs& args_in, hipStream_t s
   }
   if (p.kgroups > 1) {
     // K groups inside the workgroup: every group's slice starts inside K
-    const bool ok = p.splits == 1 && a.epi.kind != EPI_LOSS && (p.kgroups == 2 || p.kgroups == 4) &&
+    const bool ok = p.splits == 1 && (p.kgroups == 2 || p.kgroups == 4) &&
                     (p.kgroups == 2 || (p.tile == TILE_64x64 && a.epi.kind != EPI_DW_OPT)) && (size_t)(p.kgroups - 1) * p.k_per_split < (size_t)a.K &&
                     (size_t)p.kgroups * p.k_per_split >= (size_t)a.K && p.k_per_split % 32 == 0;
     if (!ok) return hipErrorInvalidValue;

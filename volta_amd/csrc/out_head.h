@@ -1,4 +1,4 @@
-// Row-level device code of the narrow output layer (L[n] <= 16 columns),
+// Row-level device code of the one-column output layer of a small batch,
 // shared by skinny.hip's output launches and the last hidden layer's
 // forward launch that also runs the output layer (gemm.hip).
 #pragma once
@@ -10,128 +10,69 @@
 
 namespace volta {
 
-// Output rows z[g][0..N) of RG rows (rows[g], valid where rows[g] >= 0),
-// computed by a whole wave: lane l sums k = l, l+64, ... in ascending order,
-// then a fixed butterfly adds the lanes.  The k loop runs in chunks of C
-// values per lane whose activation loads (all RG rows) are issued before
-// the chunk's first multiply, so a chunk costs one memory latency.  W comes
-// from the block's LDS copy `wl` (WL) -- lane l reads row k of W, so for
-// N > 1 global loads of W would touch a cache line per lane for each of its
-// N columns -- or, for one column or a W too large to stage, from global
-// memory with the chunk's other loads.  Every global load is unconditional (clamped row and k;
-// terms outside the matrix are not added), so no branch or wait separates
-// them.
-template <int NMAX, int RG, int C, bool WL>
-__device__ __forceinline__ void wave_rows(const OutLayerArgs& p, const float* wl, const int* rows,
-                                          float (*z)[NMAX]) {
+// Output values z[g] of RG rows (rows[g], valid where rows[g] >= 0) of a
+// one-column layer, computed by a whole wave: lane l sums k = l, l+64, ... in
+// ascending order, then a fixed butterfly adds the lanes.  The k loop runs in
+// chunks of C values per lane whose loads (W and all RG rows' activations) are
+// issued before the chunk's first multiply, so a chunk costs one memory
+// latency.  Every load is unconditional (clamped row and k; terms outside the
+// matrix are not added), so no branch or wait separates them.
+template <int RG, int C>
+__device__ __forceinline__ void wave_rows(const OutLayerArgs& p, const int* rows, float (*z)[1]) {
   const int lane = threadIdx.x & 63;
-  const int K = p.K, N = p.N;
-  float acc[RG][NMAX];
+  const int K = p.K;
+  float acc[RG];
 #pragma unroll
-  for (int g = 0; g < RG; ++g)
-#pragma unroll
-    for (int j = 0; j < NMAX; ++j) acc[g][j] = 0.0f;
+  for (int g = 0; g < RG; ++g) acc[g] = 0.0f;
   for (int kb = 0; kb < K; kb += 64 * C) {
-    float x[RG][C], wg[WL ? 1 : C][NMAX];
+    float x[RG][C], w[C];
 #pragma unroll
     for (int c = 0; c < C; ++c) {
       const int kc = min(kb + 64 * c + lane, K - 1);
-      if constexpr (!WL) {
-#pragma unroll
-        for (int j = 0; j < NMAX; ++j) wg[c][j] = p.W[(size_t)kc * N + min(j, N - 1)];
-      }
+      w[c] = p.W[kc];
 #pragma unroll
       for (int g = 0; g < RG; ++g) x[g][c] = p.act[(size_t)(rows[g] >= 0 ? rows[g] : 0) * K + kc];
     }
 #pragma unroll
     for (int c = 0; c < C; ++c) {
-      const int kc = min(kb + 64 * c + lane, K - 1);
-      float wv[NMAX];
-#pragma unroll
-      for (int j = 0; j < NMAX; ++j) wv[j] = WL ? wl[kc * N + min(j, N - 1)] : wg[WL ? 0 : c][j];
 #pragma unroll
       for (int g = 0; g < RG; ++g) {
-        const bool in = kb + 64 * c + lane < K && rows[g] >= 0;
-#pragma unroll
-        for (int j = 0; j < NMAX; ++j) {
-          const float t = acc[g][j] + x[g][c] * wv[j];
-          acc[g][j] = in && j < N ? t : acc[g][j];
-        }
+        const float t = acc[g] + x[g][c] * w[c];
+        acc[g] = kb + 64 * c + lane < K && rows[g] >= 0 ? t : acc[g];
       }
     }
   }
 #pragma unroll
-  for (int g = 0; g < RG; ++g)
-#pragma unroll
-    for (int j = 0; j < NMAX; ++j) z[g][j] = wave_sum(acc[g][j]);
+  for (int g = 0; g < RG; ++g) z[g][0] = wave_sum(acc[g]);
 }
 
-// Loss head of one row (same definitions as the MFMA path's loss epilogue):
-// MSE (:792-798) d = z - y, loss += d^2, delta = 2d/nt; softmax-CE
-// (interpreter.rs:762-812, autograd.rs:467-534).  head_delta forms the
-// row's deltas and returns its loss without storing anything, so every lane
-// of a wave can hold the deltas; head_row also stores z and the deltas.
-// `y` holds the row's targets (MSE), `lab` its label (CE), both loaded
-// before z was computed.  (Loops run to NMAX with a j < N guard so z stays
-// in registers.)
-template <int NMAX>
+// Loss head of one row of a one-column layer: MSE (:792-798) d = z - y,
+// loss += d^2, delta = 2d/nt; softmax-CE of one class (interpreter.rs:762-812,
+// autograd.rs:467-534).  head_delta forms the row's delta and returns its loss
+// without storing anything, so every lane of a wave can hold the delta;
+// head_row also stores z and the delta.  `y` holds the row's target (MSE),
+// `lab` its label (CE), both loaded before z was computed.
 __device__ __forceinline__ float head_delta(const OutLayerArgs& p, const float* z, const float* y, int lab,
                                             float* d) {
-  const int N = p.N;
   if (p.loss == VOLTA_LOSS_MSE) {
-    const float nt = (float)(p.B * N);
-    float acc = 0.0f;
-#pragma unroll
-    for (int j = 0; j < NMAX; ++j) {
-      if (j < N) {
-        const float dj = z[j] - y[j];
-        acc = acc + dj * dj;
-        d[j] = 2.0f * dj / nt;
-      } else {
-        d[j] = 0.0f;
-      }
-    }
-    return acc;
+    const float dj = z[0] - y[0];
+    d[0] = 2.0f * dj / (float)p.B;
+    return 0.0f + dj * dj;
   }
-  const float bf = (float)p.B;
-  float mx = -INFINITY;
-#pragma unroll
-  for (int j = 0; j < NMAX; ++j)
-    if (j < N) mx = fmaxf(mx, z[j]);
-  float sum = 0.0f;
-#pragma unroll
-  for (int j = 0; j < NMAX; ++j)
-    if (j < N) sum = sum + expf(z[j] - mx);
+  const float mx = fmaxf(-INFINITY, z[0]);
+  const float sum = 0.0f + expf(z[0] - mx);
   const float lse = mx + logf(sum);
-  float sample = __builtin_nanf("");
-#pragma unroll
-  for (int j = 0; j < NMAX; ++j) {
-    if (j < N) {
-      const bool on = j == lab;
-      if (on) sample = -(z[j] - lse);
-      d[j] = (expf(z[j] - mx) / sum - (on ? 1.0f : 0.0f)) / bf;
-    } else {
-      d[j] = 0.0f;
-    }
-  }
-  return sample;
+  const bool on = lab == 0;
+  d[0] = (expf(z[0] - mx) / sum - (on ? 1.0f : 0.0f)) / (float)p.B;
+  return on ? -(z[0] - lse) : __builtin_nanf("");
 }
 
-template <int NMAX>
 __device__ __forceinline__ float head_row(const OutLayerArgs& p, const float* z, const float* y, int lab, int m) {
-  const int N = p.N;
-  float d[NMAX];
-  const float l = head_delta<NMAX>(p, z, y, lab, d);
-  float* out = p.out + (size_t)m * N;
-  float* dd = p.delta + (size_t)m * N;
-#pragma unroll
-  for (int j = 0; j < NMAX; ++j) {
-    if (j < N) {
-      out[j] = z[j];
-      dd[j] = d[j];
-    }
-  }
-  if (p.loss != VOLTA_LOSS_MSE && (lab < 0 || lab >= N)) atomicOr(&p.scalars->flags, (uint32_t)VOLTA_STATUS_BAD_ARGUMENT);
+  float d[1];
+  const float l = head_delta(p, z, y, lab, d);
+  p.out[m] = z[0];
+  p.delta[m] = d[0];
+  if (p.loss != VOLTA_LOSS_MSE && lab != 0) atomicOr(&p.scalars->flags, (uint32_t)VOLTA_STATUS_BAD_ARGUMENT);
   return l;
 }
 
@@ -139,33 +80,28 @@ __device__ __forceinline__ float head_row(const OutLayerArgs& p, const float* z,
 constexpr int kOutDxRows = 4;
 constexpr int kOutDxMaxBlocks = (kNarrowMaxB + kOutDxRows - 1) / kOutDxRows;
 
-// Batch row m of the output layer, computed by one wave: z = act_{n-1}[m] W
-// + b, the loss head (z and delta_{n-1} stored by lane 0), and the row of
-// delta_{n-2} = (delta_{n-1} W^T) * f'(layer n-2).  Returns the row's loss
-// (0 for m >= B, whose loads are clamped and whose results are not stored).
-template <int NMAX, bool WL>
-__device__ __forceinline__ float out_dx_row(const OutLayerArgs& p, const float* w_lds, int m) {
+// Batch row m of a one-column output layer, computed by one wave: z =
+// act_{n-1}[m] W + b, the loss head (z and delta_{n-1} stored by lane 0), and
+// the row of delta_{n-2} = (delta_{n-1} W^T) * f'(layer n-2).  Returns the
+// row's loss (0 for m >= B, whose loads are clamped and whose results are not
+// stored).
+__device__ __forceinline__ float out_dx_row(const OutLayerArgs& p, int m) {
   constexpr int C = 4;
   const int lane = threadIdx.x & 63;
-  const int N = p.N, K = p.K;
+  const int K = p.K;
   const bool has = m < p.B;
   const int mc = has ? m : p.B - 1;
   const bool mse = p.loss == VOLTA_LOSS_MSE;
-  float bias[NMAX], y[NMAX];
-#pragma unroll
-  for (int j = 0; j < NMAX; ++j) {
-    bias[j] = p.bias[min(j, N - 1)];
-    y[j] = mse ? p.y[(size_t)mc * N + min(j, N - 1)] : 0.0f;
-  }
+  const float bias = p.bias[0];
+  const float y[1] = {mse ? p.y[mc] : 0.0f};
   const int lab = mse ? 0 : p.labels[mc];
   const int rows[1] = {has ? m : -1};
-  float z[1][NMAX];
-  wave_rows<NMAX, 1, C, WL>(p, w_lds, rows, z);
-#pragma unroll
-  for (int j = 0; j < NMAX; ++j) z[0][j] = z[0][j] + bias[j];
-  float d[NMAX];
-  const float row_loss = head_delta<NMAX>(p, z[0], y, lab, d);
-  if (has && lane == 0) (void)head_row<NMAX>(p, z[0], y, lab, m);
+  float z[1][1];
+  wave_rows<1, C>(p, rows, z);
+  z[0][0] = z[0][0] + bias;
+  float d[1];
+  const float row_loss = head_delta(p, z[0], y, lab, d);
+  if (has && lane == 0) (void)head_row(p, z[0], y, lab, m);
 
   // delta_{n-2} of this row
   if (has) {
@@ -173,25 +109,18 @@ __device__ __forceinline__ float out_dx_row(const OutLayerArgs& p, const float* 
     const float* pre = p.dx_pre ? p.dx_pre + (size_t)m * K : act;
     float* out = p.dx_out + (size_t)m * K;
     for (int kb = 0; kb < K; kb += 64 * C) {
-      float av[C], pv[C], wv[C][NMAX];
+      float av[C], pv[C], wv[C];
 #pragma unroll
       for (int c = 0; c < C; ++c) {
         const int kc = min(kb + 64 * c + lane, K - 1);
         av[c] = act[kc];
         pv[c] = pre[kc];
-#pragma unroll
-        for (int j = 0; j < NMAX; ++j) wv[c][j] = WL ? w_lds[kc * N + min(j, N - 1)] : p.W[(size_t)kc * N + min(j, N - 1)];
+        wv[c] = p.W[kc];
       }
 #pragma unroll
       for (int c = 0; c < C; ++c) {
-        float sacc = 0.0f;
-#pragma unroll
-        for (int j = 0; j < NMAX; ++j) {
-          const float u = sacc + d[j] * wv[c][j];
-          sacc = j < N ? u : sacc;
-        }
         const int k = kb + 64 * c + lane;
-        if (k < K) out[k] = sacc * act_derivative(p.dx_act, pv[c], av[c]);
+        if (k < K) out[k] = (0.0f + d[0] * wv[c]) * act_derivative(p.dx_act, pv[c], av[c]);
       }
     }
   }
@@ -218,12 +147,12 @@ __device__ __forceinline__ void out_head_rows(const OutLayerArgs& p, const int* 
     y[g][0] = p.y[has ? rows[g] : p.B - 1];
   }
   float z[RG][1];
-  wave_rows<1, RG, 4, false>(p, nullptr, wr, z);
+  wave_rows<RG, 4>(p, wr, z);
 #pragma unroll
   for (int g = 0; g < RG; ++g) {
     z[g][0] = z[g][0] + bias;
     float d[1];
-    const float l = head_delta<1>(p, z[g], y[g], 0, d);
+    const float l = head_delta(p, z[g], y[g], 0, d);
     if (lane == 0) {
       z_rows[g] = z[g][0];
       d_rows[g] = d[0];
@@ -249,7 +178,7 @@ __device__ __forceinline__ float out_dx_loss_sum(const float* partials, int nblo
 }
 
 __device__ __forceinline__ float out_dx_loss_denom(const OutLayerArgs& p) {
-  return p.loss == VOLTA_LOSS_MSE ? (float)(p.B * p.N) : (float)p.B;
+  return (float)p.B;  // B * 1 for MSE, B for CE
 }
 
 __device__ __forceinline__ void out_dx_finish(const OutLayerArgs& p, int nblocks, const StepNext& next) {

@@ -15,11 +15,13 @@
 //                               small-batch product on few CUs over two halves
 //                               of K into two planes, which the next forward
 //                               launch adds with the bias and activation
-//   fwd_{n-1} + loss            narrow output kernel (L_n <= 16), GEMM with the
-//                               loss head in its epilogue (<= 64), or GEMM +
-//                               loss kernel: delta_{n-1}, loss, Adam t
+//   fwd_{n-1} + loss            16-row MFMA strips with the loss head (L_n <= 64;
+//                               one column of a small batch as wave dot
+//                               products), or GEMM + loss kernel: delta_{n-1},
+//                               loss, Adam t
 //   dX_{n-1}                    outer product (L_n <= 16) or GEMM NT; merged
 //                               into the output launch where that is narrow
+//                               and the batch small
 // then, when every dW runs on the small-K tile (batch <= 256: C1-C4 up to
 // B=256):
 //   dX_i, i = n-2 .. 1          one launch each, on their own wave count (the
@@ -60,9 +62,9 @@ namespace volta {
 
 // How the output layer and the loss head run.
 enum OutMode {
-  OUT_NARROW = 0,     // L[n] <= 16: out_layer_kernel (dot products + loss head)
-  OUT_GEMM_LOSS = 1,  // L[n] <= 64: MFMA GEMM with the loss head in its epilogue
-  OUT_GEMM = 2,       // wider: MFMA GEMM, then a stand-alone loss kernel
+  OUT_COLUMN = 0,  // L[n] == 1, small batch: wave dot products + loss head
+  OUT_STRIP = 1,   // L[n] <= 64: 16-row MFMA strips + loss head (out_strip_kernel)
+  OUT_GEMM = 2,    // wider: MFMA GEMM, then a stand-alone loss kernel
 };
 
 static std::string hip_msg(const char* what, hipError_t e) {
@@ -114,13 +116,12 @@ struct Handle {
   unsigned* counters = nullptr;   // split-K arrival counters (+1: loss counter)
   int n_counters = 0;
   float* loss_partials = nullptr;  // one float per output-layer M-tile
-  int out_mode = 0;           // OUT_NARROW / OUT_GEMM_LOSS / OUT_GEMM (output layer + loss head)
+  int out_mode = 0;           // OutMode (output layer + loss head)
   bool narrow_dx = false;     // dX of the output layer as an outer product (L[n] <= 16)
   bool out_dx_merged = false; // ... formed by the output layer's own launch (out_layer_dx_kernel)
   bool fwd_head = false;      // ... and that launch folded into the last hidden forward launch (opt-in)
   bool tail_merge = false;    // ... or that launch and dX_{n-2} in one (gemm_smallm_tail; VOLTA_NO_TAIL=1: off)
   bool narrow_dw = false;     // dW of the output layer by narrow_dw_kernel
-  bool out_mfma = false;      // large batch: the narrow output layer on small-M tiles, its loss summed by dX_{n-1}
   std::vector<int> fwd_khalf; // per layer: > 0 runs its forward over two halves of K (this one first),
                               // its output formed by the next forward launch (0: one launch)
   bool keep_grads = false;    // also store dW/db in `grads` (VOLTA_KEEP_GRADS=1)
@@ -391,10 +392,10 @@ static bool enqueue_step(Handle* h, hipStream_t st, Recorder* rec = nullptr) {
       group_by += dw_cost(i).second;
     }
     set_group_width(h, group, 0);
-    defer_loss = h->dw_group && h->out_mode == OUT_NARROW && h->out_dx_merged && !h->fwd_head;
+    defer_loss = h->dw_group && h->out_mode != OUT_GEMM && h->out_dx_merged && !h->fwd_head;
     if (defer_loss) {
       group.loss_partials = h->loss_partials;
-      group.loss_blocks = out_layer_dx_blocks(B);
+      group.loss_blocks = h->out_mode == OUT_STRIP ? out_strip_blocks(B) : out_layer_dx_blocks(B);
       group.loss_denom = s.loss == VOLTA_LOSS_MSE ? (float)(B * Ln) : (float)B;
       group.loss_scalars = h->scalars;
     }
@@ -405,6 +406,7 @@ static bool enqueue_step(Handle* h, hipStream_t st, Recorder* rec = nullptr) {
       group_ok = h->dw_group && dw_group_supported(group);
     }
   }
+  const bool outer_loss = h->out_mode == OUT_STRIP && h->narrow_dx && !h->extras() && B > kNarrowMaxB;
   // The narrow output layer's arguments (layer n-1), with its dX_{n-1}
   // fields when that is formed in the same launch.
   auto out_args = [&]() {
@@ -425,13 +427,15 @@ static bool enqueue_step(Handle* h, hipStream_t st, Recorder* rec = nullptr) {
     o.scalars = h->scalars;
     o.bc_table = h->bc_table;
     o.bc_len = h->bc_len;
+    o.loss_counter = h->counters + h->n_counters - 1;
     if (h->out_dx_merged) {
       o.dx_act = s.activation;
       o.dx_pre = h->pre[n - 2];
       o.dx_out = h->delta[n - 2];
-      o.loss_counter = h->counters + h->n_counters - 1;
-      o.defer_loss = defer_loss ? 1 : 0;
     }
+    // the loss sum is left to the dW group or, at a large batch, to the
+    // outer-product dX launch
+    o.defer_loss = defer_loss || outer_loss ? 1 : 0;
     return o;
   };
   // algorithmic bytes of the narrow output layer: 4(B*r + r*c + B*c) + loss
@@ -445,7 +449,7 @@ static bool enqueue_step(Handle* h, hipStream_t st, Recorder* rec = nullptr) {
   // The output launch and dX_{n-2} in one launch when the product runs on
   // the 16-wave small-M tile and the loss sum is left to the dW group.
   bool tail = false;
-  if (h->tail_merge && defer_loss && h->out_mode == OUT_NARROW) {
+  if (h->tail_merge && defer_loss) {
     const PairOp t = make_dx(n - 2, h->gemm_ws);
     tail = tail_supported(t.plan, t.args, out_args());
   }
@@ -454,24 +458,14 @@ static bool enqueue_step(Handle* h, hipStream_t st, Recorder* rec = nullptr) {
     const LayerPlan& lp = h->layers[i];
     const bool last = i == n - 1;
     if (last && head_done) continue;
-    if (last && h->out_mfma) {
-      GemmArgs a{};
-      base_args(a);
-      a.A = h->act[i];
-      a.lda = lp.r;
-      a.B = h->params + lp.w_off;
-      a.ldb = lp.c;
-      a.M = B;
-      a.N = lp.c;
-      a.K = lp.r;
-      a.epi.kind = EPI_ROWS;
-      a.epi.bias = h->params + lp.b_off;
-      VOLTA_CHECK(launch_smallm_out_head(a, out_args(), st));
-      std::snprintf(label, sizeof label, "fwd%d+loss", i);
-      VOLTA_CHECK(mark(rec, label, 2.0 * B * lp.r * lp.c, out_bytes()));
+    if (last && h->out_mode == OUT_STRIP) {
+      VOLTA_CHECK(launch_out_strip(out_args(), h->out_dx_merged, st));
+      if (h->out_dx_merged) std::snprintf(label, sizeof label, "fwd%d+loss+dx%d", i, i);
+      else std::snprintf(label, sizeof label, "fwd%d+loss", i);
+      VOLTA_CHECK(mark(rec, label, (h->out_dx_merged ? 4.0 : 2.0) * B * lp.r * lp.c, out_bytes()));
       continue;
     }
-    if (last && h->out_mode == OUT_NARROW) {
+    if (last && h->out_mode == OUT_COLUMN) {
       const OutLayerArgs o = out_args();
       const double fb = out_bytes();
       if (tail) {
@@ -503,27 +497,15 @@ static bool enqueue_step(Handle* h, hipStream_t st, Recorder* rec = nullptr) {
     a.M = B;
     a.N = lp.c;
     a.K = lp.r;
-    a.epi.kind = last && h->out_mode == OUT_GEMM_LOSS ? EPI_LOSS : EPI_BIAS_ACT;
+    a.epi.kind = EPI_BIAS_ACT;
     a.epi.act = last ? kIdentity : h->gemm_act();
     a.epi.ldc = lp.c;
     a.epi.out = h->act[i + 1];
     a.epi.pre = last ? nullptr : h->pre[i];
     a.epi.bias = h->params + lp.b_off;
-    if (last) {
-      a.epi.loss = s.loss;
-      a.epi.y = static_cast<const float*>(h->target);
-      a.epi.labels = static_cast<const int32_t*>(h->target);
-      a.epi.delta = h->delta[n - 1];
-      a.epi.loss_partials = h->loss_partials;
-      a.epi.loss_counter = h->counters + h->n_counters - 1;
-      a.epi.loss_tiles = (B + 63) / 64;
-      a.epi.bc_table = h->bc_table;
-      a.epi.bc_len = h->bc_len;
-    }
-    std::snprintf(label, sizeof label, last && h->out_mode == OUT_GEMM_LOSS ? "fwd%d+loss" : "fwd%d", i);
-    // algorithmic bytes: 4(B*r + r*c + B*c*(2 if hidden else 1)) (+ loss head)
-    const double bytes = 4.0 * ((double)B * lp.r + (double)lp.r * lp.c + (double)B * lp.c * (last ? 1 : 2)) +
-                         (last && h->out_mode == OUT_GEMM_LOSS ? 8.0 * B * Ln : 0.0);
+    std::snprintf(label, sizeof label, "fwd%d", i);
+    // algorithmic bytes: 4(B*r + r*c + B*c*(2 if hidden else 1))
+    const double bytes = 4.0 * ((double)B * lp.r + (double)lp.r * lp.c + (double)B * lp.c * (last ? 1 : 2));
     if (!last && h->fwd_khalf[i]) {
       // two halves of K into the workspace's planes (4(B*r + r*c + 2*B*c))
       VOLTA_CHECK(launch_smallm_khalves(lp.fwd, a, h->gemm_ws, h->fwd_khalf[i], st));
@@ -742,7 +724,7 @@ static bool enqueue_step(Handle* h, hipStream_t st, Recorder* rec = nullptr) {
     std::snprintf(lx, sizeof lx, "dx%d", i);
     if (h->narrow_dx) {
       LossDefer ld;
-      if (h->out_mfma) {  // the step's loss from the output launch's strip partials
+      if (outer_loss) {  // the step's loss from the output launch's strip partials
         ld.partials = h->loss_partials;
         ld.blocks = (B + 15) / 16;
         ld.denom = s.loss == VOLTA_LOSS_MSE ? (float)(B * Ln) : (float)B;
@@ -915,40 +897,34 @@ static bool build(Handle* h) {
   h->flat = off;
 
   // GEMM plans.  Vector (16-byte) operand loads need the contiguous extent
-  // and leading dimension to be multiples of 4 floats.  The output layer's
-  // loss head runs in its GEMM when the layer fits one 64-wide tile.
+  // and leading dimension to be multiples of 4 floats.
   const int Ln = h->L[n];
-  h->out_mode = Ln <= 16 ? OUT_NARROW : Ln <= 64 ? OUT_GEMM_LOSS : OUT_GEMM;
+  // One column and at most kNarrowMaxB rows: wave dot products, one row per
+  // wave; without codegen extras their launch also forms dX_{n-1}, with them
+  // one block runs all rows, up to 32k activations (512-1024-1024-512-256-1
+  // with LayerNorm at B=64: 111.3 us a step, 112.0 on strips).  Every other
+  // layer of up to 64 columns runs on strips, whose loss and deltas take one
+  // launch (measured there).
+  const bool column = Ln == 1 && B <= kNarrowMaxB && n > 1 &&
+                      (!h->extras() || (int64_t)B * h->L[n - 1] <= 32768);
+  h->out_mode = column ? OUT_COLUMN : Ln <= kOutStripMaxN ? OUT_STRIP : OUT_GEMM;
   h->narrow_dx = Ln <= 16 && n > 1;
   const char* nod = std::getenv("VOLTA_NO_OUT_DX");
-  h->out_dx_merged = h->narrow_dx && !h->extras() && !(nod && *nod && *nod != '0') &&
-                     out_layer_dx_supported(B, h->L[n - 1], Ln);
+  h->out_dx_merged = h->narrow_dx && !h->extras() && !(nod && *nod && *nod != '0') && B <= kNarrowMaxB;
   // Opt-in: its per-workgroup release fence costs more than the launch it
   // saves on C2/C3 (0.0613 -> 0.0643, 0.1035 -> 0.1096 ms), less on C1
   // (0.0402 -> 0.0384 ms).
   const char* fh = std::getenv("VOLTA_FWD_HEAD");
-  h->fwd_head = h->out_dx_merged && Ln == 1 && fh && *fh && *fh != '0';
+  h->fwd_head = h->out_dx_merged && h->out_mode == OUT_COLUMN && fh && *fh && *fh != '0';
   const char* nt = std::getenv("VOLTA_NO_TAIL");
-  h->tail_merge = h->out_dx_merged && !h->fwd_head && Ln == 1 && n >= 3 && !(nt && *nt && *nt != '0');
+  h->tail_merge = h->out_dx_merged && h->out_mode == OUT_COLUMN && !h->fwd_head && n >= 3 && !(nt && *nt && *nt != '0');
   h->narrow_dw = Ln <= 16 && B <= kNarrowMaxB;
-  // A narrow output layer of more rows than the one-launch output kernels
-  // take (C5: 4096 rows of 10 classes) runs on MFMA, one 16-row strip per
-  // 16-wave small-M workgroup, with each row's loss head after the product;
-  // the strips' loss partials are added by the outer-product dX_{n-1}
-  // launch that follows (no loss launch of its own).  The wave dot
-  // products of out_layer_kernel plus the loss launch took 28.7 us at C5.
-  // VOLTA_OUT_MFMA=0 keeps them.
-  const char* om = std::getenv("VOLTA_OUT_MFMA");
-  h->out_mfma = h->out_mode == OUT_NARROW && !h->extras() && h->narrow_dx && !h->out_dx_merged &&
-                out_layer_blocks(B) > 1 && !(om && *om == '0');
   size_t ws_floats = 0;
   int max_tiles = 1;
   for (int i = 0; i < n; ++i) {
     LayerPlan& lp = h->layers[i];
     const bool vr = lp.r % 4 == 0, vc = lp.c % 4 == 0;
-    const bool loss_gemm = i == n - 1 && h->out_mode == OUT_GEMM_LOSS;
-    lp.fwd = gemm_plan(GEMM_NN, B, lp.c, lp.r, vr && vc, h->num_cus, !loss_gemm);
-    if (loss_gemm) lp.fwd.tile = TILE_64x64;
+    lp.fwd = gemm_plan(GEMM_NN, B, lp.c, lp.r, vr && vc, h->num_cus);
     lp.dx = gemm_plan(GEMM_NT, B, lp.r, lp.c, vc, h->num_cus);
     lp.dw = gemm_plan(GEMM_TN, lp.r, lp.c, B, vr && vc, h->num_cus);
     ws_floats = std::max(ws_floats, lp.fwd.workspace_floats(B, lp.c));
@@ -1065,7 +1041,7 @@ static bool build(Handle* h) {
   if (ws_floats) req((void**)&h->gemm_ws, ws_floats * 4);
   req((void**)&h->counters, (size_t)(h->n_counters + 1) * sizeof(unsigned));  // + the input launch's
   req((void**)&h->loss_partials,
-      (size_t)std::max({(B + 63) / 64, out_layer_blocks(B), out_layer_dx_blocks(B),
+      (size_t)std::max({out_strip_blocks(B), out_layer_dx_blocks(B),
                         h->out_mode == OUT_GEMM ? loss_head_blocks(s.loss, B, Ln) : 1}) * 4);
   size_t total = 0;
   for (auto& r : reqs) total += r.bytes;

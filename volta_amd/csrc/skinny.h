@@ -23,14 +23,14 @@ struct OutLayerArgs {
   DevScalars* scalars;
   const float2* bc_table;
   int bc_len;
-  // launch_out_layer_dx only: delta_{n-2} = (delta_{n-1} W^T) * f'(layer n-2)
+  // launches that also form delta_{n-2} = (delta_{n-1} W^T) * f'(layer n-2)
   int dx_act;               // activation of layer n-2 (enum volta_activation)
   const float* dx_pre;      // its pre-activation [B x K] (null when not kept)
   float* dx_out;            // delta_{n-2} [B x K]
   unsigned* loss_counter;   // arrival ticket of the blocks (zero between launches)
-  // launch_out_layer_dx only: 1 = leave the loss sum to a later launch (the
-  // dW group of the step): the blocks only store their partials, block 0
-  // advances the step counter, and no arrival ticket is taken
+  // 1 = leave the loss sum to a later launch of the step (the dW group or the
+  // outer-product dX): the blocks only store their partials, block 0 advances
+  // the step counter, and no arrival ticket is taken
   int defer_loss;
 };
 
@@ -55,17 +55,22 @@ struct NarrowDwArgs {
 // the batch); larger batches take the TN GEMM.
 constexpr int kNarrowMaxB = 256;
 
-int out_layer_blocks(int B);
+// The one-column output layer and its loss head in one block.
 hipError_t launch_out_layer(const OutLayerArgs& p, hipStream_t st);
-// The output layer, its loss head and the output layer's dX in one launch
-// (one batch row per wave, 4 rows per block; the last block to finish adds
-// the blocks' losses in block order).  For B <= kNarrowMaxB with a
-// K x N W of at most kOutWlFloats floats when N > 1.
+// The one-column output layer, its loss head and its dX in one launch (one
+// batch row per wave, 4 rows per block; the last block to finish adds the
+// blocks' losses in block order).  For B <= kNarrowMaxB.
 int out_layer_dx_blocks(int B);
 bool out_layer_dx_supported(int B, int K, int N);
 hipError_t launch_out_layer_dx(const OutLayerArgs& p, hipStream_t st);
+// The output layer of up to kOutStripMaxN columns on 16-row strips of the
+// batch, with the loss head, and with dX_{n-1} (p.dx_*, N <= 16) when `dx`;
+// p.partials: one float per strip, p.loss_counter: zero between launches.
+constexpr int kOutStripMaxN = 64;
+int out_strip_blocks(int B);
+hipError_t launch_out_strip(const OutLayerArgs& p, bool dx, hipStream_t st);
 // The step's loss from the per-strip partials an earlier output launch
-// stored (launch_smallm_out_head), added by block (0, 0) of a later launch
+// stored (launch_out_strip with defer_loss), added by block (0, 0) of a later launch
 // in a fixed order (a tree over each 256 strips, the chunks in order); its
 // non-finite flag likewise.  partials == null: none.
 struct LossDefer {

@@ -13,14 +13,10 @@ namespace volta {
 // rows (CE) or elements (MSE) are spread over the chip, and the step's loss is
 // formed by whichever block finishes last.
 //
-// A block leaves its loss sum in partials[block] and takes the ticket; the
-// block that arrives last adds the partials (thread t: blocks t, t + 256, ...
-// in order, then a fixed butterfly and the waves in order), so the sum does
-// not depend on the arrival order.  The partials are stored and read at agent
-// scope, past the XCDs' L2s, and a store has completed (vmcnt 0) before its
-// block takes the ticket: only the partials cross between blocks, so nothing
-// else of the L2s is written back or invalidated (an agent-scope fence per
-// block would do that).
+// A block publishes its loss sum (publish_partial); the block that finishes
+// last adds the partials (thread t: blocks t, t + 256, ... in order, then a
+// fixed butterfly and the waves in order), so the sum does not depend on the
+// arrival order.
 constexpr int kLossThreads = 256;
 constexpr int kLossWaves = kLossThreads / kWave;
 
@@ -38,26 +34,24 @@ __device__ __forceinline__ float block_sum_fixed(float v, float* lds) {
   return s;
 }
 
-// The block's sum `s` (thread 0) into the step's loss: sum / denom.
-__device__ __forceinline__ void loss_finish(float s, float denom, const LossHead& h, float* lds) {
+// The block's sum `s` (thread 0) into the step's loss: sum / denom.  `next`:
+// thread 0's step_prefetch from the kernel's start (only the block that
+// finishes last writes the counter, after every block has started).
+__device__ __forceinline__ void loss_finish(float s, float denom, const LossHead& h, const StepNext& next,
+                                            float* lds) {
   if (gridDim.x == 1) {
-    if (threadIdx.x == 0) step_epilogue(h.scalars, h.bc_table, h.bc_len, s / denom);
+    if (threadIdx.x == 0) step_finish(h.scalars, next, h.bc_table != nullptr, s / denom);
     return;
   }
   __shared__ unsigned last;
-  if (threadIdx.x == 0) {
-    __hip_atomic_store(h.partials + blockIdx.x, s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    last = __hip_atomic_fetch_add(h.counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1u;
-  }
+  if (threadIdx.x == 0) last = publish_partial(h.partials, h.counter, blockIdx.x, gridDim.x, s) ? 1u : 0u;
   __syncthreads();
   if (!last) return;  // block-uniform
   float t = 0.0f;
-  for (unsigned b = threadIdx.x; b < gridDim.x; b += kLossThreads)
-    t = t + __hip_atomic_load(h.partials + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  for (unsigned b = threadIdx.x; b < gridDim.x; b += kLossThreads) t = t + published_partial(h.partials, b);
   t = block_sum_fixed(t, lds);
   if (threadIdx.x == 0) {
-    step_epilogue(h.scalars, h.bc_table, h.bc_len, t / denom);
+    step_finish(h.scalars, next, h.bc_table != nullptr, t / denom);
     *h.counter = 0u;  // for the next step's launch
   }
 }
@@ -69,6 +63,8 @@ __global__ void __launch_bounds__(kLossThreads)
 loss_mse_kernel(const float* __restrict__ yhat, const float* __restrict__ y, float* __restrict__ delta, int nt,
                 int per, LossHead h) {
   __shared__ float lds[kLossWaves];
+  StepNext next{};
+  if (threadIdx.x == 0) next = step_prefetch(h.scalars, h.bc_table, h.bc_len);
   const float ntf = (float)nt;
   const int64_t lo = (int64_t)blockIdx.x * per;
   const int64_t hi = lo + per < nt ? lo + per : nt;
@@ -78,7 +74,7 @@ loss_mse_kernel(const float* __restrict__ yhat, const float* __restrict__ y, flo
     acc = acc + d * d;
     delta[k] = 2.0f * d / ntf;
   }
-  loss_finish(block_sum_fixed(acc, lds), ntf, h, lds);
+  loss_finish(block_sum_fixed(acc, lds), ntf, h, next, lds);
 }
 
 __device__ __forceinline__ float wave_max(float v) {
@@ -107,6 +103,8 @@ loss_ce_kernel(const float* __restrict__ z, const int32_t* __restrict__ labels, 
                int C, int rows_per_wave, LossHead h) {
   __shared__ float lds[kLossWaves];
   constexpr int R = PER > 0 ? PER : 1;
+  StepNext next{};
+  if (threadIdx.x == 0) next = step_prefetch(h.scalars, h.bc_table, h.bc_len);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const float bf = (float)B;
   float acc = 0.0f;  // lane 0: the wave's row losses in row order
@@ -158,7 +156,7 @@ loss_ce_kernel(const float* __restrict__ z, const int32_t* __restrict__ labels, 
 #pragma unroll
   for (int w = 1; w < kLossWaves; ++w) s = s + lds[w];
   __syncthreads();
-  loss_finish(s, bf, h, lds);
+  loss_finish(s, bf, h, next, lds);
 }
 
 // A step's inputs into the resident batch.  Blocks [0, xb) copy x, the rest y:
