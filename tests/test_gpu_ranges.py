@@ -124,3 +124,52 @@ def test_output_strips(loss, K, N, B, extras):
     say(f"output strips {loss} K={K} N={N} B={B} extras={extras}")
     kw = dict(layernorm=True, clip_grad=0.5) if extras else {}
     against_oracle(MlpSpec([8, K, N], "tanh", "sgd", loss, **kw), B)
+
+
+# The runtime optimizer's two access widths (whole and partial chunks, aligned
+# and misaligned tensors) and its two ways of passing pointers (64 tensors in
+# the arguments, more in a table): bit for bit the oracle, as its other tests.
+@pytest.mark.parametrize("kind", ["sgd", "adam", "rmsprop", "lars"])
+@pytest.mark.parametrize("n", [3, 64, 65])
+def test_runtime_optimizer_widths(kind, n):
+    from volta_amd.backend import RtOptimizer, config
+
+    say(f"runtime optimizer {kind} n={n}")
+    lib, ora = load_hip(), load_oracle()
+    counts = [(1023, 1024, 1025, 2048, 5)[i % 5] + (4096 if i == 1 else 0) for i in range(n)]
+    rng = np.random.default_rng(n)
+    ps = [rng.standard_normal(c + 1).astype(np.float32) for c in counts]
+    gs = [rng.standard_normal(c + 1).astype(np.float32) for c in counts]
+    dp, dg = [DeviceArray(p) for p in ps], [DeviceArray(g) for g in gs]
+    shift = [i % 3 == 2 for i in range(n)]  # misaligned parameter
+    gshift = [i % 4 == 3 for i in range(n)]
+    hp = [p.copy() for p in ps]
+    hip_opt, ora_opt = RtOptimizer(lib.lib, counts), RtOptimizer(ora.lib, counts)
+    cfg = config(kind, 0.01, weight_decay=0.01, momentum=0.9)
+    for _ in range(3):
+        hip_opt.apply(cfg, [d.ptr + 4 * s for d, s in zip(dp, shift)], [d.ptr + 4 * s for d, s in zip(dg, gshift)])
+        ora_opt.apply(cfg, [p.ctypes.data + 4 * s for p, s in zip(hp, shift)],
+                      [g.ctypes.data + 4 * s for g, s in zip(gs, gshift)])
+    for d, p in zip(dp, hp):
+        if kind == "lars":  # its norms are a tree, the oracle's sequential: rounding of the local rate
+            np.testing.assert_allclose(d.numpy(), p, rtol=1e-5, atol=1e-6)
+        else:
+            np.testing.assert_array_equal(d.numpy(), p)
+
+
+# Host-fed inference through pinned memory, and above 1 MiB through copies:
+# the rows of one call agree with a training handle's forward on the oracle.
+@pytest.mark.parametrize("L0,Ln,rows", [(5, 3, 1), (300, 1, 873), (300, 1, 874), (16, 300, 873), (16, 300, 875), (7, 2, 2050)])
+def test_host_inference(L0, Ln, rows):
+    say(f"host inference {L0} {Ln} rows={rows}")
+    spec = MlpSpec([L0, 24, Ln], "relu", "sgd")
+    ws, bs = data.he_uniform(4, spec.sizes)
+    X = data.normal(9, (rows, L0))
+    out = []
+    for lib in (load_hip(), load_oracle()):
+        t = Trainer(lib, spec, 1024)
+        t.set_all_params(ws, bs)
+        t.infer(X[: rows // 2 + 1])
+        out.append(t.infer(X))
+        t.close()
+    np.testing.assert_allclose(out[0], out[1], rtol=1e-4, atol=1e-5)

@@ -129,6 +129,11 @@ struct Handle {
   float2* bc_table = nullptr;  // own allocation (its length depends on beta1/beta2)
   int bc_len = 0;
   float* infer_x = nullptr;    // inference input rows (allocated on first use)
+  std::vector<GemmPlan> infer_plans;  // of the row count inferred last
+  int infer_plan_rows = 0;
+  size_t infer_plan_ws = 0;
+  char* infer_stage = nullptr;  // pinned [X | out] of a chunk of inference rows
+  size_t infer_stage_bytes = 0;
   float* infer_ws = nullptr;   // split-K workspace of inference plans (grown on demand)
   float* scratch = nullptr;    // this device's static scratch (allocation-free inference)
   bool dx_alone = false;       // small-batch backward: dX launches alone, dW products grouped
@@ -195,6 +200,7 @@ Handle::~Handle() {
   if (stage_free) (void)hipEventDestroy(stage_free);
   if (h_params) (void)hipHostFree(h_params);
   if (h_stage) (void)hipHostFree(h_stage);
+  if (infer_stage) (void)hipHostFree(infer_stage);
   if (h_lr) (void)hipHostFree(h_lr);
   if (bc_table) (void)hipFree(bc_table);
   if (infer_x) (void)hipFree(infer_x);
@@ -1147,11 +1153,14 @@ static bool enqueue_forward_into(Handle* h, const std::vector<GemmPlan>& plans, 
   return true;
 }
 
-// The same for rows already in h->infer_x, result in act[n]; the handle's
+// The same for rows already in h->infer_x, result in `out`; the handle's
 // inference workspace grows (hipMalloc) when a plan needs more.
-static bool enqueue_forward(Handle* h, int rows, hipStream_t st) {
-  std::vector<GemmPlan> plans;
-  const size_t ws = forward_plans(h, rows, &plans);
+static bool enqueue_forward(Handle* h, int rows, float* out, hipStream_t st) {
+  if (rows != h->infer_plan_rows) {
+    h->infer_plan_ws = forward_plans(h, rows, &h->infer_plans);
+    h->infer_plan_rows = rows;
+  }
+  const size_t ws = h->infer_plan_ws;
   if (ws > h->infer_ws_floats) {
     VOLTA_CHECK(hipStreamSynchronize(st));
     if (h->infer_ws) VOLTA_CHECK(hipFree(h->infer_ws));
@@ -1160,7 +1169,43 @@ static bool enqueue_forward(Handle* h, int rows, hipStream_t st) {
     VOLTA_CHECK(hipMalloc((void**)&h->infer_ws, ws * sizeof(float)));
     h->infer_ws_floats = ws;
   }
-  return enqueue_forward_into(h, plans, rows, h->infer_x, h->act[h->n], h->infer_ws, st);
+  return enqueue_forward_into(h, h->infer_plans, rows, h->infer_x, out, h->infer_ws, st);
+}
+
+// One chunk of host rows X [m x L0] into host out [m x Ln], synchronously.
+// Up to 1 MiB each way both cross through pinned memory that the GPU reads
+// (the input launch) and the output layer writes itself: a copy of pageable
+// memory each way took 16 of the 48 us of a one-row call of
+// 512-1024-1024-512-256-1.
+static bool infer_chunk(Handle* h, const float* X, int m, float* out) {
+  const size_t xb = (size_t)m * h->L[0] * sizeof(float), ob = (size_t)m * h->L[h->n] * sizeof(float);
+  constexpr size_t kMax = (size_t)1 << 20;
+  if (xb > kMax || ob > kMax) {
+    VOLTA_CHECK(hipMemcpyAsync(h->infer_x, X, xb, hipMemcpyHostToDevice, h->stream));
+    if (!enqueue_forward(h, m, h->act[h->n], h->stream)) return false;
+    VOLTA_CHECK(hipMemcpyAsync(out, h->act[h->n], ob, hipMemcpyDeviceToHost, h->stream));
+    VOLTA_CHECK(hipStreamSynchronize(h->stream));
+    return true;
+  }
+  const size_t out_off = align_up(xb, 256), need = out_off + ob;
+  if (need > h->infer_stage_bytes) {  // (the stream is idle between chunks)
+    if (h->infer_stage) VOLTA_CHECK(hipHostFree(h->infer_stage));
+    h->infer_stage = nullptr;
+    h->infer_stage_bytes = 0;
+    const size_t size = std::max(align_up(need, 4096), std::min(2 * need, 2 * kMax + 256));
+    VOLTA_CHECK(hipHostMalloc((void**)&h->infer_stage, size, hipHostMallocMapped | hipHostMallocCoherent));
+    h->infer_stage_bytes = size;
+  }
+  std::memcpy(h->infer_stage, X, xb);
+  InputCopy c;
+  c.x = reinterpret_cast<const uint32_t*>(h->infer_stage);
+  c.x_dst = reinterpret_cast<uint32_t*>(h->infer_x);
+  c.nx = xb / 4;
+  VOLTA_CHECK(launch_input_copy(c, h->stream));
+  if (!enqueue_forward(h, m, reinterpret_cast<float*>(h->infer_stage + out_off), h->stream)) return false;
+  VOLTA_CHECK(hipStreamSynchronize(h->stream));
+  std::memcpy(out, h->infer_stage + out_off, ob);
+  return true;
 }
 
 static void fail(Handle* h, int bits, const std::string& msg) {
@@ -1796,12 +1841,7 @@ int32_t volta_train_infer(VoltaTrainHandle* vh, const float* X, int64_t rows, fl
   }
   for (int64_t r0 = 0; r0 < rows; r0 += B) {
     const int m = (int)std::min<int64_t>(B, rows - r0);
-    if (hipMemcpyAsync(h->infer_x, X + r0 * L0, (size_t)m * L0 * sizeof(float), hipMemcpyHostToDevice,
-                       h->stream) != hipSuccess ||
-        !volta::enqueue_forward(h, m, h->stream) ||
-        hipMemcpyAsync(out + r0 * Ln, h->act[h->n], (size_t)m * Ln * sizeof(float), hipMemcpyDeviceToHost,
-                       h->stream) != hipSuccess ||
-        hipStreamSynchronize(h->stream) != hipSuccess) {
+    if (!volta::infer_chunk(h, X + r0 * L0, m, out + r0 * Ln)) {
       volta::fail(h, VOLTA_STATUS_DEVICE_ERROR, "volta_train_infer: device error");
       return -1;
     }
