@@ -5,12 +5,15 @@
 //
 // Layout: the tensors are cut into chunks of kRtChunk elements, one
 // workgroup per chunk (a host-built table maps workgroup -> tensor, chunk);
-// thread t of a chunk updates elements t, t+256, t+512, t+768, so every load
-// and store of a wave is one contiguous 256-byte run.  Every load is
-// unconditional (index clamped to the tensor), stores are guarded.  The
-// optimizer state of each kind (Adam m/v, RMSprop v/buf, Adagrad acc, LARS
-// velocity) is one device arena over all tensors, allocated zero-filled the
-// first time a configuration needs it.
+// thread t of a chunk updates the chunk's float4 t where parameter and
+// gradient are 16-byte aligned and the chunk is whole, else elements t, t+256,
+// t+512, t+768, so every access of a wave is one contiguous run either way.
+// Scalar loads are unconditional (index clamped to the tensor), stores are
+// guarded.  The optimizer state of each kind (Adam m/v, RMSprop v/buf, Adagrad
+// acc, LARS velocity) is one device arena over all tensors, allocated
+// zero-filled the first time a configuration needs it.  The pointers of a call
+// travel as kernel arguments (up to kRtInline tensors; more through a device
+// table), so a call is one launch and no copy.
 //
 // Arithmetic: the reference's f32 expressions in its order (built with
 // -ffp-contract=off, IEEE division and square root), so every update equals
@@ -31,6 +34,7 @@
 #include <vector>
 
 #include "../../include/volta_backend.h"
+#include "device_common.h"
 
 namespace volta {
 namespace {
@@ -41,20 +45,30 @@ constexpr int kRtChunk = kRtThreads * kRtPer;
 
 thread_local std::string g_rt_err;
 
-struct RtTensor {
+// What a call brings per tensor; where its state lies and its size are fixed.
+struct RtPtrs {
   float* p;
   const float* g;  // null: no gradient this step (skipped)
-  float* s0;       // first state buffer of the kind (or null)
-  float* s1;       // second state buffer (Adam v, RMSprop momentum buffer)
+};
+struct RtShape {
+  int64_t off;  // first element in a state arena
   int64_t count;
 };
 
+constexpr int kRtInline = 64;
 struct RtArgs {
-  const RtTensor* tensors;
-  const int2* blocks;  // workgroup -> (tensor, chunk)
-  float lr, b1, b2, om1, om2, bias1, bias2, eps, wd, alpha, om_alpha, mo, tc;
-  const float2* norms;  // LARS: (|p|, |g|) per tensor
+  const RtPtrs* table;    // more than kRtInline tensors (else null)
+  const RtShape* shapes;
+  const int2* blocks;     // workgroup -> (tensor, chunk)
+  float* s0;              // first state arena of the kind (or null)
+  float* s1;              // second one (Adam v, RMSprop momentum buffer)
+  float lr, b1, b2, om1, om2, eps, wd, alpha, om_alpha, mo, tc;
+  double rbias1, rbias2;  // 1 / (1 - beta^step), for div_by_const
+  const float2* norms;    // LARS: (|p|, |g|) per tensor
+  RtPtrs ptrs[kRtInline];
 };
+
+__device__ __forceinline__ RtPtrs rt_ptrs(const RtArgs& a, int i) { return a.table ? a.table[i] : a.ptrs[i]; }
 
 // The update of one element, in the reference's expression order.
 template <int KIND, bool MOM>
@@ -64,8 +78,8 @@ __device__ __forceinline__ void rt_elem(const RtArgs& a, float local_lr, float& 
   } else if constexpr (KIND == VOLTA_RT_ADAM || KIND == VOLTA_RT_ADAMW) {
     s0 = a.b1 * s0 + a.om1 * g;        // :333
     s1 = a.b2 * s1 + a.om2 * (g * g);  // :334
-    const float mh = s0 / a.bias1;
-    const float vh = s1 / a.bias2;
+    const float mh = div_by_const(s0, a.rbias1);  // the f32 quotients s0 / bias1, s1 / bias2
+    const float vh = div_by_const(s1, a.rbias2);
     if constexpr (KIND == VOLTA_RT_ADAMW)
       p = p - a.lr * (mh / (sqrtf(vh) + a.eps) + a.wd * p);  // :438
     else
@@ -90,11 +104,28 @@ __device__ __forceinline__ void rt_elem(const RtArgs& a, float local_lr, float& 
   }
 }
 
-template <int KIND, bool MOM>
+template <bool NT>
+__device__ __forceinline__ floatx4 rt_load4(const float* p) {
+  if constexpr (NT) return __builtin_nontemporal_load(reinterpret_cast<const floatx4*>(p));
+  else return *reinterpret_cast<const floatx4*>(p);
+}
+
+// HBM bound.  NT: the 16-byte loads bypass the caches, for a call whose
+// arrays together are well over the 256 MiB last-level cache: Adam over 25.2M
+// parameters (four arrays, 384 MiB) 147 -> 120 us a call, 5.9 TB/s.  Below
+// that the cache keeps what the next call reads: Adagrad over the same
+// parameters (288 MiB) 86 us without, 89 with; AdamW over 10.9M (167 MiB) 58
+// and 61.  The line between them is kRtNtBytes.  16-byte accesses, the
+// divisions by the bias corrections as multiplications and the pointers in
+// the arguments took SGD over 25.2M from 60 to 55 us and RMSprop over 6810
+// from 17.8 to 14.9.
+constexpr size_t kRtNtBytes = (size_t)336 << 20;
+template <int KIND, bool MOM, bool NT>
 __global__ void __launch_bounds__(kRtThreads) rt_apply_kernel(RtArgs a) {
   const int2 bt = a.blocks[blockIdx.x];
-  const RtTensor t = a.tensors[bt.x];
+  const RtPtrs t = rt_ptrs(a, bt.x);
   if (!t.g) return;  // whole workgroup
+  const RtShape sh = a.shapes[bt.x];
   constexpr bool kS0 = KIND != VOLTA_RT_SGD;
   constexpr bool kS1 = KIND == VOLTA_RT_ADAM || KIND == VOLTA_RT_ADAMW || (KIND == VOLTA_RT_RMSPROP && MOM);
   float local_lr = a.lr;
@@ -103,16 +134,36 @@ __global__ void __launch_bounds__(kRtThreads) rt_apply_kernel(RtArgs a) {
     // :631-635: lr * trust * |p| / (|g| + wd * |p| + eps) when both norms are positive
     if (nm.x > 0.0f && nm.y > 0.0f) local_lr = a.lr * a.tc * nm.x / (nm.y + a.wd * nm.x + a.eps);
   }
-  const int64_t base = (int64_t)bt.y * kRtChunk + threadIdx.x;
-  const int64_t last = t.count - 1;
+  float* const p0 = kS0 ? a.s0 + sh.off : nullptr;
+  float* const p1 = kS1 ? a.s1 + sh.off : nullptr;
+  const int64_t lo = (int64_t)bt.y * kRtChunk;
+  if (lo + kRtChunk <= sh.count && (((uintptr_t)t.p | (uintptr_t)t.g) & 15) == 0) {  // (the arenas are aligned)
+    const int64_t i = lo + 4 * (int)threadIdx.x;
+    floatx4 p = rt_load4<NT>(t.p + i);
+    const floatx4 g = rt_load4<NT>(t.g + i);
+    floatx4 s0 = kS0 ? rt_load4<NT>(p0 + i) : floatx4{};
+    floatx4 s1 = kS1 ? rt_load4<NT>(p1 + i) : floatx4{};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      float x = p[j], y = s0[j], z = s1[j];
+      rt_elem<KIND, MOM>(a, local_lr, x, g[j], y, z);
+      p[j] = x, s0[j] = y, s1[j] = z;
+    }
+    *reinterpret_cast<floatx4*>(t.p + i) = p;
+    if (kS0) *reinterpret_cast<floatx4*>(p0 + i) = s0;
+    if (kS1) *reinterpret_cast<floatx4*>(p1 + i) = s1;
+    return;
+  }
+  const int64_t base = lo + threadIdx.x;
+  const int64_t last = sh.count - 1;
   float p[kRtPer], g[kRtPer], s0[kRtPer], s1[kRtPer];
 #pragma unroll
   for (int j = 0; j < kRtPer; ++j) {
     const int64_t i = min(base + (int64_t)j * kRtThreads, last);
     p[j] = t.p[i];
     g[j] = t.g[i];
-    s0[j] = kS0 ? t.s0[i] : 0.0f;
-    s1[j] = kS1 ? t.s1[i] : 0.0f;
+    s0[j] = kS0 ? p0[i] : 0.0f;
+    s1[j] = kS1 ? p1[i] : 0.0f;
   }
 #pragma unroll
   for (int j = 0; j < kRtPer; ++j) rt_elem<KIND, MOM>(a, local_lr, p[j], g[j], s0[j], s1[j]);
@@ -121,8 +172,8 @@ __global__ void __launch_bounds__(kRtThreads) rt_apply_kernel(RtArgs a) {
     const int64_t i = base + (int64_t)j * kRtThreads;
     if (i <= last) {
       t.p[i] = p[j];
-      if (kS0) t.s0[i] = s0[j];
-      if (kS1) t.s1[i] = s1[j];
+      if (kS0) p0[i] = s0[j];
+      if (kS1) p1[i] = s1[j];
     }
   }
 }
@@ -146,10 +197,10 @@ __device__ __forceinline__ float2 block_sum2(float2 v, float2* sh) {
 __global__ void __launch_bounds__(kRtThreads) rt_norm_partials(RtArgs a, float2* partials) {
   __shared__ float2 sh[kRtThreads];
   const int2 bt = a.blocks[blockIdx.x];
-  const RtTensor t = a.tensors[bt.x];
+  const RtPtrs t = rt_ptrs(a, bt.x);
   if (!t.g) return;
   const int64_t base = (int64_t)bt.y * kRtChunk + threadIdx.x;
-  const int64_t last = t.count - 1;
+  const int64_t last = a.shapes[bt.x].count - 1;
   float p[kRtPer], g[kRtPer];
 #pragma unroll
   for (int j = 0; j < kRtPer; ++j) {
@@ -174,7 +225,7 @@ __global__ void __launch_bounds__(kRtThreads) rt_norm_finish(RtArgs a, const int
                                                               float2* norms) {
   __shared__ float2 sh[kRtThreads];
   const int ti = blockIdx.x;
-  if (!a.tensors[ti].g) return;
+  if (!rt_ptrs(a, ti).g) return;
   const int b0 = first_block[ti], b1 = first_block[ti + 1];
   float2 s = make_float2(0.0f, 0.0f);
   for (int b = b0 + (int)threadIdx.x; b < b1; b += kRtThreads) {
@@ -231,8 +282,9 @@ struct VoltaRtOptimizer {
   int nblocks = 0;
   int2* blocks = nullptr;       // device: workgroup -> (tensor, chunk)
   int* first_block = nullptr;   // device: n + 1 workgroup offsets
-  RtTensor* tensors = nullptr;  // device descriptor table
-  RtTensor* staging = nullptr;  // pinned host copy of the table
+  RtShape* shapes = nullptr;    // device
+  RtPtrs* table = nullptr;      // device pointer table (more than kRtInline tensors)
+  RtPtrs* staging = nullptr;    // its pinned host copy
   float2* partials = nullptr;   // LARS
   float2* norms = nullptr;
   float* state[6] = {};
@@ -258,7 +310,8 @@ void release(VoltaRtOptimizer* h) {
     if (s) (void)hipFree(s);
   if (h->blocks) (void)hipFree(h->blocks);
   if (h->first_block) (void)hipFree(h->first_block);
-  if (h->tensors) (void)hipFree(h->tensors);
+  if (h->shapes) (void)hipFree(h->shapes);
+  if (h->table) (void)hipFree(h->table);
   if (h->partials) (void)hipFree(h->partials);
   if (h->norms) (void)hipFree(h->norms);
   if (h->staging) (void)hipHostFree(h->staging);
@@ -293,11 +346,13 @@ int validate(VoltaRtOptimizer* h, const volta_rt_config& c, RtArgs& a) {
       if (c.kind == VOLTA_RT_ADAMW && !nonneg(c.weight_decay))
         return fail("AdamW weight_decay must be a finite non-negative number, got " + show(c.weight_decay));
       if (h->step > INT32_MAX) return fail("Optimizer step overflow for " + nm + " bias correction");
-      a.bias1 = 1.0f - powi_f32(c.beta1, (int32_t)h->step);
-      a.bias2 = 1.0f - powi_f32(c.beta2, (int32_t)h->step);
-      if (a.bias1 <= 0.0f || a.bias2 <= 0.0f)
-        return fail(nm + " bias correction underflowed (bias1=" + show(a.bias1) + ", bias2=" + show(a.bias2) +
+      const float bias1 = 1.0f - powi_f32(c.beta1, (int32_t)h->step);
+      const float bias2 = 1.0f - powi_f32(c.beta2, (int32_t)h->step);
+      if (bias1 <= 0.0f || bias2 <= 0.0f)
+        return fail(nm + " bias correction underflowed (bias1=" + show(bias1) + ", bias2=" + show(bias2) +
                     "); step=" + std::to_string(h->step));
+      a.rbias1 = 1.0 / (double)bias1;
+      a.rbias2 = 1.0 / (double)bias2;
       a.b1 = c.beta1;
       a.b2 = c.beta2;
       a.om1 = 1.0f - c.beta1;
@@ -342,7 +397,11 @@ int validate(VoltaRtOptimizer* h, const volta_rt_config& c, RtArgs& a) {
 
 template <int KIND, bool MOM>
 void launch_apply(VoltaRtOptimizer* h, const RtArgs& a) {
-  hipLaunchKernelGGL((rt_apply_kernel<KIND, MOM>), dim3(h->nblocks), dim3(kRtThreads), 0, h->stream, a);
+  const int arrays = 2 + (a.s0 ? 1 : 0) + (a.s1 ? 1 : 0);
+  if ((size_t)h->total * arrays * sizeof(float) > kRtNtBytes)
+    hipLaunchKernelGGL((rt_apply_kernel<KIND, MOM, true>), dim3(h->nblocks), dim3(kRtThreads), 0, h->stream, a);
+  else
+    hipLaunchKernelGGL((rt_apply_kernel<KIND, MOM, false>), dim3(h->nblocks), dim3(kRtThreads), 0, h->stream, a);
 }
 
 }  // namespace
@@ -384,11 +443,17 @@ VoltaRtOptimizer* volta_rt_optimizer_new(int32_t n, const int64_t* counts) {
   first[n] = (int)blocks.size();
   h->nblocks = (int)blocks.size();
   for (auto& c : h->created) c.assign(n, 0);
+  std::vector<RtShape> shapes(n);
+  for (int i = 0; i < n; ++i) shapes[i] = {h->off[i], h->counts[i]};
   if (!ok(hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking), "volta_rt: stream") ||
       !ok(hipMalloc((void**)&h->blocks, blocks.size() * sizeof(int2)), "volta_rt: allocation") ||
       !ok(hipMalloc((void**)&h->first_block, first.size() * sizeof(int)), "volta_rt: allocation") ||
-      !ok(hipMalloc((void**)&h->tensors, (size_t)n * sizeof(RtTensor)), "volta_rt: allocation") ||
-      !ok(hipHostMalloc((void**)&h->staging, (size_t)n * sizeof(RtTensor)), "volta_rt: pinned allocation") ||
+      !ok(hipMalloc((void**)&h->shapes, shapes.size() * sizeof(RtShape)), "volta_rt: allocation") ||
+      (n > kRtInline &&
+       (!ok(hipMalloc((void**)&h->table, (size_t)n * sizeof(RtPtrs)), "volta_rt: allocation") ||
+        !ok(hipHostMalloc((void**)&h->staging, (size_t)n * sizeof(RtPtrs)), "volta_rt: pinned allocation"))) ||
+      !ok(hipMemcpy(h->shapes, shapes.data(), shapes.size() * sizeof(RtShape), hipMemcpyHostToDevice),
+          "volta_rt: upload") ||
       !ok(hipMemcpy(h->blocks, blocks.data(), blocks.size() * sizeof(int2), hipMemcpyHostToDevice),
           "volta_rt: upload") ||
       !ok(hipMemcpy(h->first_block, first.data(), first.size() * sizeof(int), hipMemcpyHostToDevice),
@@ -428,18 +493,17 @@ int32_t volta_rt_apply_gradients(VoltaRtOptimizer* h, const volta_rt_config* cfg
     default: break;
   }
   if ((b0 >= 0 && !ensure_state(h, b0)) || (b1 >= 0 && !ensure_state(h, b1))) return -1;
-  for (int i = 0; i < h->n; ++i) {
-    RtTensor& t = h->staging[i];
-    t.p = params[i];
-    t.g = grads[i];
-    t.s0 = b0 >= 0 ? h->state[b0] + h->off[i] : nullptr;
-    t.s1 = b1 >= 0 ? h->state[b1] + h->off[i] : nullptr;
-    t.count = h->counts[i];
+  RtPtrs* ptrs = h->n > kRtInline ? h->staging : a.ptrs;
+  for (int i = 0; i < h->n; ++i) ptrs[i] = {params[i], grads[i]};
+  if (h->n > kRtInline) {
+    if (!ok(hipMemcpyAsync(h->table, h->staging, (size_t)h->n * sizeof(RtPtrs), hipMemcpyHostToDevice, h->stream),
+            "volta_rt: pointer upload"))
+      return -1;
+    a.table = h->table;
   }
-  if (!ok(hipMemcpyAsync(h->tensors, h->staging, (size_t)h->n * sizeof(RtTensor), hipMemcpyHostToDevice, h->stream),
-          "volta_rt: descriptor upload"))
-    return -1;
-  a.tensors = h->tensors;
+  a.shapes = h->shapes;
+  a.s0 = b0 >= 0 ? h->state[b0] : nullptr;
+  a.s1 = b1 >= 0 ? h->state[b1] : nullptr;
   a.blocks = h->blocks;
   if (kind == VOLTA_RT_LARS) {
     if (!h->partials && (!ok(hipMalloc((void**)&h->partials, (size_t)h->nblocks * sizeof(float2)), "volta_rt: LARS") ||
