@@ -173,3 +173,20 @@ def test_host_inference(L0, Ln, rows):
         out.append(t.infer(X))
         t.close()
     np.testing.assert_allclose(out[0], out[1], rtol=1e-4, atol=1e-5)
+
+
+# Sizes of no particular multiple through the small-K dW tiles (rows of 1 to 5
+# elements, one past a tile, several 64-k slices), the small-M tile's 16-byte
+# loads moved back inside their rows (K of 1 to 5 and remainders of a wave's
+# range) and the 64x64 tiles' (larger batches).
+@pytest.mark.parametrize("sizes,B", [([1, 2, 3, 4], 1), ([3, 5, 2, 5], 2), ([5, 33, 31, 6], 65), ([4, 65, 64, 7], 64),
+                                     ([63, 130, 1, 9, 2], 17), ([257, 18, 515, 3], 256), ([70, 1025, 34, 1], 130),
+                                     ([13, 397, 250, 101, 7], 77), ([301, 703, 66, 2], 300), ([530, 1030, 67], 515),
+                                     ([2, 771, 3, 770, 5], 641)])
+@pytest.mark.parametrize("opt", ["sgd", "adam"])
+def test_ragged_layers(sizes, B, opt):
+    """Adam divides each gradient by its own size, so a gradient of rounding
+    size moves a weight by up to lr either way: lr is small enough that three
+    such steps stay under the absolute tolerance."""
+    say(f"ragged layers {sizes} B={B} {opt}")
+    against_oracle(MlpSpec(sizes, "tanh", opt), B, lr=0.02 if opt == "sgd" else 3e-6)

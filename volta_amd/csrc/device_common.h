@@ -13,6 +13,25 @@ typedef float floatx16 __attribute__((ext_vector_type(16)));
 
 constexpr int kWave = 64;
 
+// Four consecutive floats at any 4-byte aligned address, one 16-byte access
+// (the memory pipeline takes dword-aligned 16-byte loads and stores; one that
+// crosses a cache line costs two).
+typedef float floatx4u __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ floatx4 load4u(const float* p) { return *reinterpret_cast<const floatx4u*>(p); }
+__device__ __forceinline__ void store4u(float* p, const floatx4& x) { *reinterpret_cast<floatx4u*>(p) = x; }
+
+// Elements c .. c + 3 of a row of n floats whose load was moved back to start
+// at min(c, n - 4) to stay inside it: v holds elements from there, `sh` is how
+// far it moved (c - min(c, n - 4)); elements past the row's end read as 0.
+__device__ __forceinline__ floatx4 unshift4(const floatx4& v, int sh) {
+  floatx4 r;
+  r[0] = sh == 0 ? v[0] : sh == 1 ? v[1] : sh == 2 ? v[2] : sh == 3 ? v[3] : 0.0f;
+  r[1] = sh == 0 ? v[1] : sh == 1 ? v[2] : sh == 2 ? v[3] : 0.0f;
+  r[2] = sh == 0 ? v[2] : sh == 1 ? v[3] : 0.0f;
+  r[3] = sh == 0 ? v[3] : 0.0f;
+  return r;
+}
+
 // Per-handle scalars the captured step reads and writes on the device, so a
 // graph replay needs no host-side argument patching.
 struct DevScalars {

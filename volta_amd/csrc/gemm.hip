@@ -59,50 +59,52 @@ struct LdsTile {
 // Load the ROWS x BK tile of an operand (rows = M or N index) starting at
 // (row0, k0) into registers, 4 consecutive floats per slot along the
 // contiguous dimension.  Out-of-range elements read as 0.
+//
+// Without VEC (rows whose 16-byte runs are not aligned, or whose length is no
+// multiple of 4) the 16-byte loads are moved back inside the row where they
+// would pass its end, unconditionally (clamped row), and put right by store();
+// rows of fewer than 4 elements are loaded one by one.
 template <int ROWS, int BK, bool KC, bool VEC, int THREADS>
 struct TileLoader {
   static constexpr int kSlots = ROWS * BK / 4;
   static constexpr int kPerThread = (kSlots + THREADS - 1) / THREADS;
   floatx4 v[kPerThread];
+  int rows_, K_, row0_, k0_;  // without VEC: the tile store() puts right
+
+  // slot -> the tile's row (M or N index) and k of its four elements
+  static __device__ __forceinline__ void coords(int slot, int& r, int& kk) {
+    if (KC) {  // (row, 4 consecutive k)
+      r = slot / (BK / 4);
+      kk = (slot % (BK / 4)) * 4;
+    } else {   // (k, 4 consecutive rows)
+      kk = slot / (ROWS / 4);
+      r = (slot % (ROWS / 4)) * 4;
+    }
+  }
 
   __device__ __forceinline__ void load(const float* __restrict__ p, int ld, int rows, int K,
                                        int row0, int k0, int tid) {
+    if constexpr (!VEC) rows_ = rows, K_ = K, row0_ = row0, k0_ = k0;
 #pragma unroll
     for (int it = 0; it < kPerThread; ++it) {
       const int slot = tid + it * THREADS;
       floatx4 x = {0.f, 0.f, 0.f, 0.f};
-      if (slot < kSlots) {
-        int r, kk;
-        if (KC) {  // slot -> (row, 4 consecutive k)
-          r = slot / (BK / 4);
-          kk = (slot % (BK / 4)) * 4;
-        } else {   // slot -> (k, 4 consecutive rows)
-          kk = slot / (ROWS / 4);
-          r = (slot % (ROWS / 4)) * 4;
-        }
-        const int gr = row0 + r, gk = k0 + kk;
-        if (KC) {
-          if (gr < rows) {
-            const float* src = p + (size_t)gr * ld + gk;
-            if (VEC) {
-              if (gk < K) x = *reinterpret_cast<const floatx4*>(src);
-            } else {
-#pragma unroll
-              for (int e = 0; e < 4; ++e)
-                if (gk + e < K) x[e] = src[e];
-            }
-          }
+      int r, kk;
+      coords(slot, r, kk);
+      const int gr = row0 + r, gk = k0 + kk;
+      if constexpr (VEC) {
+        if (slot < kSlots && gr < rows && gk < K)
+          x = *reinterpret_cast<const floatx4*>(KC ? p + (size_t)gr * ld + gk : p + (size_t)gk * ld + gr);
+      } else {
+        const int n = KC ? K : rows;                              // the contiguous extent,
+        const int c = KC ? gk : gr;                               // the place in it,
+        const int line = KC ? min(gr, rows - 1) : min(gk, K - 1);  // and the line
+        const float* src = p + (size_t)line * ld;
+        if (n >= 4) {
+          x = load4u(src + min(c, n - 4));
         } else {
-          if (gk < K) {
-            const float* src = p + (size_t)gk * ld + gr;
-            if (VEC) {
-              if (gr < rows) x = *reinterpret_cast<const floatx4*>(src);
-            } else {
 #pragma unroll
-              for (int e = 0; e < 4; ++e)
-                if (gr + e < rows) x[e] = src[e];
-            }
-          }
+          for (int e = 0; e < 4; ++e) x[e] = src[min(c + e, n - 1)];
         }
       }
       v[it] = x;
@@ -115,15 +117,18 @@ struct TileLoader {
       const int slot = tid + it * THREADS;
       if (slot < kSlots) {
         int r, kk;
-        if (KC) {
-          r = slot / (BK / 4);
-          kk = (slot % (BK / 4)) * 4;
-          *reinterpret_cast<floatx4*>(lds + r * LdsTile<ROWS, BK, KC>::kStride + kk) = v[it];
-        } else {
-          kk = slot / (ROWS / 4);
-          r = (slot % (ROWS / 4)) * 4;
-          *reinterpret_cast<floatx4*>(lds + kk * LdsTile<ROWS, BK, KC>::kStride + r) = v[it];
+        coords(slot, r, kk);
+        floatx4 x = v[it];
+        if constexpr (!VEC) {
+          const int gr = row0_ + r, gk = k0_ + kk;
+          const int n = KC ? K_ : rows_, c = KC ? gk : gr;
+          const bool in = KC ? gr < rows_ : gk < K_;
+          if (n >= 4) x = unshift4(x, c - min(c, n - 4));
+#pragma unroll
+          for (int e = 0; e < 4; ++e) x[e] = in && c + e < n ? x[e] : 0.0f;
         }
+        *reinterpret_cast<floatx4*>(lds + (KC ? r * LdsTile<ROWS, BK, KC>::kStride + kk
+                                              : kk * LdsTile<ROWS, BK, KC>::kStride + r)) = x;
       }
     }
   }
@@ -1419,11 +1424,23 @@ __device__ __forceinline__ void smallm_tile(const GemmArgs& args, int blk, float
           for (int s = 0; s < 4; ++s) fb[g][s] = pb[(size_t)(kl + s) * ldb];
         }
       } else {
+        // 16-byte loads moved back inside the wave's range (compute() undoes
+        // the move); fewer than 4 k: one by one
+        if (K >= 4) {
+          const int kl = min(k, kend - 4);
+          fa[g] = load4u(pa + kl);
+          if (B_KC) fb[g] = load4u(pb + kl);
+        } else {
 #pragma unroll
-        for (int s = 0; s < 4; ++s) {
-          const int kl = min(k + s, kend - 1);
-          fa[g][s] = pa[kl];
-          fb[g][s] = B_KC ? pb[kl] : pb[(size_t)kl * ldb];
+          for (int s = 0; s < 4; ++s) {
+            const int kl = min(k + s, kend - 1);
+            fa[g][s] = pa[kl];
+            if (B_KC) fb[g][s] = pb[kl];
+          }
+        }
+        if (!B_KC) {
+#pragma unroll
+          for (int s = 0; s < 4; ++s) fb[g][s] = pb[(size_t)min(k + s, kend - 1) * ldb];
         }
       }
     }
@@ -1451,11 +1468,18 @@ __device__ __forceinline__ void smallm_tile(const GemmArgs& args, int blk, float
   static_assert(kSmallChunk % 4 == 0, "a chunk must hold whole rounds of the four accumulators");
   float dr = 0.0f;  // head operand: delta_{n-1} of the lane's row
   // (the head operand's A values replace the chunk's act values in fa)
-  auto compute = [&](floatx4(&fa)[CH], const floatx4(&fb)[CH], int kc) {
+  auto compute = [&](floatx4(&fa)[CH], floatx4(&fb)[CH], int kc) {
 #pragma unroll
     for (int g = 0; g < CH; ++g) {
       if (kc + 16 * g < kend) {  // wave-uniform
         const int k = kc + 16 * g + 4 * q;
+        if constexpr (!VEC) {
+          if (K >= 4 && kc + 16 * g + 16 > kend) {  // wave-uniform: the range's last group
+            const int sh = k - min(k, kend - 4);
+            fa[g] = unshift4(fa[g], sh);
+            if (B_KC) fb[g] = unshift4(fb[g], sh);
+          }
+        }
         floatx4 xa;  // head operand: the lane's four A values of the group
         if constexpr (AH == 3) {
 #pragma unroll
@@ -1868,7 +1892,13 @@ static_assert(kDwT * (kDwTW + 1) <= kDwK * kDwS, "the wide dW tile fits over the
 // slice into two accumulators per block (even groups, odd groups) and then
 // the two: every element of dW sums the same products in the same order,
 // so the two forms give bit-identical results.
-template <int EPI, int TN = kDwT>
+//
+// VEC: M, N and the leading dimensions are multiples of 4 and every operand
+// 16-byte aligned.  Otherwise the operands' 16-byte loads are moved back
+// inside their row where they would pass its end (put right when the slice is
+// stored), the tile's float4 of W, m and v likewise, and rows of fewer than 4
+// elements are loaded one by one: same products, same order.
+template <int EPI, int TN = kDwT, bool VEC = true>
 __device__ __forceinline__ void dw_smallk_tile(const GemmArgs& args, int blk, float* lds, int tid) {
   static_assert(EPI == EPI_DW_OPT || EPI == EPI_STORE, "epilogues of the dW tile");
   static_assert(TN == kDwT || TN == kDwTW, "tile widths of the dW tile");
@@ -1894,6 +1924,15 @@ __device__ __forceinline__ void dw_smallk_tile(const GemmArgs& args, int blk, fl
   const EpiArgs& e = args.epi;
   const floatx4 zero4 = {0.f, 0.f, 0.f, 0.f};
 
+  // without VEC: elements c .. c + 3 of a row of n floats, as loaded (moved
+  // back inside the row), and put right (0 past its end)
+  auto row4 = [](const float* row, int c, int n) {
+    if (n >= 4) return load4u(row + min(c, n - 4));
+    return floatx4{row[0], row[min(1, n - 1)], row[min(2, n - 1)], 0.0f};
+  };
+  auto fix4 = [&](const floatx4& v, int c, int n) {
+    return c < n ? unshift4(v, n >= 4 ? c - min(c, n - 4) : c) : zero4;
+  };
   // One 64-k slice of both operands: 64 rows of 8 float4 of A (two per
   // thread) and 64 rows of TN/4 float4 of B (TN/16 per thread).
   floatx4 xa[2], xb[BIT];
@@ -1904,10 +1943,14 @@ __device__ __forceinline__ void dw_smallk_tile(const GemmArgs& args, int blk, fl
       const int kk = slot >> 3, c4 = (slot & 7) * 4;
       const int k = k0 + kk;
       const bool kok = k < K;
-      const bool aok = kok && m0 + c4 < M;
       const size_t ka = kok ? (size_t)k : 0;
-      const floatx4 va = *reinterpret_cast<const floatx4*>(args.A + ka * args.lda + (aok ? m0 + c4 : 0));
-      xa[it] = aok ? va : zero4;
+      if constexpr (VEC) {
+        const bool aok = kok && m0 + c4 < M;
+        const floatx4 va = *reinterpret_cast<const floatx4*>(args.A + ka * args.lda + (aok ? m0 + c4 : 0));
+        xa[it] = aok ? va : zero4;
+      } else {
+        xa[it] = row4(args.A + ka * args.lda, m0 + c4, M);
+      }
     }
 #pragma unroll
     for (int it = 0; it < BIT; ++it) {
@@ -1915,23 +1958,29 @@ __device__ __forceinline__ void dw_smallk_tile(const GemmArgs& args, int blk, fl
       const int kk = slot / CPR, c4 = (slot % CPR) * 4;
       const int k = k0 + kk;
       const bool kok = k < K;
-      const bool bok = kok && n0 + c4 < N;
       const size_t kb = kok ? (size_t)k : 0;
-      const floatx4 vb = *reinterpret_cast<const floatx4*>(args.B + kb * args.ldb + (bok ? n0 + c4 : 0));
-      xb[it] = bok ? vb : zero4;
+      if constexpr (VEC) {
+        const bool bok = kok && n0 + c4 < N;
+        const floatx4 vb = *reinterpret_cast<const floatx4*>(args.B + kb * args.ldb + (bok ? n0 + c4 : 0));
+        xb[it] = bok ? vb : zero4;
+      } else {
+        xb[it] = row4(args.B + kb * args.ldb, n0 + c4, N);
+      }
     }
   };
-  auto store_slice = [&]() {
+  auto store_slice = [&](int k0) {
 #pragma unroll
     for (int it = 0; it < 2; ++it) {
       const int slot = tid + 256 * it;
       const int kk = slot >> 3, c4 = (slot & 7) * 4;
+      if constexpr (!VEC) xa[it] = k0 + kk < K ? fix4(xa[it], m0 + c4, M) : zero4;
       *reinterpret_cast<floatx4*>(la + kk * kDwS + c4) = xa[it];
     }
 #pragma unroll
     for (int it = 0; it < BIT; ++it) {
       const int slot = tid + 256 * it;
       const int kk = slot / CPR, c4 = (slot % CPR) * 4;
+      if constexpr (!VEC) xb[it] = k0 + kk < K ? fix4(xb[it], n0 + c4, N) : zero4;
       *reinterpret_cast<floatx4*>(lb + kk * SB + c4) = xb[it];
     }
   };
@@ -1945,9 +1994,10 @@ __device__ __forceinline__ void dw_smallk_tile(const GemmArgs& args, int blk, fl
 #pragma unroll
   for (int j = 0; j < EIT; ++j) {
     const int gm = m0 + row0 + j * RSTEP;
-    own[j] = gm < M && gn < N;  // N % 4 == 0: the whole float4 is in range
+    own[j] = gm < M && gn < N;  // VEC: N % 4 == 0, the whole float4 is in range
     o[j] = own[j] ? (uint32_t)gm * (uint32_t)e.ldc + (uint32_t)gn : 0u;
   }
+  const int ncols = min(4, N - gn);  // without VEC: the thread's columns in range
   const int bn = n0 + (tid & (TN - 1));
   const bool do_db = EPI == EPI_DW_OPT && args.colsum_b && e.b && tm == 0;
 
@@ -1963,9 +2013,30 @@ __device__ __forceinline__ void dw_smallk_tile(const GemmArgs& args, int blk, fl
   // waves per SIMD without spills)
   constexpr int EARLY = TN == kDwT ? EIT : 1;
   auto load_state = [&](int j) {
-    w4[j] = *reinterpret_cast<const floatx4*>(e.out + o[j]);
-    m4[j] = *reinterpret_cast<const floatx4*>(pm + o[j]);
-    v4[j] = *reinterpret_cast<const floatx4*>(pv + o[j]);
+    if constexpr (VEC) {
+      w4[j] = *reinterpret_cast<const floatx4*>(e.out + o[j]);
+      m4[j] = *reinterpret_cast<const floatx4*>(pm + o[j]);
+      v4[j] = *reinterpret_cast<const floatx4*>(pv + o[j]);
+    } else {  // (as loaded; put right before the update)
+      const size_t row = own[j] ? o[j] - (uint32_t)gn : 0u;
+      const int c = own[j] ? gn : 0;
+      w4[j] = row4(e.out + row, c, N);
+      m4[j] = row4(pm + row, c, N);
+      v4[j] = row4(pv + row, c, N);
+    }
+  };
+  // stores of the thread's float4 j
+  auto put4 = [&](float* p, int j, const floatx4& x) {
+    if (!own[j]) return;
+    if constexpr (VEC) {
+      *reinterpret_cast<floatx4*>(p + o[j]) = x;
+    } else if (ncols == 4) {
+      store4u(p + o[j], x);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+        if (i < ncols) p[o[j] + i] = x[i];
+    }
   };
   auto load_bias_state = [&]() {
     const float* pb = e.b ? e.b : e.out;
@@ -1996,7 +2067,7 @@ __device__ __forceinline__ void dw_smallk_tile(const GemmArgs& args, int blk, fl
       __syncthreads();  // the previous slice is consumed
       load_slice(k0);
     }
-    store_slice();
+    store_slice(k0);
     __syncthreads();
     if (do_db && tid < TN) {
       // batch order; each batch of 8 reads is issued before its first add
@@ -2050,12 +2121,17 @@ __device__ __forceinline__ void dw_smallk_tile(const GemmArgs& args, int blk, fl
 
   if constexpr (EPI == EPI_STORE) {
 #pragma unroll
-    for (int j = 0; j < EIT; ++j)
-      if (own[j]) *reinterpret_cast<floatx4*>(e.out + o[j]) = g4[j];
+    for (int j = 0; j < EIT; ++j) put4(e.out, j, g4[j]);
   } else {
 #pragma unroll
-    for (int j = 0; j < EIT; ++j)
-      if (own[j] && e.grad) *reinterpret_cast<floatx4*>(e.grad + o[j]) = g4[j];
+    for (int j = 0; j < EIT; ++j) {
+      if (e.grad) put4(e.grad, j, g4[j]);
+      if constexpr (!VEC) {
+        w4[j] = fix4(w4[j], own[j] ? gn : 0, N);
+        m4[j] = fix4(m4[j], own[j] ? gn : 0, N);
+        v4[j] = fix4(v4[j], own[j] ? gn : 0, N);
+      }
+    }
     const float lr = e.scalars->lr;
     const AdamRcp rc = adam_rcp_of(e);
     const uint32_t vec_end = (uint32_t)(e.count - e.count % 8);
@@ -2087,20 +2163,18 @@ __device__ __forceinline__ void dw_smallk_tile(const GemmArgs& args, int blk, fl
         m4[j][i] = sm[i];
         v4[j][i] = sv[i];
       }
-      if (own[j]) {
-        *reinterpret_cast<floatx4*>(e.out + o[j]) = w4[j];
-        if (e.opt != VOLTA_OPT_SGD) *reinterpret_cast<floatx4*>(e.m + o[j]) = m4[j];
-        if (e.opt == VOLTA_OPT_ADAM || e.opt == VOLTA_OPT_ADAMW) *reinterpret_cast<floatx4*>(e.v + o[j]) = v4[j];
-      }
+      put4(e.out, j, w4[j]);
+      if (e.opt != VOLTA_OPT_SGD) put4(e.m, j, m4[j]);
+      if (e.opt == VOLTA_OPT_ADAM || e.opt == VOLTA_OPT_ADAMW) put4(e.v, j, v4[j]);
     }
     if (do_db && tid < TN && bn < N) bst.update_store(e, bn, N, db, rc);
   }
 }
 
-template <int EPI>
+template <int EPI, bool VEC>
 __global__ void __launch_bounds__(256) gemm_dw_smallk(GemmArgs args) {
   __shared__ __attribute__((aligned(16))) float lds[kDwLds];
-  dw_smallk_tile<EPI>(args, blockIdx.x, lds, threadIdx.x);
+  dw_smallk_tile<EPI, kDwT, VEC>(args, blockIdx.x, lds, threadIdx.x);
 }
 
 // ---------------------------------------------------------------------------
@@ -2499,21 +2573,24 @@ static bool smallm_vec_ok(const GemmArgs& a, int layout) {
   return a.K % 4 == 0 && a.lda % 4 == 0 && al(a.A) && (layout != GEMM_NT || (a.ldb % 4 == 0 && al(a.B)));
 }
 
-// The small-K dW tile: 16-byte rows of both operands and of W_i and its state.
 static bool dw_smallk_ok(const GemmArgs& a, int layout) {
-  const auto al = [](const void* p) { return ((uintptr_t)p & 15u) == 0; };
   const EpiArgs& e = a.epi;
   if (layout != GEMM_TN || (e.kind != EPI_DW_OPT && e.kind != EPI_STORE)) return false;
-  if (a.M % 4 || a.N % 4 || a.lda % 4 || a.ldb % 4 || e.ldc % 4 || !al(a.A) || !al(a.B) || !al(e.out)) return false;
-  if (e.kind == EPI_DW_OPT && (!al(e.m) || !al(e.v) || !al(e.grad))) return false;
   if (a.colsum_b && e.kind != EPI_DW_OPT) return false;
-  return (size_t)a.M * e.ldc < ((size_t)1 << 30);
+  return a.lda >= a.M && a.ldb >= a.N && e.ldc >= a.N && (size_t)a.M * e.ldc < ((size_t)1 << 30);
+}
+
+// Its VEC form: 16-byte rows of both operands and of W_i and its state.
+static bool dw_smallk_vec(const GemmArgs& a) {
+  const auto al = [](const void* p) { return ((uintptr_t)p & 15u) == 0; };
+  const EpiArgs& e = a.epi;
+  if (a.M % 4 || a.N % 4 || a.lda % 4 || a.ldb % 4 || e.ldc % 4 || !al(a.A) || !al(a.B) || !al(e.out)) return false;
+  return e.kind != EPI_DW_OPT || (al(e.m) && al(e.v) && al(e.grad));
 }
 
 static hipError_t launch_smallm(const GemmArgs& a, int layout, bool vec, int waves, bool stage, hipStream_t st) {
   if (vec && !smallm_vec_ok(a, layout)) return hipErrorInvalidValue;
   if (waves != 4 && waves != 8 && waves != 16) return hipErrorInvalidValue;
-  if (layout == GEMM_NT && waves == 16 && !vec) return hipErrorInvalidValue;
   const int k = a.epi.kind;
   if (layout == GEMM_NN) {
     if (k == EPI_BIAS_ACT) return launch_smallm_epi<false, EPI_BIAS_ACT>(a, vec, waves, stage, st);
@@ -2703,8 +2780,12 @@ hipError_t gemm_launch(const GemmPlan& p, const GemmArgs& args_in, hipStream_t s
   if (p.tile == TILE_DW_SMALLK) {
     if (p.splits != 1 || !dw_smallk_ok(a, p.layout)) return hipErrorInvalidValue;
     const dim3 grid(p.tiles(a.M, a.N));
-    if (a.epi.kind == EPI_DW_OPT) hipLaunchKernelGGL(gemm_dw_smallk<EPI_DW_OPT>, grid, dim3(256), 0, st, a);
-    else hipLaunchKernelGGL(gemm_dw_smallk<EPI_STORE>, grid, dim3(256), 0, st, a);
+    const bool vec = dw_smallk_vec(a), opt = a.epi.kind == EPI_DW_OPT;
+    if (!vec && !p.ragged) return hipErrorInvalidValue;
+    if (opt && vec) hipLaunchKernelGGL((gemm_dw_smallk<EPI_DW_OPT, true>), grid, dim3(256), 0, st, a);
+    else if (opt) hipLaunchKernelGGL((gemm_dw_smallk<EPI_DW_OPT, false>), grid, dim3(256), 0, st, a);
+    else if (vec) hipLaunchKernelGGL((gemm_dw_smallk<EPI_STORE, true>), grid, dim3(256), 0, st, a);
+    else hipLaunchKernelGGL((gemm_dw_smallk<EPI_STORE, false>), grid, dim3(256), 0, st, a);
     if ((err = hipGetLastError()) != hipSuccess) return err;
     return mark(rec, label, 2.0 * a.M * a.N * a.K, bytes);
   }
@@ -2774,12 +2855,11 @@ struct DwSmallOp {  // dW on small-K tiles, optimizer epilogue
   }
 };
 
-template <int NMAX>
 struct NarrowDwOp {  // staged delta in the launch's LDS
   using Args = NarrowDwArgs;
   static constexpr int kLds = 0;
   static __device__ __forceinline__ void run(const NarrowDwArgs& p, int blk, float* lds) {
-    narrow_dw_block<NMAX>(p, blk, lds);
+    narrow_dw_block<1>(p, blk, lds);
   }
 };
 
@@ -2830,7 +2910,7 @@ bool pair_supported(const PairOp& a, const PairOp& b) {
       return o.plan.vec && o.plan.splits == 1 && o.plan.layout == GEMM_NT && o.args.epi.kind == EPI_DX_ACT &&
              o.plan.waves == 4 && smallm_vec_ok(o.args, GEMM_NT);
     if (o.plan.tile == TILE_DW_SMALLK)
-      return o.plan.splits == 1 && o.args.epi.kind == EPI_DW_OPT && dw_smallk_ok(o.args, GEMM_TN);
+      return o.plan.splits == 1 && o.args.epi.kind == EPI_DW_OPT && dw_smallk_ok(o.args, GEMM_TN) && dw_smallk_vec(o.args);
     // GemmOp64 runs K slice blk / tiles of ceil(K / k_per_split) and the
     // pair launches tiles * splits blocks, so the two must agree: a plan
     // whose slices run as K groups inside one workgroup (kgroups > 1,
@@ -2844,7 +2924,7 @@ bool pair_supported(const PairOp& a, const PairOp& b) {
            (o.args.epi.kind != EPI_DW_OPT || (size_t)o.args.M * o.args.epi.ldc < ((size_t)1 << 30));
   };
   auto narrow_ok = [](const PairOp& o) {
-    return o.nd.N >= 1 && o.nd.N <= 16 && o.nd.B >= 1 && o.nd.B <= kNarrowMaxB &&
+    return o.nd.N == 1 && o.nd.B >= 1 && o.nd.B <= kNarrowMaxB &&
            (o.nd.opt == VOLTA_OPT_SGD || o.nd.opt == VOLTA_OPT_ADAM || o.nd.opt == VOLTA_OPT_ADAGRAD);
   };
   const PairOp* ops[2] = {&a, &b};
@@ -2880,14 +2960,6 @@ static hipError_t launch_pair_t(const typename OA::Args& a, int na, const typena
   return hipGetLastError();
 }
 
-template <class OA>
-static hipError_t launch_with_narrow(const typename OA::Args& aa, int na, const PairOp& b, hipStream_t st) {
-  const int nb = op_blocks(b);
-  if (b.nd.N <= 1) return launch_pair_t<OA, NarrowDwOp<1>>(aa, na, b.nd, nb, st);
-  if (b.nd.N <= 4) return launch_pair_t<OA, NarrowDwOp<4>>(aa, na, b.nd, nb, st);
-  return launch_pair_t<OA, NarrowDwOp<16>>(aa, na, b.nd, nb, st);
-}
-
 static hipError_t reduce_after(const PairOp& o, hipStream_t st) {
   if (o.kind != PAIR_GEMM || o.plan.splits == 1) return hipSuccess;
   GemmArgs a = o.args;
@@ -2902,17 +2974,16 @@ static hipError_t reduce_after(const PairOp& o, hipStream_t st) {
 // workgroups [start[i], start[i+1]) after them.
 static_assert(sizeof(DwGroup) <= 4000, "DwGroup is passed by value as a kernel argument (4 KiB limit)");
 
-// Five waves per SIMD (at most 96 registers) where the narrow part's state
-// fits them (NMAX <= 4); the 16-wide narrow dW needs more (at 96 it spilled
-// 27 registers), so four.
-template <int NMAX, int TN>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NMAX <= 4 ? 5 : 3))) dw_group_kernel(DwGroup d) {
+// Five waves per SIMD (at most 96 registers); four where a product's rows are
+// not 16-byte aligned (VEC false: every product then takes that form).
+template <int TN, bool VEC>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VEC ? 5 : 4))) dw_group_kernel(DwGroup d) {
   __shared__ __attribute__((aligned(16))) float lds[TN == kDwT ? kDwLds : (kDwLdsW > kDwLds ? kDwLdsW : kDwLds)];
   int b = blockIdx.x;
   if (b == 0 && threadIdx.x == 0 && d.loss_partials)
     deferred_loss_finish(d.loss_scalars, d.loss_partials, d.loss_blocks, d.loss_denom);
   if (b < d.narrow_blocks) {
-    narrow_dw_block<NMAX, true>(d.nd, b, lds);
+    narrow_dw_block<1, true>(d.nd, b, lds);
     return;
   }
   b -= d.narrow_blocks;
@@ -2920,36 +2991,38 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NMAX <
 #pragma unroll
   for (int k = 1; k < kMaxDwGroup; ++k)
     if (k < d.n && b >= d.start[k]) i = k;
-  dw_smallk_tile<EPI_DW_OPT, TN>(d.g[i], b - d.start[i], lds, threadIdx.x);
+  dw_smallk_tile<EPI_DW_OPT, TN, VEC>(d.g[i], b - d.start[i], lds, threadIdx.x);
 }
 
 int dw_group_tiles(const GemmArgs& a, int tile_n) {
   return ((a.M + kDwT - 1) / kDwT) * ((a.N + tile_n - 1) / tile_n);
 }
 
-// The group kernel a launch of `narrow_n` narrow columns and tile width
-// `tile_n` runs (as dw_group_launch selects it).
-static const void* dw_group_fn(int narrow_n, int tile_n) {
-  if (tile_n == kDwTW) {
-    if (narrow_n <= 1) return reinterpret_cast<const void*>(&dw_group_kernel<1, kDwTW>);
-    if (narrow_n <= 4) return reinterpret_cast<const void*>(&dw_group_kernel<4, kDwTW>);
-    return reinterpret_cast<const void*>(&dw_group_kernel<16, kDwTW>);
-  }
-  if (narrow_n <= 1) return reinterpret_cast<const void*>(&dw_group_kernel<1, kDwT>);
-  if (narrow_n <= 4) return reinterpret_cast<const void*>(&dw_group_kernel<4, kDwT>);
-  return reinterpret_cast<const void*>(&dw_group_kernel<16, kDwT>);
+static bool dw_group_vec(const DwGroup& d) {
+  for (int i = 0; i < d.n; ++i)
+    if (!dw_smallk_vec(d.g[i])) return false;
+  return true;
+}
+
+// The group kernel for tile width `tile_n` (as dw_group_launch selects it).
+static const void* dw_group_fn(bool vec, int tile_n) {
+  if (tile_n == kDwTW)
+    return vec ? reinterpret_cast<const void*>(&dw_group_kernel<kDwTW, true>)
+               : reinterpret_cast<const void*>(&dw_group_kernel<kDwTW, false>);
+  return vec ? reinterpret_cast<const void*>(&dw_group_kernel<kDwT, true>)
+             : reinterpret_cast<const void*>(&dw_group_kernel<kDwT, false>);
 }
 
 int dw_group_pick_tile_n(const DwGroup& d, int num_cus) {
-  const int nn = d.narrow_blocks ? d.nd.N : 1;
+  const bool vec = dw_group_vec(d);
   int t32 = d.narrow_blocks, t64 = d.narrow_blocks;
   for (int i = 0; i < d.n; ++i) {
     t32 += dw_group_tiles(d.g[i], kDwT);
     t64 += dw_group_tiles(d.g[i], kDwTW);
   }
   int r32 = 0, r64 = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&r32, dw_group_fn(nn, kDwT), 256, 0) != hipSuccess ||
-      hipOccupancyMaxActiveBlocksPerMultiprocessor(&r64, dw_group_fn(nn, kDwTW), 256, 0) != hipSuccess ||
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&r32, dw_group_fn(vec, kDwT), 256, 0) != hipSuccess ||
+      hipOccupancyMaxActiveBlocksPerMultiprocessor(&r64, dw_group_fn(vec, kDwTW), 256, 0) != hipSuccess ||
       r32 < 1 || r64 < 1) {
     (void)hipGetLastError();
     return kDwT;
@@ -2968,7 +3041,7 @@ bool dw_group_supported(const DwGroup& d) {
   }
   if (d.narrow_blocks) {
     const NarrowDwArgs& p = d.nd;
-    if (p.N < 1 || p.N > 16 || p.B < 1 || p.B > kNarrowMaxB || narrow_lds_floats_n(p.B, p.N) > kDwLds) return false;
+    if (p.N != 1 || p.B < 1 || p.B > kNarrowMaxB || narrow_lds_floats_n(p.B, p.N) > kDwLds) return false;
     if (p.opt != VOLTA_OPT_SGD && p.opt != VOLTA_OPT_ADAM && p.opt != VOLTA_OPT_ADAGRAD) return false;
     if (d.narrow_blocks != (p.R + kNarrowRows - 1) / kNarrowRows) return false;
   }
@@ -2979,16 +3052,13 @@ hipError_t dw_group_launch(const DwGroup& d, hipStream_t st, Recorder* rec, cons
                            double bytes) {
   if (!dw_group_supported(d)) return hipErrorInvalidValue;
   const dim3 grid(d.narrow_blocks + d.start[d.n]);
-  const int nn = d.narrow_blocks ? d.nd.N : 1;
-  // (the same selection as dw_group_fn)
+  const bool vec = dw_group_vec(d);  // (the same selection as dw_group_fn)
   if (d.tile_n == kDwTW) {
-    if (nn <= 1) hipLaunchKernelGGL((dw_group_kernel<1, kDwTW>), grid, dim3(256), 0, st, d);
-    else if (nn <= 4) hipLaunchKernelGGL((dw_group_kernel<4, kDwTW>), grid, dim3(256), 0, st, d);
-    else hipLaunchKernelGGL((dw_group_kernel<16, kDwTW>), grid, dim3(256), 0, st, d);
+    if (vec) hipLaunchKernelGGL((dw_group_kernel<kDwTW, true>), grid, dim3(256), 0, st, d);
+    else hipLaunchKernelGGL((dw_group_kernel<kDwTW, false>), grid, dim3(256), 0, st, d);
   } else {
-    if (nn <= 1) hipLaunchKernelGGL((dw_group_kernel<1, kDwT>), grid, dim3(256), 0, st, d);
-    else if (nn <= 4) hipLaunchKernelGGL((dw_group_kernel<4, kDwT>), grid, dim3(256), 0, st, d);
-    else hipLaunchKernelGGL((dw_group_kernel<16, kDwT>), grid, dim3(256), 0, st, d);
+    if (vec) hipLaunchKernelGGL((dw_group_kernel<kDwT, true>), grid, dim3(256), 0, st, d);
+    else hipLaunchKernelGGL((dw_group_kernel<kDwT, false>), grid, dim3(256), 0, st, d);
   }
   const hipError_t err = hipGetLastError();
   if (err != hipSuccess) return err;
@@ -3006,24 +3076,19 @@ hipError_t pair_launch(const PairOp& a, const PairOp& b, hipStream_t st, Recorde
   hipError_t err;
   const bool b_small = b.kind == PAIR_GEMM && b.plan.tile == TILE_DW_SMALLK;
   if (a.kind == PAIR_GEMM && a.plan.layout == GEMM_NT && a.plan.tile == TILE_SMALLM) {
-    if (b.kind != PAIR_GEMM) err = launch_with_narrow<SmallDxOp>(aa, na, b, st);
+    if (b.kind != PAIR_GEMM) err = launch_pair_t<SmallDxOp, NarrowDwOp>(aa, na, b.nd, nb, st);
     else if (b_small) err = launch_pair_t<SmallDxOp, DwSmallOp>(aa, na, bb, nb, st);
     else err = launch_pair_t<SmallDxOp, DwOp>(aa, na, bb, nb, st);
   } else if (a.kind == PAIR_GEMM && a.plan.layout == GEMM_NT) {
-    err = b.kind == PAIR_GEMM ? launch_pair_t<DxOp, DwOp>(aa, na, bb, nb, st) : launch_with_narrow<DxOp>(aa, na, b, st);
+    err = b.kind == PAIR_GEMM ? launch_pair_t<DxOp, DwOp>(aa, na, bb, nb, st)
+                              : launch_pair_t<DxOp, NarrowDwOp>(aa, na, b.nd, nb, st);
   } else if (a.kind == PAIR_GEMM) {
     err = b_small ? launch_pair_t<DwSmallOp, DwSmallOp>(aa, na, bb, nb, st)
                   : launch_pair_t<DwOp, DwOp>(aa, na, bb, nb, st);
   } else if (b_small) {
-    if (a.nd.N <= 1) err = launch_pair_t<NarrowDwOp<1>, DwSmallOp>(a.nd, na, bb, nb, st);
-    else if (a.nd.N <= 4) err = launch_pair_t<NarrowDwOp<4>, DwSmallOp>(a.nd, na, bb, nb, st);
-    else err = launch_pair_t<NarrowDwOp<16>, DwSmallOp>(a.nd, na, bb, nb, st);
-  } else if (a.nd.N <= 1) {
-    err = launch_pair_t<NarrowDwOp<1>, DwOp>(a.nd, na, bb, nb, st);
-  } else if (a.nd.N <= 4) {
-    err = launch_pair_t<NarrowDwOp<4>, DwOp>(a.nd, na, bb, nb, st);
+    err = launch_pair_t<NarrowDwOp, DwSmallOp>(a.nd, na, bb, nb, st);
   } else {
-    err = launch_pair_t<NarrowDwOp<16>, DwOp>(a.nd, na, bb, nb, st);
+    err = launch_pair_t<NarrowDwOp, DwOp>(a.nd, na, bb, nb, st);
   }
   if (err != hipSuccess) return err;
   if ((err = mark(rec, label, flops, bytes)) != hipSuccess) return err;
@@ -3116,7 +3181,16 @@ GemmPlan gemm_plan(int layout, int M, int N, int K, bool vec, int num_cus, bool 
   const char* ns = std::getenv("VOLTA_NT_SPLIT_MIN");
   const long nt_split_min = ns && *ns ? std::atol(ns) : 131072L;
   const bool nt_long = layout == GEMM_NT && nt_split_min > 0 && K >= 1024 && (long)M * K >= nt_split_min;
-  if (small_m && (layout == GEMM_NN || layout == GEMM_NT) && p.splits > 1 && M <= small_max && !nt_long) {
+  // Likewise a product of a short reduction whose 64x64 grid leaves half the
+  // CUs idle: it is all start-up, and 16x16 tiles give each thread one output
+  // to finish instead of 16.  Their operand re-reads (32 rows of K per tile)
+  // set the other bound.  13-397-250-101-7 at B=77 60.3 -> 34.0 us a step,
+  // 130-23-110-19-10 at B=1 40.7 -> 25.8, 5-200-22-100 at B=2048 103.6 -> 82.8,
+  // 200-500-500-10 at B=700 90 -> 80; past the bound 256-512-512-10 at B=1024
+  // (2048 tiles of K = 512) 94.7 -> 100.
+  const size_t tiles16 = (size_t)((M + 15) / 16) * ((N + 15) / 16);
+  const bool short_k = small_max > 0 && K < 512 && 2 * tiles <= num_cus && tiles16 * K <= (size_t)12 * 256 * num_cus;
+  if (small_m && (layout == GEMM_NN || layout == GEMM_NT) && ((p.splits > 1 && M <= small_max && !nt_long) || short_k)) {
     p.tile = TILE_SMALLM;
     p.splits = 1;
     p.k_per_split = K;
@@ -3127,8 +3201,10 @@ GemmPlan gemm_plan(int layout, int M, int N, int K, bool vec, int num_cus, bool 
   // default; VOLTA_DW_SMALLK_MAX_K changes the limit, 0 turns the tile off).
   const char* dk = std::getenv("VOLTA_DW_SMALLK_MAX_K");
   const int dw_kmax = dk && *dk ? std::atoi(dk) : 256;
-  if (layout == GEMM_TN && vec && M % 4 == 0 && N % 4 == 0 && K <= dw_kmax) {
+  // A one-column dW (the output layer's) is narrow_dw_kernel's instead.
+  if (layout == GEMM_TN && N > 1 && K <= dw_kmax) {
     p.tile = TILE_DW_SMALLK;
+    p.ragged = !vec || M % 4 || N % 4;
     p.splits = 1;
     p.k_per_split = K;
   }

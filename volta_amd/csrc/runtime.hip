@@ -924,7 +924,7 @@ static bool build(Handle* h) {
   h->fwd_head = h->out_dx_merged && h->out_mode == OUT_COLUMN && fh && *fh && *fh != '0';
   const char* nt = std::getenv("VOLTA_NO_TAIL");
   h->tail_merge = h->out_dx_merged && h->out_mode == OUT_COLUMN && !h->fwd_head && n >= 3 && !(nt && *nt && *nt != '0');
-  h->narrow_dw = Ln <= 16 && B <= kNarrowMaxB;
+  h->narrow_dw = Ln == 1 && B <= kNarrowMaxB;
   size_t ws_floats = 0;
   int max_tiles = 1;
   for (int i = 0; i < n; ++i) {

@@ -7,7 +7,7 @@
 //   out_layer_dx_kernel  the same for one column and a small batch, as wave
 //                        dot products (out_layer_kernel: without dX)
 //   outer_dx_kernel      delta_{n-2} = (delta_{n-1} W^T) * f'   (K = L[n])
-//   narrow_dw_kernel     dW = act^T delta, db, optimizer update (N = L[n])
+//   narrow_dw_kernel     one column: dW = act^T delta, db, optimizer update
 //
 // Every sum has a fixed order: MFMA k groups and pairwise trees (out_strip),
 // per-lane k-strided partials then a fixed butterfly (out_layer), a
@@ -427,10 +427,9 @@ outer_dx_kernel(const float* __restrict__ delta, const float* __restrict__ W, in
 }
 
 // Stand-alone launch: 64 rows of W per block.
-template <int NMAX>
 __global__ void __launch_bounds__(kNarrowThreads) narrow_dw_kernel(NarrowDwArgs p) {
   extern __shared__ float lds[];
-  narrow_dw_block<NMAX>(p, blockIdx.x, lds);
+  narrow_dw_block<1>(p, blockIdx.x, lds);
 }
 
 // ---------------------------------------------------------------------------
@@ -466,16 +465,10 @@ hipError_t launch_outer_dx(const float* delta, const float* W, int B, int R, int
 }
 
 hipError_t launch_narrow_dw(const NarrowDwArgs& p, hipStream_t st) {
-  if (p.N > 16 || p.N < 1 || p.B < 1 || p.B > kNarrowMaxB) return hipErrorInvalidValue;
+  if (p.N != 1 || p.B < 1 || p.B > kNarrowMaxB) return hipErrorInvalidValue;
   if (p.opt != VOLTA_OPT_SGD && p.opt != VOLTA_OPT_ADAM && p.opt != VOLTA_OPT_ADAGRAD) return hipErrorInvalidValue;
   const int blocks = (p.R + kNarrowRows - 1) / kNarrowRows;
-  const dim3 block(kNarrowThreads);
-  if (p.N <= 1)
-    hipLaunchKernelGGL(narrow_dw_kernel<1>, dim3(blocks), block, narrow_lds_floats<1>(p.B, p.N) * 4, st, p);
-  else if (p.N <= 4)
-    hipLaunchKernelGGL(narrow_dw_kernel<4>, dim3(blocks), block, narrow_lds_floats<4>(p.B, p.N) * 4, st, p);
-  else
-    hipLaunchKernelGGL(narrow_dw_kernel<16>, dim3(blocks), block, narrow_lds_floats<16>(p.B, p.N) * 4, st, p);
+  hipLaunchKernelGGL(narrow_dw_kernel, dim3(blocks), dim3(kNarrowThreads), narrow_lds_floats<1>(p.B, p.N) * 4, st, p);
   return hipGetLastError();
 }
 
