@@ -190,3 +190,29 @@ def test_ragged_layers(sizes, B, opt):
     such steps stay under the absolute tolerance."""
     say(f"ragged layers {sizes} B={B} {opt}")
     against_oracle(MlpSpec(sizes, "tanh", opt), B, lr=0.02 if opt == "sgd" else 3e-6)
+
+
+# The 128x64 direct-to-LDS tile (a grid of a tile per CU, sizes of any
+# multiple): integer operands are exact in every order; last stages of 1 to 32
+# k, 16- and 4-byte loads.
+@pytest.mark.parametrize("M,N,K", [(2048, 1024, 128), (1925, 1003, 131), (2044, 1020, 160), (1921, 961, 161),
+                                   (1001, 1985, 255)])
+@pytest.mark.parametrize("layout", [0, 1, 2])
+def test_mid_tile_integer_exact(M, N, K, layout):
+    say(f"mid tile {M}x{N}x{K} layout {layout}")
+    rng = np.random.default_rng(M + layout)
+    A = rng.integers(-4, 5, (M, K)).astype(np.float32)
+    B = rng.integers(-4, 5, (K, N)).astype(np.float32)
+    dA = DeviceArray(np.ascontiguousarray(A.T) if layout == 2 else A)
+    dB = DeviceArray(np.ascontiguousarray(B.T) if layout == 1 else B)
+    dC = DeviceArray(np.zeros((M, N), np.float32))
+    lib = load_hip()
+    assert lib.lib.volta_hip_gemm(layout, dA.ptr, dB.ptr, dC.ptr, M, N, K, -1, 0) == 0, lib.last_error()
+    np.testing.assert_array_equal(dC.numpy(), A @ B)
+
+
+@pytest.mark.parametrize("sizes,B,act", [([132, 1992, 1004, 2], 2000, "gelu"), ([131, 1990, 1001, 3], 1999, "relu")])
+def test_mid_tile_step(sizes, B, act):
+    """Its three epilogues in a training step (products of 256 and 512 tiles)."""
+    say(f"mid tile step {sizes} B={B}")
+    against_oracle(MlpSpec(sizes, act, "sgd"), B, lr=0.02, steps=2)

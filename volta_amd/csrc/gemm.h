@@ -84,6 +84,7 @@ struct GemmPlan {
   bool inkernel_reduce = false;  // split-K reduced by the last slice (else a second kernel)
   int waves = 0;                 // TILE_SMALLM: waves per workgroup (4 or 8)
   int kgroups = 1;               // 64x64 / 128x128: K slices inside one workgroup (splits = 1)
+  bool mid = false;              // TILE_64x64 / TILE_128x128: run as 128x64 direct-to-LDS tiles (gemm_mid), whole K
   bool ragged = false;           // TILE_DW_SMALLK: rows of W or of an operand may not be 16-byte aligned
   bool stage = true;             // TILE_SMALLM at 16 waves: operands staged in LDS (VOLTA_SMALLM_STAGE=0: off)
   int tiles(int M, int N) const {

@@ -1247,6 +1247,192 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) g
   }
 }
 
+// ---------------------------------------------------------------------------
+// 128x64 direct-to-LDS tile for sizes of any multiple (plan.mid): eight waves
+// of one 32x32 block each, BK = 32, two stages of 24 KB in LDS, so two
+// workgroups (four waves per SIMD) share a CU and one's barriers lie under the
+// other's MFMAs.  Rows and columns past the matrix are loaded from its last
+// one and never stored; k past its end (the last stage only) is loaded from
+// its last one and masked at the MFMAs.  VEC: 16-byte load instructions (16
+// and 8 per stage); otherwise, where a row's 16-byte runs are not aligned or
+// its length is no multiple of 4, 4-byte ones (64 and 32), whose lanes cover
+// one whole LDS row.
+//
+// LDS layouts as the 256x256 tile's: K-contiguous [rows][32 k] in 16-byte
+// chunks, (row r, k-quad q) at chunk r*8 + (q ^ ((r >> 1) & 7)); MN-contiguous
+// [32 k][rows].  Sums run in the same k order as every 32x32 tile's (k-group
+// g, lane half h, step s: k = 8g + 4h + s).
+//
+// The grid decides where it wins: a 128x128 tile of 2000x3000 outputs has 384
+// tiles for 256 CUs (a second round half empty), this one 752 (measured at
+// gemm_plan).
+// ---------------------------------------------------------------------------
+constexpr int kMidM = 128, kMidN = 64, kMidK = 32;
+
+// The loads of a ROWS x 32 operand tile by 8 waves.  `rows`: the operand's M
+// or N extent, `K` its k extent.
+template <int ROWS, bool KC, bool VEC>
+__device__ __forceinline__ void mid_load(const float* __restrict__ p, int ld, int rows, int K, int row0, int k0,
+                                         float* tile, int wave, int lane) {
+  constexpr int kInstr = ROWS * kMidK / (VEC ? 256 : 64);
+#pragma unroll
+  for (int t = 0; t < kInstr / 8; ++t) {
+    const int j = wave + 8 * t;
+    int r, k;  // this lane's row and k (the first of four with VEC)
+    if constexpr (VEC && KC) {
+      r = 8 * j + (lane >> 3);
+      k = 4 * ((lane & 7) ^ ((r >> 1) & 7));
+    } else if constexpr (VEC) {
+      constexpr int kLanes = ROWS / 4;  // lanes per k row
+      k = (64 / kLanes) * j + lane / kLanes;
+      r = 4 * (lane % kLanes);
+    } else if constexpr (KC) {
+      r = 2 * j + (lane >> 5);
+      const int c = lane & 31;
+      k = 4 * ((c >> 2) ^ ((r >> 1) & 7)) + (c & 3);
+    } else {
+      k = (64 * j) / ROWS;
+      r = (64 * j) % ROWS + lane;
+    }
+    const int gr = min(row0 + r, rows - (VEC && !KC ? 4 : 1)), gk = min(k0 + k, K - (VEC && KC ? 4 : 1));
+    const float* src = p + (KC ? (size_t)gr * ld + gk : (size_t)gk * ld + gr);
+    if constexpr (VEC) __builtin_amdgcn_global_load_lds((const void*)src, (LdsVoidPtr)(tile + 256 * j), 16, 0, 0);
+    else __builtin_amdgcn_global_load_lds((const void*)src, (LdsVoidPtr)(tile + 64 * j), 4, 0, 0);
+  }
+}
+
+template <int ROWS, bool KC>
+__device__ __forceinline__ floatx4 mid_frag(const float* tile, int row, int h, int g) {
+  if constexpr (KC) {
+    return *reinterpret_cast<const floatx4*>(tile + 4 * (row * 8 + ((2 * g + h) ^ ((row >> 1) & 7))));
+  } else {
+    floatx4 f;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) f[s] = tile[(8 * g + 4 * h + s) * ROWS + row];
+    return f;
+  }
+}
+
+template <bool A_KC, bool B_KC, bool VEC, int EPI>
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) gemm_mid(GemmArgs args) {
+  __shared__ __attribute__((aligned(16))) float lds_a0[kMidM * kMidK];
+  __shared__ __attribute__((aligned(16))) float lds_b0[kMidN * kMidK];
+  __shared__ __attribute__((aligned(16))) float lds_a1[kMidM * kMidK];
+  __shared__ __attribute__((aligned(16))) float lds_b1[kMidN * kMidK];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave >> 1, wn = wave & 1, h = lane >> 5, l32 = lane & 31;
+  const int M = args.M, N = args.N, K = args.K;
+  const int tiles_n = (N + kMidN - 1) / kMidN;
+  const int bx = xcd_tile(blockIdx.x, (M + kMidM - 1) / kMidM, tiles_n);
+  const int tm = bx / tiles_n, tn = bx % tiles_n;
+  const int m0 = tm * kMidM, n0 = tn * kMidN;
+  constexpr bool kColsum = EPI == EPI_DW_OPT && !B_KC;
+  const bool colsum = kColsum && args.colsum_b && tm == 0 && wm == 0;
+  float cs = 0.0f;
+  floatx16 acc;
+#pragma unroll
+  for (int v = 0; v < 16; ++v) acc[v] = 0.0f;
+  const int arow = wm * 32 + l32, bcol = wn * 32 + l32;
+  // one stage of `nk` k (32, or fewer in the last one)
+  auto compute = [&](const float* a_s, const float* b_s, int nk) {
+    floatx4 fa_n = mid_frag<kMidM, A_KC>(a_s, arow, h, 0), fb_n = mid_frag<kMidN, B_KC>(b_s, bcol, h, 0);
+#pragma unroll
+    for (int g = 0; g < kMidK / 8; ++g) {
+      floatx4 fa = fa_n, fb = fb_n;
+      if (g + 1 < kMidK / 8) {
+        fa_n = mid_frag<kMidM, A_KC>(a_s, arow, h, g + 1);
+        fb_n = mid_frag<kMidN, B_KC>(b_s, bcol, h, g + 1);
+      }
+      if (nk < kMidK) {  // uniform: the last stage
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+          const bool in = 8 * g + 4 * h + s < nk;
+          fa[s] = in ? fa[s] : 0.0f;
+          fb[s] = in ? fb[s] : 0.0f;
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+      for (int s = 0; s < 4; ++s) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[s], fb[s], acc, 0, 0, 0);
+      __builtin_amdgcn_s_setprio(0);
+      __builtin_amdgcn_sched_barrier(0);
+      if (kColsum && colsum) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s) cs = cs + fb[s];
+      }
+    }
+  };
+  auto load = [&](int st, float* a, float* b) {
+    mid_load<kMidM, A_KC, VEC>(args.A, args.lda, M, K, m0, st * kMidK, a, wave, lane);
+    mid_load<kMidN, B_KC, VEC>(args.B, args.ldb, N, K, n0, st * kMidK, b, wave, lane);
+  };
+  // Stage s reads buffer s & 1; the loads of stage s + 1 go to the other
+  // buffer, which every wave finished reading before the barrier of stage s.
+  const int S = (K + kMidK - 1) / kMidK;
+  load(0, lds_a0, lds_b0);
+  for (int s = 0; s < S; s += 2) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (s + 1 < S) load(s + 1, lds_a1, lds_b1);
+    __builtin_amdgcn_sched_barrier(0);  // the loads stay ahead of this stage's MFMAs
+    compute(lds_a0, lds_b0, min(kMidK, K - s * kMidK));
+    if (s + 1 >= S) break;  // uniform
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (s + 2 < S) load(s + 2, lds_a0, lds_b0);
+    __builtin_amdgcn_sched_barrier(0);
+    compute(lds_a1, lds_b1, min(kMidK, K - (s + 1) * kMidK));
+  }
+  if (kColsum && colsum) cs = cs + __shfl_xor(cs, 32, kWave);
+  const EpiArgs& e = args.epi;
+  if constexpr (EPI == EPI_DW_OPT) {  // in two halves: the state of 16 elements at once would spill
+    block_epilogue<EPI>(e, acc, m0 + wm * 32 + 4 * h, n0 + bcol, M, N, 0, 8);
+    __builtin_amdgcn_sched_barrier(0);
+    block_epilogue<EPI>(e, acc, m0 + wm * 32 + 4 * h, n0 + bcol, M, N, 8, 16);
+  } else {
+    block_epilogue<EPI>(e, acc, m0 + wm * 32 + 4 * h, n0 + bcol, M, N);
+  }
+  if constexpr (kColsum) {
+    if (colsum && h == 0 && e.b && n0 + bcol < N) apply_bias_update(e, n0 + bcol, N, cs, adam_rcp_of(e));
+  }
+}
+
+// 16-byte loads of gemm_mid: aligned operands whose contiguous extents are
+// multiples of 4 (and so never pass a row's end partly).
+static bool mid_vec_ok(const GemmArgs& a, int layout) {
+  const int ca = layout == GEMM_TN ? a.M : a.K, cb = layout == GEMM_NT ? a.K : a.N;
+  return ca % 4 == 0 && cb % 4 == 0 && a.lda % 4 == 0 && a.ldb % 4 == 0 && (((uintptr_t)a.A | (uintptr_t)a.B) & 15) == 0;
+}
+
+template <bool A_KC, bool B_KC, int EPI>
+static hipError_t launch_mid_epi(const GemmArgs& a, int layout, hipStream_t st) {
+  const dim3 grid(((a.M + kMidM - 1) / kMidM) * ((a.N + kMidN - 1) / kMidN));
+  if (mid_vec_ok(a, layout)) hipLaunchKernelGGL((gemm_mid<A_KC, B_KC, true, EPI>), grid, dim3(512), 0, st, a);
+  else hipLaunchKernelGGL((gemm_mid<A_KC, B_KC, false, EPI>), grid, dim3(512), 0, st, a);
+  return hipGetLastError();
+}
+
+static hipError_t launch_mid(const GemmArgs& a, int layout, hipStream_t st) {
+  const int k = a.epi.kind;
+  switch (layout) {
+    case GEMM_NN:
+      if (k == EPI_BIAS_ACT) return launch_mid_epi<true, false, EPI_BIAS_ACT>(a, layout, st);
+      if (k == EPI_STORE) return launch_mid_epi<true, false, EPI_STORE>(a, layout, st);
+      break;
+    case GEMM_NT:
+      if (k == EPI_DX_ACT) return launch_mid_epi<true, true, EPI_DX_ACT>(a, layout, st);
+      if (k == EPI_STORE) return launch_mid_epi<true, true, EPI_STORE>(a, layout, st);
+      break;
+    case GEMM_TN:
+      if (k == EPI_DW_OPT) return launch_mid_epi<false, false, EPI_DW_OPT>(a, layout, st);
+      if (k == EPI_STORE) return launch_mid_epi<false, false, EPI_STORE>(a, layout, st);
+      break;
+  }
+  return hipErrorInvalidValue;
+}
+
 // Whether the 128x128 direct-to-LDS tile serves a product: exact
 // 128-multiples, K a multiple of 128 and at least 1024 (a shorter K keeps
 // the 64x64 grid's several workgroups per CU), 16-byte aligned operand rows,
@@ -2741,6 +2927,11 @@ hipError_t gemm_launch(const GemmPlan& p, const GemmArgs& args_in, hipStream_t s
     if ((err = launch_smallm(a, p.layout, p.vec, p.waves, p.stage, st)) != hipSuccess) return err;
     return mark(rec, label, 2.0 * a.M * a.N * a.K, bytes);
   }
+  if (p.mid) {
+    if (p.splits != 1 || p.kgroups != 1) return hipErrorInvalidValue;
+    if ((err = launch_mid(a, p.layout, st)) != hipSuccess) return err;
+    return mark(rec, label, 2.0 * a.M * a.N * a.K, bytes);
+  }
   if (p.tile == TILE_BIG) {
     // exact tiles and 16-byte aligned operands, or no launch
     const bool fits = p.splits == 1 && a.M % kBigBM == 0 && a.N % kBigBM == 0 && a.K % (2 * kBigBK) == 0 &&
@@ -2916,7 +3107,7 @@ bool pair_supported(const PairOp& a, const PairOp& b) {
     // whose slices run as K groups inside one workgroup (kgroups > 1,
     // splits 1) launches on its own.
     const int kps = std::max(o.plan.k_per_split, 1);
-    return o.plan.tile == TILE_64x64 && o.plan.vec && !o.plan.inkernel_reduce && o.plan.kgroups == 1 &&
+    return o.plan.tile == TILE_64x64 && !o.plan.mid && o.plan.vec && !o.plan.inkernel_reduce && o.plan.kgroups == 1 &&
            (o.args.K + kps - 1) / kps == o.plan.splits &&
            ((o.plan.layout == GEMM_NT && o.args.epi.kind == EPI_DX_ACT) ||
             (o.plan.layout == GEMM_TN && o.args.epi.kind == EPI_DW_OPT)) &&
@@ -3242,6 +3433,26 @@ GemmPlan gemm_plan(int layout, int M, int N, int K, bool vec, int num_cus, bool 
   if (((kg && *kg == '1') || kg_auto) && small_m && !p.inkernel_reduce && p.splits > 1 && p.splits <= kg_max) {
     p.kgroups = p.splits;
     p.splits = 1;
+  }
+  // The 128x64 direct-to-LDS tile (gemm_mid) for what is left to the
+  // register-staged tiles: a grid of about a tile per CU or more whose last
+  // round is not mostly empty, K >= 128 (VOLTA_BIG128=0: off).  The share of
+  // the rounds that is filled has to be 0.7 against 128x128 tiles and 0.8
+  // against 64x64 ones, whose finer grid wastes less: 2000x3000 (752 tiles,
+  // 0.98) K = 3000 417 -> 318 us, its dW of 1500x3000 (564, 0.73) K = 2000
+  // 307 -> 232, 2000x1000 (256, 1.0) K = 3000 128 -> 107; below, a dW of
+  // 3000x1000 (384, 0.75) K = 2000 135 -> 156, 2000x1203 (304, 0.59) K = 801
+  // 73 -> 79; too few tiles, 1024x1024 (128) K = 1024 27 -> 41.
+  const char* b128 = std::getenv("VOLTA_BIG128");
+  const int mid_tiles = ((M + kMidM - 1) / kMidM) * ((N + kMidN - 1) / kMidN);
+  const int mid_slots = (mid_tiles + num_cus - 1) / num_cus * num_cus;
+  if (small_m && !p.inkernel_reduce && (p.tile == TILE_64x64 || p.tile == TILE_128x128) && M >= kMidM && N >= kMidN &&
+      K >= 128 && 10 * mid_tiles >= 9 * num_cus && 10 * mid_tiles >= (p.tile == TILE_64x64 ? 8 : 7) * mid_slots &&
+      !(b128 && *b128 == '0')) {
+    p.mid = true;
+    p.splits = 1;
+    p.kgroups = 1;
+    p.k_per_split = K;
   }
   return p;
 }

@@ -99,6 +99,7 @@ int32_t volta_hip_gemm(int32_t layout, const float* A, const float* B, float* Cm
     p.splits = 1;
     p.k_per_split = K;
   }
+  if (force_tile >= 0 || force_splits != 0) p.mid = false;
   if (force_tile >= 0) p.ragged = false;  // a tile asked for by name runs in its aligned form
   if (force_tile == TILE_NARROW_TN) narrow_tn_split_plan(M, K, cus, &p.k_per_split, &p.splits);
   if (force_splits != 0) {
