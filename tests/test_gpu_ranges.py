@@ -216,3 +216,14 @@ def test_mid_tile_step(sizes, B, act):
     """Its three epilogues in a training step (products of 256 and 512 tiles)."""
     say(f"mid tile step {sizes} B={B}")
     against_oracle(MlpSpec(sizes, act, "sgd"), B, lr=0.02, steps=2)
+
+
+# The codegen extras' backward launch (rows beside 64-column blocks) and the
+# launch that ends their first phase (clip sums, biases, gamma and beta), alone
+# and together, over several steps of the dropout stream.
+@pytest.mark.parametrize("extras", [dict(layernorm=True), dict(dropout_p=0.2), dict(clip_grad=0.3),
+                                    dict(layernorm=True, dropout_p=0.3, clip_grad=0.2)])
+@pytest.mark.parametrize("sizes,B", [([5, 2, 1], 1), ([9, 64, 65, 3], 33), ([70, 257, 130, 100], 20), ([16, 40, 12], 300)])
+def test_extras_launches(sizes, B, extras):
+    say(f"extras {sizes} B={B} {extras}")
+    against_oracle(MlpSpec(sizes, "tanh", "sgd", **extras), B)

@@ -26,30 +26,30 @@ struct HiddenFwdArgs {
   const DevScalars* scalars;  // rng = the step's starting state
 };
 
-// One hidden layer's backward extras on delta [B x c] (gradient w.r.t. the
-// layer's final output): LayerNorm backward, dropout mask, activation
-// derivative (softmax: the row form y * (d - dot(d, y))), in that order.
+// One hidden layer's backward extras (`din`: gradient w.r.t. the layer's
+// final output): LayerNorm backward, dropout mask, activation derivative
+// (softmax: the row form y * (d - dot(d, y))), in that order, and the
+// LayerNorm gradients' column sums.
 struct HiddenBwdArgs {
-  float* delta;          // [B x c], updated in place
+  const float* din;      // [B x c]: dL/d(layer output); with LayerNorm not `delta` itself
+  float* delta;          // [B x c]: dL/d(pre-activation)
   const float* act;      // layer output (after LayerNorm / dropout)
   const float* pre;      // pre-activation
   int B, c, act_kind;
   const float* gamma;    // LayerNorm (null: off), pre-update values
   const float* beta;
   const float* inv_std;
-  float* dgamma;         // [c] column sums (written by ln_bwd_cols)
+  float* dgamma;         // [c] column sums (LayerNorm)
   float* dbeta;
   const uint8_t* mask;   // dropout (null: off)
   float keep_scale;
+  DevScalars* scalars;   // rng_draws > 0: the dropout stream advances by that many draws (once per step)
+  uint64_t rng_draws;
 };
 
 hipError_t launch_hidden_fwd(const HiddenFwdArgs& a, hipStream_t st);
-// LayerNorm backward: gamma/beta gradients (columns), then the row pass
-// (with dropout mask and activation derivative), then gamma/beta -= lr * grad.
-hipError_t launch_hidden_bwd(const HiddenBwdArgs& a, float* gamma, float* beta, const DevScalars* scalars,
-                             hipStream_t st);
-// Advance the step's dropout state by `draws` (after the forward).
-hipError_t launch_rng_advance(DevScalars* scalars, uint64_t draws, hipStream_t st);
+// One launch; gamma and beta are left for the step's extras tail to update.
+hipError_t launch_hidden_bwd(const HiddenBwdArgs& a, hipStream_t st);
 
 // Gradient clipping over every layer's delta (up to 16 buffers): the global
 // norm, scale = clip/norm when the norm exceeds clip (else 1, kept in
@@ -63,6 +63,33 @@ struct ClipArgs {
   DevScalars* scalars;   // receives clip_scale
 };
 constexpr int kClipBlocks = 256;
-hipError_t launch_clip(const ClipArgs& a, hipStream_t st);
+// The last pass of the clip (the partial sums are formed by the extras tail).
+hipError_t launch_clip_apply(const ClipArgs& a, hipStream_t st);
+
+// Sum of squares of every delta element, by block `block` of kClipBlocks (256
+// threads): a fixed contiguous range of the layers' deltas taken in layer
+// order; lanes add their strided elements, then a fixed butterfly and wave
+// order.  Into partials[block].
+__device__ __forceinline__ void clip_partial_block(const ClipArgs& a, int block, float* wave_part) {
+  int64_t total = 0;
+  for (int i = 0; i < a.n; ++i) total += a.count[i];
+  const int64_t chunk = (total + kClipBlocks - 1) / kClipBlocks;
+  const int64_t lo = (int64_t)block * chunk, hi = lo + chunk < total ? lo + chunk : total;
+  float s = 0.0f;
+  int layer = 0;
+  int64_t layer_lo = 0;
+  for (int64_t g = lo + threadIdx.x; g < hi; g += blockDim.x) {
+    while (g >= layer_lo + a.count[layer]) {
+      layer_lo += a.count[layer];
+      ++layer;
+    }
+    const float v = a.delta[layer][g - layer_lo];
+    s = s + v * v;
+  }
+  s = wave_sum(s);
+  if ((threadIdx.x & 63) == 0) wave_part[threadIdx.x >> 6] = s;
+  __syncthreads();
+  if (threadIdx.x == 0) a.partials[block] = wave_part[0] + wave_part[1] + wave_part[2] + wave_part[3];
+}
 
 }  // namespace volta

@@ -157,10 +157,10 @@ __global__ void __launch_bounds__(256) hidden_fwd_kernel(HiddenFwdArgs a) {
 // (:829-838).  A block covers 64 columns; wave w sums rows b = w, w + 4, ...
 // in batch order (its loads unrolled eight rows deep), and the four wave
 // partials are added in wave order.
-__global__ void __launch_bounds__(256) ln_bwd_cols_kernel(HiddenBwdArgs a) {
+__device__ __forceinline__ void ln_bwd_cols(const HiddenBwdArgs& a, int block) {
   __shared__ float pg[4][64], pb[4][64];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int j = blockIdx.x * 64 + lane;
+  const int j = block * 64 + lane;
   const int jj = j < a.c ? j : a.c - 1;  // loads stay in bounds; the store is guarded
   const float g = a.gamma[jj], be = a.beta[jj];
   float dg = 0.0f, db = 0.0f;
@@ -168,7 +168,7 @@ __global__ void __launch_bounds__(256) ln_bwd_cols_kernel(HiddenBwdArgs a) {
   for (int b = w; b < a.B; b += 4) {
     const size_t k = (size_t)b * a.c + jj;
     const float xh = (a.act[k] - be) / (g + 1e-12f);
-    const float dout = a.delta[k];
+    const float dout = a.din[k];
     dg = dg + dout * xh;
     db = db + dout;
   }
@@ -185,9 +185,10 @@ __global__ void __launch_bounds__(256) ln_bwd_cols_kernel(HiddenBwdArgs a) {
 // thread 0 in column order), dropout mask, activation derivative.  ReLU's
 // derivative takes the pre-activation (the output is no longer relu(pre));
 // sigmoid/tanh take the layer output as the reference does.
-__global__ void __launch_bounds__(256) hidden_bwd_rows_kernel(HiddenBwdArgs a) {
+__device__ __forceinline__ void hidden_bwd_row(const HiddenBwdArgs& a, int b) {
   __shared__ float part[4];
-  const int b = blockIdx.x, c = a.c;
+  const int c = a.c;
+  const float* din = a.din + (size_t)b * c;
   float* d = a.delta + (size_t)b * c;
   const float* y = a.act + (size_t)b * c;
   float sum_d = 0.0f, sum_dxh = 0.0f, is = 0.0f;
@@ -197,7 +198,7 @@ __global__ void __launch_bounds__(256) hidden_bwd_rows_kernel(HiddenBwdArgs a) {
     for (int j = threadIdx.x; j < c; j += blockDim.x) {
       const float g = a.gamma[j];
       const float xh = (y[j] - a.beta[j]) / (g + 1e-12f);
-      const float dout = d[j];
+      const float dout = din[j];
       s1 = s1 + dout * g;
       s2 = s2 + dout * g * xh;
     }
@@ -207,7 +208,7 @@ __global__ void __launch_bounds__(256) hidden_bwd_rows_kernel(HiddenBwdArgs a) {
   }
   const float* pre = a.pre + (size_t)b * c;
   for (int j = threadIdx.x; j < c; j += blockDim.x) {
-    float x = d[j];
+    float x = din[j];
     if (a.gamma) {
       const float g = a.gamma[j];
       const float xh = (y[j] - a.beta[j]) / (g + 1e-12f);
@@ -231,43 +232,16 @@ __global__ void __launch_bounds__(256) hidden_bwd_rows_kernel(HiddenBwdArgs a) {
   }
 }
 
-__global__ void __launch_bounds__(256) ln_update_kernel(float* gamma, float* beta, const float* dg, const float* db,
-                                                        int c, const DevScalars* s) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= c) return;
-  const float lr = s->lr;
-  gamma[j] = gamma[j] - lr * dg[j];
-  beta[j] = beta[j] - lr * db[j];
-}
-
-__global__ void rng_advance_kernel(DevScalars* s, uint64_t draws) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) s->rng = lcg_jump(s->rng, draws);
-}
-
-// Sum of squares of every delta element: block k covers a fixed contiguous
-// range of the layers' deltas taken in layer order; lanes add their strided
-// elements, then a fixed butterfly and wave order.
-__global__ void __launch_bounds__(256) clip_partials_kernel(ClipArgs a) {
-  __shared__ float wave_part[4];
-  int64_t total = 0;
-  for (int i = 0; i < a.n; ++i) total += a.count[i];
-  const int64_t chunk = (total + gridDim.x - 1) / gridDim.x;
-  const int64_t lo = (int64_t)blockIdx.x * chunk, hi = lo + chunk < total ? lo + chunk : total;
-  float s = 0.0f;
-  int layer = 0;
-  int64_t layer_lo = 0;
-  for (int64_t g = lo + threadIdx.x; g < hi; g += blockDim.x) {
-    while (g >= layer_lo + a.count[layer]) {
-      layer_lo += a.count[layer];
-      ++layer;
-    }
-    const float v = a.delta[layer][g - layer_lo];
-    s = s + v * v;
-  }
-  s = wave_sum(s);
-  if ((threadIdx.x & 63) == 0) wave_part[threadIdx.x >> 6] = s;
-  __syncthreads();
-  if (threadIdx.x == 0) a.partials[blockIdx.x] = wave_part[0] + wave_part[1] + wave_part[2] + wave_part[3];
+// Blocks [0, B) run the rows, the rest (LayerNorm) 64 columns each: both only
+// read `din`, and gamma and beta keep their values until the extras tail, so
+// they share a launch (column sums, rows and the gamma/beta update as three
+// launches a layer, rows in place, took the step of 512-1024-1024-512-256-1
+// with every extra 150.4 us at B=64, with this and the tail 113).
+__global__ void __launch_bounds__(256) hidden_bwd_kernel(HiddenBwdArgs a) {
+  // the dropout stream moves on once the step has drawn all its masks
+  if (a.rng_draws && blockIdx.x == 0 && threadIdx.x == 0) a.scalars->rng = lcg_jump(a.scalars->rng, a.rng_draws);
+  if ((int)blockIdx.x < a.B) hidden_bwd_row(a, blockIdx.x);
+  else ln_bwd_cols(a, blockIdx.x - a.B);
 }
 
 // The clip factor from the partial sums of squares (every block forms the
@@ -300,36 +274,20 @@ hipError_t launch_hidden_fwd(const HiddenFwdArgs& a, hipStream_t st) {
   return hipGetLastError();
 }
 
-hipError_t launch_hidden_bwd(const HiddenBwdArgs& a, float* gamma, float* beta, const DevScalars* scalars,
-                             hipStream_t st) {
-  const int cb = (a.c + 255) / 256;
-  if (a.gamma) {
-    hipLaunchKernelGGL(ln_bwd_cols_kernel, dim3((a.c + 63) / 64), dim3(256), 0, st, a);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-  }
-  hipLaunchKernelGGL(hidden_bwd_rows_kernel, dim3(a.B), dim3(256), 0, st, a);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess || !a.gamma) return e;
-  hipLaunchKernelGGL(ln_update_kernel, dim3(cb), dim3(256), 0, st, gamma, beta, a.dgamma, a.dbeta, a.c, scalars);
+hipError_t launch_hidden_bwd(const HiddenBwdArgs& a, hipStream_t st) {
+  if (a.gamma && (a.din == a.delta || !a.dgamma || !a.dbeta)) return hipErrorInvalidValue;
+  const int blocks = a.B + (a.gamma ? (a.c + 63) / 64 : 0);
+  hipLaunchKernelGGL(hidden_bwd_kernel, dim3(blocks), dim3(256), 0, st, a);
   return hipGetLastError();
 }
 
-hipError_t launch_rng_advance(DevScalars* scalars, uint64_t draws, hipStream_t st) {
-  hipLaunchKernelGGL(rng_advance_kernel, dim3(1), dim3(64), 0, st, scalars, draws);
-  return hipGetLastError();
-}
-
-hipError_t launch_clip(const ClipArgs& a, hipStream_t st) {
+hipError_t launch_clip_apply(const ClipArgs& a, hipStream_t st) {
   if (a.n < 1 || a.n > 16 || !a.partials || !a.scalars) return hipErrorInvalidValue;
   int64_t total = 0;
   for (int i = 0; i < a.n; ++i) {
     if (!a.delta[i] || a.count[i] < 1) return hipErrorInvalidValue;
     total += a.count[i];
   }
-  hipLaunchKernelGGL(clip_partials_kernel, dim3(kClipBlocks), dim3(256), 0, st, a);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
   const int blocks = (int)std::min<int64_t>((total + 255) / 256, 2048);
   hipLaunchKernelGGL(clip_apply_kernel, dim3(blocks), dim3(256), 0, st, a);
   return hipGetLastError();

@@ -6,6 +6,7 @@
 #include <algorithm>
 
 #include "device_common.h"
+#include "extras.h"
 #include "recorder.h"
 #include "skinny.h"
 
@@ -139,9 +140,30 @@ bool fwd_head_supported(const GemmPlan& p, const GemmArgs& a, const OutLayerArgs
 hipError_t launch_fwd_head(const GemmPlan& p, const GemmArgs& a, const OutLayerArgs& o, unsigned* strip_counters,
                            int n_counters, hipStream_t st);
 
-// b_i update (optimizer of EpiArgs: opt, b, bm, bv, bgrad, b1, b2, eps,
-// scalars) from db_i = the column sums of delta_i [B x N], b ascending.
-hipError_t launch_bias_update(const EpiArgs& e, const float* delta, int B, int N, hipStream_t st);
+// What a step with codegen extras does between its last delta and its dW
+// products, in one launch: the clip's partial sums of squares and, for steps
+// whose dW launches run without the fused column sums (clipping forms db from
+// the deltas before they are scaled, :936-955), b_i from db_i = the column
+// sums of delta_i [B x N]; gamma and beta -= lr * gradient of every LayerNorm.
+struct ExtrasTail {
+  ClipArgs clip{};                // n == 0: no clipping (then no bias updates)
+  int B = 0;
+  EpiArgs opt{};                  // the optimizer (opt, b1, b2, eps, scalars)
+  int n_bias = 0;
+  struct Bias {
+    const float* delta;
+    float *b, *bm, *bv, *bgrad;
+    int N;
+  } bias[VOLTA_MAX_LAYER_SIZES - 1];
+  int n_ln = 0;
+  struct Norm {
+    float *gamma, *beta;
+    const float *dgamma, *dbeta;
+    int c;
+  } ln[VOLTA_MAX_LAYER_SIZES - 1];
+};
+static_assert(sizeof(ExtrasTail) <= 4000, "ExtrasTail is passed by value as a kernel argument (4 KiB limit)");
+hipError_t launch_extras_tail(const ExtrasTail& t, hipStream_t st);
 
 // One operation of a paired launch (two independent operations of the
 // backward pass in one kernel launch: no buffer one writes is touched by the

@@ -3457,15 +3457,14 @@ GemmPlan gemm_plan(int layout, int M, int N, int K, bool vec, int num_cus, bool 
   return p;
 }
 
-// Bias update from db[n] = sum_b delta[b][n] (:931-933), for steps whose
-// dW launches run without the fused column sums (gradient clipping forms db
-// from the deltas before they are scaled, :936-955).  A block covers 64
+// Bias update from db[n] = sum_b delta[b][n] (:931-933).  A block covers 64
 // columns; wave w sums rows b = w, w + 4, ... in batch order (loads unrolled
 // eight rows deep), and the four partials are added in wave order.
-__global__ void __launch_bounds__(256) bias_update_kernel(EpiArgs e, const float* __restrict__ delta, int B, int N) {
+__device__ __forceinline__ void bias_update_block(const EpiArgs& e, const float* __restrict__ delta, int B, int N,
+                                                  int block) {
   __shared__ float part[4][64];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int n = blockIdx.x * 64 + lane;
+  const int n = block * 64 + lane;
   const int nn = n < N ? n : N - 1;  // loads stay in bounds; the update is guarded
   float db = 0.0f;
 #pragma unroll 8
@@ -3476,12 +3475,63 @@ __global__ void __launch_bounds__(256) bias_update_kernel(EpiArgs e, const float
     apply_bias_update(e, n, N, ((part[0][lane] + part[1][lane]) + part[2][lane]) + part[3][lane], adam_rcp_of(e));
 }
 
-hipError_t launch_bias_update(const EpiArgs& e, const float* delta, int B, int N, hipStream_t st) {
-  if (!e.b || !e.scalars || !delta || B < 1 || N < 1) return hipErrorInvalidValue;
+// Blocks: the clip's partial sums, then 64 columns of a bias each, then 256
+// elements of a LayerNorm each.  One launch of a step's independent small work
+// (one per bias and LayerNorm before: hidden_bwd_kernel has the figures).
+__global__ void __launch_bounds__(256) extras_tail_kernel(ExtrasTail t) {
+  __shared__ float wave_part[4];
+  int b = blockIdx.x;
+  if (t.clip.n > 0) {
+    if (b < kClipBlocks) {
+      clip_partial_block(t.clip, b, wave_part);
+      return;
+    }
+    b -= kClipBlocks;
+  }
+  for (int i = 0; i < t.n_bias; ++i) {  // block-uniform
+    const int blocks = (t.bias[i].N + 63) / 64;
+    if (b < blocks) {
+      EpiArgs e = t.opt;
+      e.b = t.bias[i].b;
+      e.bm = t.bias[i].bm;
+      e.bv = t.bias[i].bv;
+      e.bgrad = t.bias[i].bgrad;
+      bias_update_block(e, t.bias[i].delta, t.B, t.bias[i].N, b);
+      return;
+    }
+    b -= blocks;
+  }
+  for (int i = 0; i < t.n_ln; ++i) {
+    const int blocks = (t.ln[i].c + 255) / 256;
+    if (b < blocks) {
+      const int j = b * 256 + (int)threadIdx.x;
+      if (j >= t.ln[i].c) return;
+      const float lr = t.opt.scalars->lr;
+      t.ln[i].gamma[j] = t.ln[i].gamma[j] - lr * t.ln[i].dgamma[j];
+      t.ln[i].beta[j] = t.ln[i].beta[j] - lr * t.ln[i].dbeta[j];
+      return;
+    }
+    b -= blocks;
+  }
+}
+
+hipError_t launch_extras_tail(const ExtrasTail& t, hipStream_t st) {
+  int blocks = t.clip.n > 0 ? kClipBlocks : 0;
+  if (!t.opt.scalars || t.n_bias > VOLTA_MAX_LAYER_SIZES - 1 || t.n_ln > VOLTA_MAX_LAYER_SIZES - 1) return hipErrorInvalidValue;
+  if (t.clip.n < 0 || t.clip.n > 16 || (t.clip.n > 0 && !t.clip.partials)) return hipErrorInvalidValue;
+  for (int i = 0; i < t.clip.n; ++i)
+    if (!t.clip.delta[i] || t.clip.count[i] < 1) return hipErrorInvalidValue;
   // the state apply_bias_update reads: m for Adagrad, m and v for Adam and AdamW
-  const bool adam = e.opt == VOLTA_OPT_ADAM || e.opt == VOLTA_OPT_ADAMW;
-  if (e.opt != VOLTA_OPT_SGD && (!e.bm || (adam && !e.bv))) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(bias_update_kernel, dim3((N + 63) / 64), dim3(256), 0, st, e, delta, B, N);
+  const bool adam = t.opt.opt == VOLTA_OPT_ADAM || t.opt.opt == VOLTA_OPT_ADAMW;
+  for (int i = 0; i < t.n_bias; ++i) {
+    const auto& x = t.bias[i];
+    if (!x.b || !x.delta || t.B < 1 || x.N < 1) return hipErrorInvalidValue;
+    if (t.opt.opt != VOLTA_OPT_SGD && (!x.bm || (adam && !x.bv))) return hipErrorInvalidValue;
+    blocks += (x.N + 63) / 64;
+  }
+  for (int i = 0; i < t.n_ln; ++i) blocks += (t.ln[i].c + 255) / 256;
+  if (!blocks) return hipSuccess;
+  hipLaunchKernelGGL(extras_tail_kernel, dim3(blocks), dim3(256), 0, st, t);
   return hipGetLastError();
 }
 

@@ -153,6 +153,7 @@ struct Handle {
   std::vector<float*> ln_dg, ln_db;  // gradients [L[i+1]]
   std::vector<uint8_t*> mask;        // dropout keep mask [B x L[i+1]]
   float* clip_partials = nullptr;    // [kClipBlocks]
+  float* ext_din = nullptr;          // LayerNorm: dL/d(layer output) of the layer being passed [B x widest]
   bool hidden_ext() const { return ext_ln || ext_drop || ext_softmax; }
   bool extras() const { return hidden_ext() || ext_clip; }
   // activation of the hidden layers' GEMM epilogue (softmax runs after it)
@@ -555,12 +556,6 @@ static bool enqueue_step(Handle* h, hipStream_t st, Recorder* rec = nullptr) {
       VOLTA_CHECK(launch_hidden_fwd(hidden_fwd_args(h, i, B, true), st));
       std::snprintf(label, sizeof label, "fwd%d.ln_dropout", i);
       VOLTA_CHECK(mark(rec, label, 0.0, 4.0 * 3.0 * B * lp.c));
-      if (h->ext_drop && i == n - 2) {
-        uint64_t draws = 0;
-        for (int k = 0; k < n - 1; ++k) draws += (uint64_t)B * h->L[k + 1];
-        VOLTA_CHECK(launch_rng_advance(h->scalars, draws, st));
-        VOLTA_CHECK(mark(rec, "rng_advance", 0.0, 0.0));
-      }
     }
   }
   if (h->out_mode == OUT_GEMM) {  // output layer wider than one tile: stand-alone loss head
@@ -609,21 +604,25 @@ static bool enqueue_step(Handle* h, hipStream_t st, Recorder* rec = nullptr) {
   if (h->extras()) {
     // Codegen extras (:824-892, :936-955).  Phase 1, i = n-1 .. 0: the
     // hidden layer's LayerNorm backward, dropout mask and f' (its dX ran
-    // with the identity derivative), b_i from db_i when clipping (db comes
-    // from the unscaled deltas), dX_i.  Then the clip scales every delta,
-    // and phase 2 runs dW_i (W_i only when clipping).  No paired launches:
-    // the clip needs every delta before the first dW.
+    // with the identity derivative, with LayerNorm into ext_din), dX_i.  Then
+    // one launch updates every gamma and beta and, when clipping, b_i from
+    // db_i (which comes from the unscaled deltas) and sums the squares; the
+    // clip scales every delta, and phase 2 runs dW_i (W_i only when
+    // clipping).  No paired launches: the clip needs every delta before the
+    // first dW.
     const int dx_act = h->hidden_ext() ? kIdentity : s.activation;
     for (int i = n - 1; i >= 0; --i) {
       const LayerPlan& lp = h->layers[i];
       if (i != n - 1 && h->hidden_ext()) {
         HiddenBwdArgs a{};
+        a.din = h->ext_ln ? h->ext_din : h->delta[i];
         a.delta = h->delta[i];
         a.act = h->act[i + 1];
         a.pre = h->pre[i];
         a.B = B;
         a.c = lp.c;
         a.act_kind = s.activation;
+        a.scalars = h->scalars;
         if (h->ext_ln) {
           a.gamma = h->ln_g[i];
           a.beta = h->ln_b[i];
@@ -634,53 +633,60 @@ static bool enqueue_step(Handle* h, hipStream_t st, Recorder* rec = nullptr) {
         if (h->ext_drop) {
           a.mask = h->mask[i];
           a.keep_scale = 1.0f / (1.0f - s.dropout_p);
+          if (i == 0)  // the step's last layer pass: the stream moves on
+            for (int k = 0; k < n - 1; ++k) a.rng_draws += (uint64_t)B * h->L[k + 1];
         }
-        VOLTA_CHECK(launch_hidden_bwd(a, h->ext_ln ? h->ln_g[i] : nullptr, h->ext_ln ? h->ln_b[i] : nullptr,
-                                      h->scalars, st));
+        VOLTA_CHECK(launch_hidden_bwd(a, st));
         std::snprintf(lx, sizeof lx, "bwd%d.ln_dropout", i);
         VOLTA_CHECK(mark(rec, lx, 0.0, 4.0 * 5.0 * B * lp.c));
       }
-      if (h->ext_clip) {
-        EpiArgs e{};
-        e.opt = s.optimizer == VOLTA_OPT_ADAMW ? VOLTA_OPT_ADAM : s.optimizer;
-        e.b = h->params + lp.b_off;
-        e.bm = h->opt_a ? h->opt_a + lp.b_off : nullptr;
-        e.bv = h->opt_b ? h->opt_b + lp.b_off : nullptr;
-        e.bgrad = h->keep_grads ? h->grads + lp.b_off : nullptr;
-        e.b1 = s.beta1;
-        e.b2 = s.beta2;
-        e.eps = s.eps;
-        e.scalars = h->scalars;
-        VOLTA_CHECK(launch_bias_update(e, h->delta[i], B, lp.c, st));
-        std::snprintf(lx, sizeof lx, "db%d+opt", i);
-        VOLTA_CHECK(mark(rec, lx, (double)B * lp.c, 4.0 * B * lp.c));
-      }
       if (i == 0) break;
       std::snprintf(lx, sizeof lx, "dx%d", i);
+      float* dx_out = h->ext_ln ? h->ext_din : h->delta[i - 1];
       if (i == n - 1 && h->narrow_dx) {
         VOLTA_CHECK(launch_outer_dx(h->delta[i], h->params + lp.w_off, B, lp.r, lp.c, dx_act, h->act[i],
-                                    h->pre[i - 1], h->delta[i - 1], st));
+                                    h->pre[i - 1], dx_out, st));
         VOLTA_CHECK(mark(rec, lx, dx_cost(i).first, dx_cost(i).second));
       } else {
         PairOp o = make_dx(i, ws0);
         o.args.epi.act = dx_act;
+        o.args.epi.out = dx_out;
         if (!run_single(o, lx, dx_cost(i))) return false;
       }
     }
-    if (h->ext_clip) {
-      ClipArgs c{};
-      c.n = n;
-      for (int i = 0; i < n; ++i) {
-        c.delta[i] = h->delta[i];
-        c.count[i] = (int64_t)B * h->L[i + 1];
-      }
-      c.clip = s.clip_grad;
-      c.partials = h->clip_partials;
-      c.scalars = h->scalars;
-      VOLTA_CHECK(launch_clip(c, st));
+    if (h->ext_ln || h->ext_clip) {
+      ExtrasTail t;
+      t.B = B;
+      t.opt.opt = s.optimizer == VOLTA_OPT_ADAMW ? VOLTA_OPT_ADAM : s.optimizer;
+      t.opt.b1 = s.beta1;
+      t.opt.b2 = s.beta2;
+      t.opt.eps = s.eps;
+      t.opt.scalars = h->scalars;
+      for (int i = 0; i < n - 1 && h->ext_ln; ++i)
+        t.ln[t.n_ln++] = {h->ln_g[i], h->ln_b[i], h->ln_dg[i], h->ln_db[i], h->L[i + 1]};
       double cnt = 0.0;
-      for (int i = 0; i < n; ++i) cnt += (double)B * h->L[i + 1];
-      VOLTA_CHECK(mark(rec, "clip", 3.0 * cnt, 12.0 * cnt));
+      for (int i = 0; i < n && h->ext_clip; ++i) {
+        const LayerPlan& lp = h->layers[i];
+        t.bias[t.n_bias++] = {h->delta[i],
+                              h->params + lp.b_off,
+                              h->opt_a ? h->opt_a + lp.b_off : nullptr,
+                              h->opt_b ? h->opt_b + lp.b_off : nullptr,
+                              h->keep_grads ? h->grads + lp.b_off : nullptr,
+                              lp.c};
+        t.clip.delta[i] = h->delta[i];
+        t.clip.count[i] = (int64_t)B * lp.c;
+        cnt += (double)B * lp.c;
+      }
+      t.clip.n = h->ext_clip ? n : 0;
+      t.clip.clip = s.clip_grad;
+      t.clip.partials = h->clip_partials;
+      t.clip.scalars = h->scalars;
+      VOLTA_CHECK(launch_extras_tail(t, st));
+      VOLTA_CHECK(mark(rec, "extras_tail", 2.0 * cnt, 8.0 * cnt));
+      if (h->ext_clip) {
+        VOLTA_CHECK(launch_clip_apply(t.clip, st));
+        VOLTA_CHECK(mark(rec, "clip", cnt, 8.0 * cnt));
+      }
     }
     // phase 2: every dW (W only when clipping: b_i took its update above)
     auto ext_dw = [&](int i) {
@@ -1043,6 +1049,7 @@ static bool build(Handle* h) {
     if (h->ext_drop) req((void**)&h->mask[i], (size_t)B * c);
   }
   if (h->ext_clip) req((void**)&h->clip_partials, kClipBlocks * 4);
+  if (h->ext_ln) req((void**)&h->ext_din, (size_t)B * *std::max_element(h->L.begin() + 1, h->L.end() - 1) * 4);
   for (int i = 0; i < n; ++i) req((void**)&h->delta[i], (size_t)B * h->L[i + 1] * 4);
   if (ws_floats) req((void**)&h->gemm_ws, ws_floats * 4);
   req((void**)&h->counters, (size_t)(h->n_counters + 1) * sizeof(unsigned));  // + the input launch's
