@@ -96,8 +96,8 @@ struct GemmPlan {
   size_t workspace_floats(int M, int N) const { return splits > 1 ? (size_t)splits * (M + 1) * N : 0; }
 };
 
-// Tile and split-K plan of one product.  `small_m`: the small-M tile may be
-// chosen (NN/NT products whose epilogue is per element: not the loss head).
+// Tile and split-K plan of one product.  `small_m`: the tiles that finish
+// whole outputs in one launch (small-M, K groups, 128x64) may be chosen.
 GemmPlan gemm_plan(int layout, int M, int N, int K, bool vec, int num_cus, bool small_m = true);
 // TILE_NARROW_TN's K slice (a multiple of 4, at most 128) and split count
 // for an M x N x K product on num_cus CUs.

@@ -3335,7 +3335,7 @@ GemmPlan gemm_plan(int layout, int M, int N, int K, bool vec, int num_cus, bool 
   const int bk = p.tile == TILE_64x64_K64 ? 64 : 32;
   // Smallest K slice (VOLTA_SPLITK_MIN_K): 128, and 64 for a forward product
   // with few enough rows for the small-M tile below (a plan that splits K is
-  // what sends it there, K >= 128; the loss-head GEMM of those batches too).
+  // what sends it there, K >= 128).
   // 64 for every forward product split C4 B=1024's fwd3 (1024 x 256, K =
   // 512, 64 tiles) eight ways instead of four: 0.2398 -> 0.2380 ms/step with
   // 128, the reduce reading half the planes.
@@ -3423,9 +3423,7 @@ GemmPlan gemm_plan(int layout, int M, int N, int K, bool vec, int num_cus, bool 
   // (fwd2 17.8 -> 25.8 us), the dW pairs and a short-K dX pair are faster
   // paired, and 128x128 tiles lose their second workgroup per CU (C5 4.63
   // -> 4.64 ms).  VOLTA_KGROUPS=1 takes them wherever they apply, 0
-  // nowhere.  Only where the epilogue is per element (small_m is false for
-  // the loss-head product); such a product launches on its own, never in a
-  // paired launch.
+  // nowhere.  Such a product launches on its own, never in a paired launch.
   const char* kg = std::getenv("VOLTA_KGROUPS");
   const int kg_max = p.tile == TILE_64x64 && layout != GEMM_TN ? 4 : p.tile == TILE_64x64 || p.tile == TILE_128x128 ? 2 : 1;
   const bool kg_auto = !(kg && *kg) && (layout == GEMM_NN || (layout == GEMM_NT && K >= 1024)) &&
