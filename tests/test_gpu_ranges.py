@@ -8,7 +8,7 @@ import numpy as np
 import pytest
 
 from tests.oracle_lib import load_oracle
-from tests.test_gpu_parity import assert_params_close, close_enough, run_steps, say
+from tests.test_gpu_parity import _launch_labels, assert_params_close, close_enough, run_steps, say
 from volta_amd import DeviceArray, data, load_hip
 from volta_amd.abi import STATUS_BAD_ARGUMENT, STATUS_NONFINITE_LOSS, MlpSpec, Trainer
 
@@ -227,3 +227,15 @@ def test_mid_tile_step(sizes, B, act):
 def test_extras_launches(sizes, B, extras):
     say(f"extras {sizes} B={B} {extras}")
     against_oracle(MlpSpec(sizes, "tanh", "sgd", **extras), B)
+
+
+# Nine weight layers with an output of a few columns: every dW in one launch
+# (the most products a group holds), also with the codegen extras.
+@pytest.mark.parametrize("B", [7, 256])
+@pytest.mark.parametrize("extras", [{}, dict(dropout_p=0.2, clip_grad=0.5)])
+def test_dw_group_of_nine(B, extras):
+    say(f"dW group of nine layers B={B} {extras}")
+    spec = MlpSpec([20, 24, 16, 33, 40, 16, 24, 20, 12, 3], "tanh", "sgd", **extras)
+    dws = [label for label in _launch_labels({}, spec, B) if label.startswith("dw")]
+    assert len(dws) == 1 and dws[0].count("|") == 8, dws
+    against_oracle(spec, B)
