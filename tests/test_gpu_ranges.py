@@ -27,6 +27,52 @@ def against_oracle(spec, B, lr=0.01, steps=3, seed=7):
     assert_params_close(wh, bh, wo, bo, spec.text())
 
 
+def resumed_run(lib, spec, B, lr, steps=3, seed=7):
+    """Losses, parameters and optimizer state after `steps` steps from an optimizer state 1000 steps old:
+    first moments of about 1e-3, second ones of about 1e-6 (Adagrad: 1e-4).  A weight moves by about lr a
+    step, whatever its gradient, and by an error of a gradient e by about 100 lr e."""
+    ws, bs = data.he_uniform(seed, spec.sizes)
+    t = Trainer(lib, spec, B)
+    t.set_all_params(ws, bs)
+    rng, parts = np.random.default_rng(seed), []
+    for a in [x for pair in zip(ws, bs) for x in pair]:
+        parts.append((1e-3 * rng.standard_normal(a.size), (1e-4 if spec.optimizer == "adagrad" else 1e-6) *
+                      (0.5 + rng.random(a.size))))
+    state = []
+    for i in range(0, len(parts), 2):  # per layer: the moments of W and b, then their second moments
+        if spec.optimizer in ("adam", "adamw"):
+            state += [parts[i][0], parts[i + 1][0]]
+        if spec.optimizer != "sgd":
+            state += [parts[i][1], parts[i + 1][1]]
+    if state:
+        t.set_state(np.concatenate(state).astype(np.float32), 1000)
+    losses = []
+    for s in range(steps):
+        t.step(*data.batch(seed + 1 + s, spec.sizes, B, spec.loss), lr)
+        losses.append(t.loss())
+    out = losses, *t.get_params(), t.get_state()[0]
+    assert t.status() == 0
+    t.close()
+    return out
+
+
+def resumed_against_oracle(spec, B, lr=1e-3, steps=3):
+    """A resumed run, HIP against oracle: the state within rel 1e-4 and 1e-4 of its rms (what a step adds to it is
+    a gradient's share, which differs by some 1e-6 of the gradients' rms)."""
+    lh, wh, bh, sh = resumed_run(load_hip(), spec, B, lr, steps)
+    lo, wo, bo, so = resumed_run(load_oracle(), spec, B, lr, steps)
+    ok, mx, _ = close_enough(lh, lo)
+    assert ok, f"losses differ, max abs {mx:.3e}\n hip={lh}\n ora={lo}"
+    assert_params_close(wh, bh, wo, bo, spec.text())
+    pos = 0
+    for r, c in spec.shapes() if so.size else []:
+        for n in (r * c, c) * (so.size // sum(r * c + c for r, c in spec.shapes())):
+            a, b = sh[pos:pos + n], so[pos:pos + n]
+            ok, mx, bad = close_enough(a, b, 1e-4, 1e-4 * float(np.sqrt(np.mean(b.astype(np.float64) ** 2))))
+            assert ok, f"{spec.text()}: state at {pos}: {bad} of {n} differ, max abs {mx:.3e}"
+            pos += n
+
+
 # Stand-alone loss heads (more than 64 outputs): one wave per row, rows of up
 # to 64, 128, 256 and 1024 columns in registers and longer ones read again;
 # four rows per block, several rows per wave above 4096 rows.
@@ -239,3 +285,22 @@ def test_dw_group_of_nine(B, extras):
     dws = [label for label in _launch_labels({}, spec, B) if label.startswith("dw")]
     assert len(dws) == 1 and dws[0].count("|") == 8, dws
     against_oracle(spec, B)
+
+
+# dW groups of aligned and ragged products (an output of a few columns, a
+# ragged first or middle layer), on 32x32 and 32x64 tiles: bit for bit the
+# products launched one by one, each in its own form.
+@pytest.mark.parametrize("sizes,B", [([32, 64, 96, 10], 64), ([30, 64, 128, 4], 33), ([64, 33, 32, 8], 256),
+                                     ([20, 48, 16, 3], 1), ([132, 260, 68, 2], 130)])
+@pytest.mark.parametrize("tile_n", ["32", "64"])
+@pytest.mark.parametrize("opt", ["adam", "adagrad"])
+def test_dw_group_mixed_forms(monkeypatch, sizes, B, tile_n, opt):
+    say(f"mixed dW group {sizes} B={B} tile_n={tile_n} {opt}")
+    spec = MlpSpec(sizes, "tanh", opt)
+    monkeypatch.setenv("VOLTA_DW_GROUP_TN", tile_n)
+    resumed_against_oracle(spec, B)
+    _, w0, b0, s0 = resumed_run(load_hip(), spec, B, 1e-3)
+    monkeypatch.setenv("VOLTA_NO_PAIR", "1")
+    _, w1, b1, s1 = resumed_run(load_hip(), spec, B, 1e-3)
+    for a, b in zip(w0 + b0 + [s0], w1 + b1 + [s1]):
+        np.testing.assert_array_equal(a, b)

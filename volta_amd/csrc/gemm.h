@@ -200,6 +200,7 @@ struct DwGroup {
   int n = 0;                        // small-K dW products (plan TILE_DW_SMALLK)
   GemmArgs g[kMaxDwGroup];
   int start[kMaxDwGroup + 1] = {};  // first workgroup of product i after the narrow ones; start[n] = total
+  unsigned ragged = 0;              // bit i: product i's rows may not be 16-byte aligned (set by the launch)
   int tile_n = 32;                  // columns of the small-K tiles: 32, or 64 (the wide form, same results)
   int narrow_blocks = 0;            // 0: no narrow dW
   NarrowDwArgs nd{};

@@ -2084,7 +2084,9 @@ static_assert(kDwT * (kDwTW + 1) <= kDwK * kDwS, "the wide dW tile fits over the
 // inside their row where they would pass its end (put right when the slice is
 // stored), the tile's float4 of W, m and v likewise, and rows of fewer than 4
 // elements are loaded one by one: same products, same order.
-template <int EPI, int TN = kDwT, bool VEC = true>
+//
+// LATE: all of W, m and v are loaded after the product (fewer registers).
+template <int EPI, int TN = kDwT, bool VEC = true, bool LATE = false>
 __device__ __forceinline__ void dw_smallk_tile(const GemmArgs& args, int blk, float* lds, int tid) {
   static_assert(EPI == EPI_DW_OPT || EPI == EPI_STORE, "epilogues of the dW tile");
   static_assert(TN == kDwT || TN == kDwTW, "tile widths of the dW tile");
@@ -2197,7 +2199,7 @@ __device__ __forceinline__ void dw_smallk_tile(const GemmArgs& args, int blk, fl
   // the state loaded before the product (all of it in the 32-wide form; the
   // wide form's second float4 after it, which keeps the kernel within five
   // waves per SIMD without spills)
-  constexpr int EARLY = TN == kDwT ? EIT : 1;
+  constexpr int EARLY = LATE ? 0 : TN == kDwT ? EIT : 1;
   auto load_state = [&](int j) {
     if constexpr (VEC) {
       w4[j] = *reinterpret_cast<const floatx4*>(e.out + o[j]);
@@ -3165,10 +3167,19 @@ static hipError_t reduce_after(const PairOp& o, hipStream_t st) {
 // workgroups [start[i], start[i+1]) after them.
 static_assert(sizeof(DwGroup) <= 4000, "DwGroup is passed by value as a kernel argument (4 KiB limit)");
 
-// Five waves per SIMD (at most 96 registers); four where a product's rows are
-// not 16-byte aligned (VEC false: every product then takes that form).
-template <int TN, bool VEC>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VEC ? 5 : 4))) dw_group_kernel(DwGroup d) {
+// Each product takes its own form of the tile (d.ragged: rows that may not be
+// 16-byte aligned), chosen per workgroup where a group has both.  One form for
+// all put the 2048-wide products of 512-2048-2048-512-3 on moved-back loads
+// for its output layer's sake: Adam at B=128 124.3 us a step, 119.3 with a
+// form each (118.3 with 4 outputs, where every product is aligned); SGD 114.7
+// and 110.0; 512-2048-2048-512-10 128.6 and 123.6.
+// Five waves per SIMD (at most 96 registers); the ragged 32x64 form alone
+// takes 106 and runs at four, and beside the aligned one loads its state late
+// to stay within 94.
+enum DwForm { DW_ALIGNED = 0, DW_RAGGED = 1, DW_MIXED = 2 };
+template <int TN, int FORM>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FORM == DW_RAGGED ? 4 : 5)))
+dw_group_kernel(DwGroup d) {
   __shared__ __attribute__((aligned(16))) float lds[TN == kDwT ? kDwLds : (kDwLdsW > kDwLds ? kDwLdsW : kDwLds)];
   int b = blockIdx.x;
   if (b == 0 && threadIdx.x == 0 && d.loss_partials)
@@ -3182,38 +3193,49 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VEC ? 
 #pragma unroll
   for (int k = 1; k < kMaxDwGroup; ++k)
     if (k < d.n && b >= d.start[k]) i = k;
-  dw_smallk_tile<EPI_DW_OPT, TN, VEC>(d.g[i], b - d.start[i], lds, threadIdx.x);
+  if (FORM == DW_RAGGED || (FORM == DW_MIXED && (d.ragged >> i & 1u)))  // workgroup-uniform
+    dw_smallk_tile<EPI_DW_OPT, TN, false, FORM == DW_MIXED && TN == kDwTW>(d.g[i], b - d.start[i], lds, threadIdx.x);
+  else
+    dw_smallk_tile<EPI_DW_OPT, TN, true>(d.g[i], b - d.start[i], lds, threadIdx.x);
 }
 
 int dw_group_tiles(const GemmArgs& a, int tile_n) {
   return ((a.M + kDwT - 1) / kDwT) * ((a.N + tile_n - 1) / tile_n);
 }
 
-static bool dw_group_vec(const DwGroup& d) {
-  for (int i = 0; i < d.n; ++i)
-    if (!dw_smallk_vec(d.g[i])) return false;
-  return true;
+// Bit i: product i takes the ragged form.
+static unsigned dw_group_ragged(const DwGroup& d) {
+  unsigned m = 0;
+  for (int i = 0; i < d.n; ++i) m |= dw_smallk_vec(d.g[i]) ? 0u : 1u << i;
+  return m;
 }
 
-// The group kernel for tile width `tile_n` (as dw_group_launch selects it).
-static const void* dw_group_fn(bool vec, int tile_n) {
+// The group kernel for tile width `tile_n` and the products' forms.
+typedef void (*DwGroupFn)(DwGroup);
+static DwGroupFn dw_group_fn(const DwGroup& d, int tile_n) {
+  const unsigned ragged = dw_group_ragged(d);
+  const int form = ragged == 0 ? DW_ALIGNED : ragged == (1u << d.n) - 1u ? DW_RAGGED : DW_MIXED;
   if (tile_n == kDwTW)
-    return vec ? reinterpret_cast<const void*>(&dw_group_kernel<kDwTW, true>)
-               : reinterpret_cast<const void*>(&dw_group_kernel<kDwTW, false>);
-  return vec ? reinterpret_cast<const void*>(&dw_group_kernel<kDwT, true>)
-             : reinterpret_cast<const void*>(&dw_group_kernel<kDwT, false>);
+    return form == DW_ALIGNED  ? dw_group_kernel<kDwTW, DW_ALIGNED>
+           : form == DW_RAGGED ? dw_group_kernel<kDwTW, DW_RAGGED>
+                               : dw_group_kernel<kDwTW, DW_MIXED>;
+  return form == DW_ALIGNED  ? dw_group_kernel<kDwT, DW_ALIGNED>
+         : form == DW_RAGGED ? dw_group_kernel<kDwT, DW_RAGGED>
+                             : dw_group_kernel<kDwT, DW_MIXED>;
 }
 
 int dw_group_pick_tile_n(const DwGroup& d, int num_cus) {
-  const bool vec = dw_group_vec(d);
   int t32 = d.narrow_blocks, t64 = d.narrow_blocks;
   for (int i = 0; i < d.n; ++i) {
     t32 += dw_group_tiles(d.g[i], kDwT);
     t64 += dw_group_tiles(d.g[i], kDwTW);
   }
   int r32 = 0, r64 = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&r32, dw_group_fn(vec, kDwT), 256, 0) != hipSuccess ||
-      hipOccupancyMaxActiveBlocksPerMultiprocessor(&r64, dw_group_fn(vec, kDwTW), 256, 0) != hipSuccess ||
+  const auto resident = [&](int* r, int tile_n) {
+    return hipOccupancyMaxActiveBlocksPerMultiprocessor(r, reinterpret_cast<const void*>(dw_group_fn(d, tile_n)), 256,
+                                                        0);
+  };
+  if (resident(&r32, kDwT) != hipSuccess || resident(&r64, kDwTW) != hipSuccess ||
       r32 < 1 || r64 < 1) {
     (void)hipGetLastError();
     return kDwT;
@@ -3243,14 +3265,9 @@ hipError_t dw_group_launch(const DwGroup& d, hipStream_t st, Recorder* rec, cons
                            double bytes) {
   if (!dw_group_supported(d)) return hipErrorInvalidValue;
   const dim3 grid(d.narrow_blocks + d.start[d.n]);
-  const bool vec = dw_group_vec(d);  // (the same selection as dw_group_fn)
-  if (d.tile_n == kDwTW) {
-    if (vec) hipLaunchKernelGGL((dw_group_kernel<kDwTW, true>), grid, dim3(256), 0, st, d);
-    else hipLaunchKernelGGL((dw_group_kernel<kDwTW, false>), grid, dim3(256), 0, st, d);
-  } else {
-    if (vec) hipLaunchKernelGGL((dw_group_kernel<kDwT, true>), grid, dim3(256), 0, st, d);
-    else hipLaunchKernelGGL((dw_group_kernel<kDwT, false>), grid, dim3(256), 0, st, d);
-  }
+  DwGroup g = d;
+  g.ragged = dw_group_ragged(d);
+  hipLaunchKernelGGL(dw_group_fn(d, d.tile_n), grid, dim3(256), 0, st, g);
   const hipError_t err = hipGetLastError();
   if (err != hipSuccess) return err;
   return mark(rec, label, flops, bytes);
