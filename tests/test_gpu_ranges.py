@@ -304,3 +304,35 @@ def test_dw_group_mixed_forms(monkeypatch, sizes, B, tile_n, opt):
     _, w1, b1, s1 = resumed_run(load_hip(), spec, B, 1e-3)
     for a, b in zip(w0 + b0 + [s0], w1 + b1 + [s1]):
         np.testing.assert_array_equal(a, b)
+
+
+# A handle's staging memory is pinned with the handle: host-fed steps and host
+# inference of any row count, in turn, pin nothing and use the same slots (four
+# of a ring, two, one above 1 MiB) without disturbing each other.
+@pytest.mark.parametrize("L0,B,Ln", [(5, 3, 2), (100, 257, 9), (300, 900, 3), (16, 900, 300)])
+def test_staging_is_the_handles(L0, B, Ln):
+    say(f"staging L0={L0} B={B} Ln={Ln}")
+    lib = load_hip()
+    pinned = lib.lib.volta_hip_pinned_allocations
+    spec = MlpSpec([L0, 24, Ln], "tanh", "sgd")
+    ws, bs = data.he_uniform(5, spec.sizes)
+    batches = [data.batch(60 + s, spec.sizes, B, "mse") for s in range(7)]
+    X = data.normal(8, (2 * B + 3, L0))
+    got = []
+    for infer in (False, True):
+        t = Trainer(lib, spec, B)
+        before = pinned()
+        t.set_all_params(ws, bs)
+        for s, (x, y) in enumerate(batches):
+            t.step(x, y, 0.05)
+            if infer:
+                t.infer(X[: 1 + s * X.shape[0] // 7])
+        out = t.infer(X)
+        assert pinned() == before
+        got.append((out, t.loss(), *t.get_params()))
+        assert t.status() == 0
+        t.close()
+    (o0, l0, w0, b0), (o1, l1, w1, b1) = got
+    assert l0 == l1
+    for a, b in zip([o0] + w0 + b0, [o1] + w1 + b1):
+        np.testing.assert_array_equal(a, b)

@@ -26,6 +26,7 @@ HIP_EXTRA = {
                                    C.c_int32, C.c_int32, C.c_int32, C.c_int32, C.c_int32]),
     "volta_hip_gemm_plan": (C.c_int32, [C.c_int32] * 7 + [C.POINTER(C.c_int32)]),
     "volta_hip_arena_bytes": (C.c_int64, [C.c_void_p]),
+    "volta_hip_pinned_allocations": (C.c_int64, []),
     "volta_hip_optimizer": (C.c_int32, [C.c_int32, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int64]
                             + [C.c_float] * 7),
     "volta_hip_profile_step": (C.c_int32, [C.c_void_p, C.c_int32, C.c_char_p, C.c_int32]),

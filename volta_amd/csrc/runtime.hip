@@ -41,6 +41,7 @@
 // weights, as in the reference's two-phase backward.
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -132,8 +133,6 @@ struct Handle {
   std::vector<GemmPlan> infer_plans;  // of the row count inferred last
   int infer_plan_rows = 0;
   size_t infer_plan_ws = 0;
-  char* infer_stage = nullptr;  // pinned [X | out] of a chunk of inference rows
-  size_t infer_stage_bytes = 0;
   float* infer_ws = nullptr;   // split-K workspace of inference plans (grown on demand)
   float* scratch = nullptr;    // this device's static scratch (allocation-free inference)
   bool dx_alone = false;       // small-batch backward: dX launches alone, dW products grouped
@@ -172,7 +171,8 @@ struct Handle {
   // Pinned staging of host-fed steps, slots of [X | gap | Y]: a ring read by
   // the step's input launch, which reports the number of the step whose slot
   // it has read in *stage_done; or, for large inputs, one slot read by a copy
-  // engine (stage_free: it may be overwritten).
+  // engine (stage_free: it may be overwritten).  Host inference takes a slot
+  // likewise, with the output rows in the place of Y.
   char* h_stage = nullptr;
   size_t stage_bytes = 0, stage_y_off = 0;  // of one slot; of Y in it
   int stage_slots = 1;
@@ -201,7 +201,6 @@ Handle::~Handle() {
   if (stage_free) (void)hipEventDestroy(stage_free);
   if (h_params) (void)hipHostFree(h_params);
   if (h_stage) (void)hipHostFree(h_stage);
-  if (infer_stage) (void)hipHostFree(infer_stage);
   if (h_lr) (void)hipHostFree(h_lr);
   if (bc_table) (void)hipFree(bc_table);
   if (infer_x) (void)hipFree(infer_x);
@@ -873,7 +872,15 @@ static float* scratch_address(int dev) {
 
 constexpr size_t kStageRingMax = (size_t)1 << 20;  // largest staging slot of the ring
 
-static bool build(Handle* h) {
+static std::atomic<int64_t> g_pinned_allocs{0};  // pinned_alloc calls (test hook)
+// Pinned host memory.  All of a handle's is allocated with the handle: pinning
+// takes longer than a small call (70 to 330 us of a first host-fed step).
+static hipError_t pinned_alloc(void** p, size_t bytes, unsigned flags) {
+  g_pinned_allocs.fetch_add(1);
+  return hipHostMalloc(p, bytes, flags);
+}
+
+static bool build(Handle* h, bool infer_only) {
   const volta_mlp_spec& s = h->spec;
   const int n = h->n, B = h->B;
   VOLTA_CHECK(hipGetDevice(&h->device));
@@ -1069,18 +1076,24 @@ static bool build(Handle* h) {
   if (!make_bc_table(h)) return false;
 
   // Host side: pinned parameter mirror, input staging, lr slots.
-  VOLTA_CHECK(hipHostMalloc((void**)&h->h_params, (size_t)h->flat * 4, hipHostMallocDefault));
+  VOLTA_CHECK(pinned_alloc((void**)&h->h_params, (size_t)h->flat * 4, hipHostMallocDefault));
   // Staging slots [X | gap | Y], laid out as act_0 and the targets are in the
   // arena.  Up to 1 MiB a ring that the input launch reads (four slots while
-  // they fit 256 KiB, else two): the host runs ahead of the GPU, and no copy engine has to be handed the stream and
-  // hand it back (256-512-512-256-1 at B=64: 47.4 -> 34.1 us a step,
-  // 300-1655-200-17 at B=629, 0.8 MB a step: 205 -> 196).  Past that one slot
-  // for a copy engine, whose 57 GB/s a kernel's reads of host memory do not
-  // reach (33 MB a step: 1790 us against 1920).
+  // they fit 256 KiB, else two): the host runs ahead of the GPU, and no copy
+  // engine has to be handed the stream and hand it back (256-512-512-256-1 at
+  // B=64: 47.4 -> 34.1 us a step, 300-1655-200-17 at B=629, 0.8 MB a step:
+  // 205 -> 196).  Past that one slot for a copy engine, whose 57 GB/s a
+  // kernel's reads of host memory do not reach (33 MB a step: 1790 us against
+  // 1920).  An inference model's calls wait for their results: one slot.
   h->stage_y_off = align_up((size_t)B * h->L[0] * 4, 256);
   h->stage_bytes = align_up(h->stage_y_off + (size_t)B * std::max(h->L[n], 1) * 4, 256);
-  h->stage_slots = h->stage_bytes > kStageRingMax ? 1 : 4 * h->stage_bytes <= kStageRingMax / 4 ? 4 : 2;
-  VOLTA_CHECK(hipHostMalloc((void**)&h->h_lr, Handle::kLrSlots * sizeof(float), hipHostMallocDefault));
+  h->stage_slots = infer_only || h->stage_bytes > kStageRingMax ? 1 : 4 * h->stage_bytes <= kStageRingMax / 4 ? 4 : 2;
+  const size_t stage_total = h->stage_slots * h->stage_bytes;
+  VOLTA_CHECK(pinned_alloc((void**)&h->h_stage, stage_total + 256, hipHostMallocMapped | hipHostMallocCoherent));
+  h->stage_done = reinterpret_cast<uint32_t*>(h->h_stage + stage_total);
+  *h->stage_done = 0;
+  VOLTA_CHECK(hipEventCreateWithFlags(&h->stage_free, hipEventDisableTiming));
+  VOLTA_CHECK(pinned_alloc((void**)&h->h_lr, Handle::kLrSlots * sizeof(float), hipHostMallocDefault));
   for (auto& e : h->lr_ev) VOLTA_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
 
   // Reference init: LCG Xavier-uniform W from one stream seeded 42, b = 0.
@@ -1179,42 +1192,6 @@ static bool enqueue_forward(Handle* h, int rows, float* out, hipStream_t st) {
   return enqueue_forward_into(h, h->infer_plans, rows, h->infer_x, out, h->infer_ws, st);
 }
 
-// One chunk of host rows X [m x L0] into host out [m x Ln], synchronously.
-// Up to 1 MiB each way both cross through pinned memory that the GPU reads
-// (the input launch) and the output layer writes itself: a copy of pageable
-// memory each way took 16 of the 48 us of a one-row call of
-// 512-1024-1024-512-256-1.
-static bool infer_chunk(Handle* h, const float* X, int m, float* out) {
-  const size_t xb = (size_t)m * h->L[0] * sizeof(float), ob = (size_t)m * h->L[h->n] * sizeof(float);
-  constexpr size_t kMax = (size_t)1 << 20;
-  if (xb > kMax || ob > kMax) {
-    VOLTA_CHECK(hipMemcpyAsync(h->infer_x, X, xb, hipMemcpyHostToDevice, h->stream));
-    if (!enqueue_forward(h, m, h->act[h->n], h->stream)) return false;
-    VOLTA_CHECK(hipMemcpyAsync(out, h->act[h->n], ob, hipMemcpyDeviceToHost, h->stream));
-    VOLTA_CHECK(hipStreamSynchronize(h->stream));
-    return true;
-  }
-  const size_t out_off = align_up(xb, 256), need = out_off + ob;
-  if (need > h->infer_stage_bytes) {  // (the stream is idle between chunks)
-    if (h->infer_stage) VOLTA_CHECK(hipHostFree(h->infer_stage));
-    h->infer_stage = nullptr;
-    h->infer_stage_bytes = 0;
-    const size_t size = std::max(align_up(need, 4096), std::min(2 * need, 2 * kMax + 256));
-    VOLTA_CHECK(hipHostMalloc((void**)&h->infer_stage, size, hipHostMallocMapped | hipHostMallocCoherent));
-    h->infer_stage_bytes = size;
-  }
-  std::memcpy(h->infer_stage, X, xb);
-  InputCopy c;
-  c.x = reinterpret_cast<const uint32_t*>(h->infer_stage);
-  c.x_dst = reinterpret_cast<uint32_t*>(h->infer_x);
-  c.nx = xb / 4;
-  VOLTA_CHECK(launch_input_copy(c, h->stream));
-  if (!enqueue_forward(h, m, reinterpret_cast<float*>(h->infer_stage + out_off), h->stream)) return false;
-  VOLTA_CHECK(hipStreamSynchronize(h->stream));
-  std::memcpy(out, h->infer_stage + out_off, ob);
-  return true;
-}
-
 static void fail(Handle* h, int bits, const std::string& msg) {
   if (h) h->status |= bits;
   set_last_error(msg);
@@ -1247,8 +1224,12 @@ static bool launch_step(Handle* h) {
 // Wait until the device has read the staging slot of host-fed step `seq`.
 static bool stage_wait(Handle* h, uint32_t seq) {
   for (int spin = 0; (int32_t)(__atomic_load_n(h->stage_done, __ATOMIC_ACQUIRE) - seq) < 0; ++spin) {
-    if (spin % 4096 != 4095) continue;
-    // an idle stream has run every launch; an error ends the wait
+    __builtin_ia32_pause();
+    if (spin % 128 != 127) continue;
+    // an idle stream has run every launch; an error ends the wait (asked
+    // often: the runtime retires finished launches meanwhile, and with a
+    // query every 1024 pauses a 33.7 us step of 256-512-512-256-1 at B=64
+    // took 37.1)
     const hipError_t e = hipStreamQuery(h->stream);
     if (e == hipSuccess) return true;
     if (e != hipErrorNotReady) {
@@ -1259,15 +1240,21 @@ static bool stage_wait(Handle* h, uint32_t seq) {
   return true;
 }
 
-// The staging slots, on the handle's first host-fed step (a program whose
-// inputs are on the device never pins them).
-static bool stage_alloc(Handle* h) {
-  VOLTA_CHECK(hipEventCreateWithFlags(&h->stage_free, hipEventDisableTiming));
-  VOLTA_CHECK(hipHostMalloc((void**)&h->h_stage, h->stage_slots * h->stage_bytes + 256,
-                            hipHostMallocMapped | hipHostMallocCoherent));
-  h->stage_done = reinterpret_cast<uint32_t*>(h->h_stage + h->stage_slots * h->stage_bytes);
-  *h->stage_done = 0;
-  return true;
+// The next host-fed step's staging slot, once the device has read what it last
+// held (null: a device error), and on the ring that step's number, *seq, which
+// the launch that reads the slot reports.
+static char* stage_slot(Handle* h, uint32_t* seq) {
+  *seq = 0;
+  if (h->stage_slots == 1) {
+    const hipError_t e = hipEventSynchronize(h->stage_free);
+    if (e == hipSuccess) return h->h_stage;
+    set_last_error(hip_msg("hipEventSynchronize", e));
+    return nullptr;
+  }
+  *seq = h->stage_seq + 1;
+  // the slot's previous user, stage_slots steps ago
+  if (!stage_wait(h, *seq - (uint32_t)h->stage_slots)) return nullptr;
+  return h->h_stage + (*seq % (uint32_t)h->stage_slots) * h->stage_bytes;
 }
 
 static InputCopy input_copy(const Handle* h, const void* X, const void* Y, size_t ybytes) {
@@ -1283,31 +1270,56 @@ static InputCopy input_copy(const Handle* h, const void* X, const void* Y, size_
 
 // Stage host inputs through pinned memory so the caller may reuse X/Y at once.
 static bool stage_inputs(Handle* h, const float* X, const void* Y, size_t ybytes) {
-  const size_t xbytes = (size_t)h->B * h->L[0] * 4;
-  if (!h->h_stage && !stage_alloc(h)) return false;
-  if (h->stage_slots == 1) {
-    VOLTA_CHECK(hipEventSynchronize(h->stage_free));
-    std::memcpy(h->h_stage, X, xbytes);
-    std::memcpy(h->h_stage + h->stage_y_off, Y, ybytes);
-    // act_0 and the targets are adjacent in the arena as in the slot (the gap
-    // is copied too): one transfer
-    if (static_cast<char*>(h->target) != reinterpret_cast<char*>(h->act[0]) + h->stage_y_off) return false;
-    VOLTA_CHECK(hipMemcpyAsync(h->act[0], h->h_stage, h->stage_y_off + ybytes, hipMemcpyHostToDevice, h->stream));
-    VOLTA_CHECK(hipEventRecord(h->stage_free, h->stream));
+  uint32_t seq = 0;
+  char* slot = stage_slot(h, &seq);
+  if (!slot) return false;
+  std::memcpy(slot, X, (size_t)h->B * h->L[0] * 4);
+  std::memcpy(slot + h->stage_y_off, Y, ybytes);
+  if (h->stage_slots > 1) {
+    InputCopy c = input_copy(h, slot, slot + h->stage_y_off, ybytes);
+    c.done = h->stage_done;
+    c.seq = seq;
+    c.ticket = h->counters + h->n_counters;
+    VOLTA_CHECK(launch_input_copy(c, h->stream));
+    h->stage_seq = seq;
     return true;
   }
-  const uint32_t seq = h->stage_seq + 1;
-  // the slot's previous user, stage_slots steps ago
-  if (!stage_wait(h, seq - (uint32_t)h->stage_slots)) return false;
-  char* slot = h->h_stage + (seq % (uint32_t)h->stage_slots) * h->stage_bytes;
-  std::memcpy(slot, X, xbytes);
-  std::memcpy(slot + h->stage_y_off, Y, ybytes);
-  InputCopy c = input_copy(h, slot, slot + h->stage_y_off, ybytes);
-  c.done = h->stage_done;
-  c.seq = seq;
-  c.ticket = h->counters + h->n_counters;
+  // act_0 and the targets are adjacent in the arena as in the slot (the gap
+  // is copied too): one transfer
+  if (static_cast<char*>(h->target) != reinterpret_cast<char*>(h->act[0]) + h->stage_y_off) return false;
+  VOLTA_CHECK(hipMemcpyAsync(h->act[0], slot, h->stage_y_off + ybytes, hipMemcpyHostToDevice, h->stream));
+  VOLTA_CHECK(hipEventRecord(h->stage_free, h->stream));
+  return true;
+}
+
+// One chunk of host rows X [m x L0] into host out [m x Ln], synchronously.
+// Up to 1 MiB each way both cross through a staging slot that the GPU reads
+// (the input launch) and the output layer writes itself: a copy of pageable
+// memory each way took 16 of the 48 us of a one-row call of
+// 512-1024-1024-512-256-1.
+static bool infer_chunk(Handle* h, const float* X, int m, float* out) {
+  const size_t xb = (size_t)m * h->L[0] * sizeof(float), ob = (size_t)m * h->L[h->n] * sizeof(float);
+  constexpr size_t kMax = (size_t)1 << 20;
+  if (xb > kMax || ob > kMax) {
+    VOLTA_CHECK(hipMemcpyAsync(h->infer_x, X, xb, hipMemcpyHostToDevice, h->stream));
+    if (!enqueue_forward(h, m, h->act[h->n], h->stream)) return false;
+    VOLTA_CHECK(hipMemcpyAsync(out, h->act[h->n], ob, hipMemcpyDeviceToHost, h->stream));
+    VOLTA_CHECK(hipStreamSynchronize(h->stream));
+    return true;
+  }
+  uint32_t seq = 0;  // (not used up: the slot is free again before the call returns)
+  char* slot = stage_slot(h, &seq);  // (m <= B rows: X and the output rows fit its two parts)
+  if (!slot) return false;
+  std::memcpy(slot, X, xb);
+  InputCopy c;
+  c.x = reinterpret_cast<const uint32_t*>(slot);
+  c.x_dst = reinterpret_cast<uint32_t*>(h->infer_x);
+  c.nx = xb / 4;
   VOLTA_CHECK(launch_input_copy(c, h->stream));
-  h->stage_seq = seq;
+  const bool queued = enqueue_forward(h, m, reinterpret_cast<float*>(slot + h->stage_y_off), h->stream);
+  VOLTA_CHECK(hipStreamSynchronize(h->stream));  // the slot is free again, also where a launch failed
+  if (!queued) return false;
+  std::memcpy(out, slot + h->stage_y_off, ob);
   return true;
 }
 
@@ -1351,9 +1363,7 @@ using volta::set_last_error;
 
 static Handle* H(VoltaTrainHandle* h) { return reinterpret_cast<Handle*>(h); }
 
-extern "C" {
-
-VoltaTrainHandle* volta_train_init_spec(const volta_mlp_spec* spec, int32_t batch) {
+static VoltaTrainHandle* make_handle(const volta_mlp_spec* spec, int32_t batch, bool infer_only) {
   std::string why;
   if (!spec || !volta::validate_spec(*spec, &why)) {
     set_last_error("volta_train_init_spec: invalid spec: " + why);
@@ -1377,8 +1387,14 @@ VoltaTrainHandle* volta_train_init_spec(const volta_mlp_spec* spec, int32_t batc
   h->B = batch;
   h->n = spec->n_sizes - 1;
   h->L.assign(spec->sizes, spec->sizes + spec->n_sizes);
-  if (!volta::build(h.get())) return nullptr;
+  if (!volta::build(h.get(), infer_only)) return nullptr;
   return reinterpret_cast<VoltaTrainHandle*>(h.release());
+}
+
+extern "C" {
+
+VoltaTrainHandle* volta_train_init_spec(const volta_mlp_spec* spec, int32_t batch) {
+  return make_handle(spec, batch, false);
 }
 
 VoltaTrainHandle* volta_train_init(int32_t batch) {
@@ -1708,6 +1724,9 @@ int64_t volta_train_debug_buffer(VoltaTrainHandle* vh, int32_t kind, int32_t lay
   return (int64_t)count;
 }
 
+// Pinned host allocations made by the handles so far.  Test use.
+int64_t volta_hip_pinned_allocations(void) { return volta::g_pinned_allocs.load(); }
+
 // Bytes of the handle's device arena (reported by the benchmark).
 int64_t volta_hip_arena_bytes(VoltaTrainHandle* vh) {
   Handle* h = H(vh);
@@ -1936,7 +1955,7 @@ VoltaTrainHandle* volta_infer_model_create(int32_t n_sizes, const int32_t* sizes
   }
   volta_mlp_spec s;
   volta_mlp_spec_default(&s, n_sizes, sizes, VOLTA_ACT_RELU, VOLTA_OPT_SGD, VOLTA_LOSS_MSE);
-  VoltaTrainHandle* vh = volta_train_init_spec(&s, kInferModelChunk);
+  VoltaTrainHandle* vh = make_handle(&s, kInferModelChunk, true);
   if (!vh) return nullptr;
   Handle* h = H(vh);
   h->infer_linear = hidden_act == -1;
