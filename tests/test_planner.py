@@ -105,6 +105,22 @@ def test_small_batch_tiles():
     assert plan(TN, 512, 1024, 64, env={"VOLTA_DW_SMALLK_MAX_K": "0"})[0] == TILE_64
 
 
+def test_short_reduction_line():
+    """A product with K < 512 on at most half a 64x64 tile per CU takes 16x16
+    tiles at any batch; with K >= 256 and whole tiles across, only up to three
+    eighths of a tile per CU, where the split 64x64 grid catches up."""
+    for layout in (NN, NT):
+        assert plan(layout, 1024, 256, 256)[0] == TILE_SMALLM  # 64 tiles
+        assert plan(layout, 1024, 384, 384)[0] == TILE_SMALLM  # 96
+        assert plan(layout, 1600, 320, 320)[0] == TILE_64  # 125
+        assert plan(layout, 2048, 256, 256)[0] == TILE_64  # 128
+        assert plan(layout, 3500, 128, 384)[0] == TILE_64  # 110, a part of a tile down only
+        assert plan(layout, 1024, 400, 400)[0] == TILE_SMALLM  # 112, a part of a tile across
+        assert plan(layout, 4096, 128, 128)[0] == TILE_SMALLM  # 128, K < 256
+        assert plan(layout, 4096, 192, 128)[0] == TILE_64  # 192
+        assert plan(layout, 1024, 512, 512)[0] == TILE_64  # K >= 512
+
+
 def test_planner_rejects_bad_arguments():
     out = (C.c_int32 * 6)()
     lib = load_hip()

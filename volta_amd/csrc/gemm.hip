@@ -3392,12 +3392,19 @@ GemmPlan gemm_plan(int layout, int M, int N, int K, bool vec, int num_cus, bool 
   // Likewise a product of a short reduction whose 64x64 grid leaves half the
   // CUs idle: it is all start-up, and 16x16 tiles give each thread one output
   // to finish instead of 16.  Their operand re-reads (32 rows of K per tile)
-  // set the other bound.  13-397-250-101-7 at B=77 60.3 -> 34.0 us a step,
+  // set one bound: 13-397-250-101-7 at B=77 60.3 -> 34.0 us a step,
   // 130-23-110-19-10 at B=1 40.7 -> 25.8, 5-200-22-100 at B=2048 103.6 -> 82.8,
   // 200-500-500-10 at B=700 90 -> 80; past the bound 256-512-512-10 at B=1024
-  // (2048 tiles of K = 512) 94.7 -> 100.
+  // (2048 tiles of K = 512) 94.7 -> 100.  From K = 256 on the 64x64 grid is
+  // split in two, and with whole tiles across it catches up at three eighths of
+  // the CUs (64x64 against 16x16, us a step of w-w-w-w-10): 384 wide at B=1024
+  // (96 tiles) 122.4 and 120.9, 448 at B=896 (98) 125.5 and 130.5, 320 at
+  // B=1600 (125) 128.2 and 137.0, 256 at B=2048 (128) 121.0 and 122.8; with a
+  // part of a tile across, 400 at B=1024 (112) 133.3 and 126.3, 300 at B=1500
+  // (120) 125.2 and 124.0.
   const size_t tiles16 = (size_t)((M + 15) / 16) * ((N + 15) / 16);
-  const bool short_k = small_max > 0 && K < 512 && 2 * tiles <= num_cus && tiles16 * K <= (size_t)12 * 256 * num_cus;
+  const bool short_k = small_max > 0 && K < 512 && 2 * tiles <= num_cus && tiles16 * K <= (size_t)12 * 256 * num_cus &&
+                       (K < 256 || N % 64 != 0 || 8 * tiles <= 3 * num_cus);
   if (small_m && (layout == GEMM_NN || layout == GEMM_NT) && ((p.splits > 1 && M <= small_max && !nt_long) || short_k)) {
     p.tile = TILE_SMALLM;
     p.splits = 1;
