@@ -203,6 +203,22 @@ def test_runtime_optimizer_widths(kind, n):
             np.testing.assert_array_equal(d.numpy(), p)
 
 
+# Large states, on loads past the caches and, where a call writes more than
+# 352 MiB, on 4-byte accesses: bit for bit the oracle.
+@pytest.mark.parametrize("kind,count", [("adam", 26_000_003), ("adam", 31_500_001), ("adagrad", 47_000_001)])
+def test_runtime_optimizer_large(kind, count):
+    from volta_amd.backend import RtOptimizer, config
+
+    say(f"runtime optimizer {kind} count={count}")
+    rng = np.random.default_rng(count)
+    p, g = rng.standard_normal(count, np.float32), rng.standard_normal(count, np.float32)
+    dp, dg = DeviceArray(p), DeviceArray(g)
+    cfg = config(kind, 0.01, weight_decay=0.01)
+    RtOptimizer(load_hip().lib, [count]).apply(cfg, [dp.ptr], [dg.ptr])
+    RtOptimizer(load_oracle().lib, [count]).apply(cfg, [p.ctypes.data], [g.ctypes.data])
+    np.testing.assert_array_equal(dp.numpy(), p)
+
+
 # Host-fed inference through pinned memory, and above 1 MiB through copies:
 # the rows of one call agree with a training handle's forward on the oracle.
 @pytest.mark.parametrize("L0,Ln,rows", [(5, 3, 1), (300, 1, 873), (300, 1, 874), (16, 300, 873), (16, 300, 875), (7, 2, 2050)])

@@ -6,8 +6,9 @@
 // Layout: the tensors are cut into chunks of kRtChunk elements, one
 // workgroup per chunk (a host-built table maps workgroup -> tensor, chunk);
 // thread t of a chunk updates the chunk's float4 t where parameter and
-// gradient are 16-byte aligned and the chunk is whole, else elements t, t+256,
-// t+512, t+768, so every access of a wave is one contiguous run either way.
+// gradient are 16-byte aligned, the chunk is whole and the call's arrays are
+// not too large (at the kernel), else elements t, t+256, t+512, t+768, so every
+// access of a wave is one contiguous run either way.
 // Scalar loads are unconditional (index clamped to the tensor), stores are
 // guarded.  The optimizer state of each kind (Adam m/v, RMSprop v/buf, Adagrad
 // acc, LARS velocity) is one device arena over all tensors, allocated
@@ -70,6 +71,18 @@ struct RtArgs {
 
 __device__ __forceinline__ RtPtrs rt_ptrs(const RtArgs& a, int i) { return a.table ? a.table[i] : a.ptrs[i]; }
 
+// The same, chosen at compile time: scalar loads into scalar registers, where
+// the choice above is a flat load into vector registers.  The norm kernels
+// take this one (2 GiB of parameters and gradients: 322 us with the other,
+// 257 with this).  rt_apply_kernel keeps the other, whose later start suits
+// its streams better: SGD, 512 MiB on alternating states, 135 us against 156;
+// Adagrad, 2 GiB, 612 against 650.
+template <bool TABLE>
+__device__ __forceinline__ RtPtrs rt_ptrs_scalar(const RtArgs& a, int i) {
+  if constexpr (TABLE) return a.table[i];
+  else return a.ptrs[i];
+}
+
 // The update of one element, in the reference's expression order.
 template <int KIND, bool MOM>
 __device__ __forceinline__ void rt_elem(const RtArgs& a, float local_lr, float& p, float g, float& s0, float& s1) {
@@ -104,23 +117,36 @@ __device__ __forceinline__ void rt_elem(const RtArgs& a, float local_lr, float& 
   }
 }
 
+// How a call's arrays are read: 16-byte accesses through the caches, 16-byte
+// loads past them, or 4-byte accesses.
+enum RtAccess { RT_QUADS = 0, RT_QUADS_NT = 1, RT_WORDS = 2 };
+
 template <bool NT>
 __device__ __forceinline__ floatx4 rt_load4(const float* p) {
   if constexpr (NT) return __builtin_nontemporal_load(reinterpret_cast<const floatx4*>(p));
   else return *reinterpret_cast<const floatx4*>(p);
 }
 
-// HBM bound.  NT: the 16-byte loads bypass the caches, for a call whose
-// arrays together are well over the 256 MiB last-level cache: Adam over 25.2M
-// parameters (four arrays, 384 MiB) 147 -> 120 us a call, 5.9 TB/s.  Below
-// that the cache keeps what the next call reads: Adagrad over the same
-// parameters (288 MiB) 86 us without, 89 with; AdamW over 10.9M (167 MiB) 58
-// and 61.  The line between them is kRtNtBytes.  16-byte accesses, the
-// divisions by the bias corrections as multiplications and the pointers in
-// the arguments took SGD over 25.2M from 60 to 55 us and RMSprop over 6810
-// from 17.8 to 14.9.
-constexpr size_t kRtNtBytes = (size_t)336 << 20;
-template <int KIND, bool MOM, bool NT>
+// HBM bound.  Which access is the fastest depends on what the 256 MiB
+// last-level cache still holds of the state from the call before (us a call;
+// a state again and again / two states in turn / other work's 640 MiB between):
+//   up to kRtCacheBytes in all arrays, it serves the next call's reads: 16-byte
+//   accesses through the caches.  Adagrad, 288 MiB: 86 / 103 / 116 (4-byte
+//   accesses 92 / 106 / 118, past the caches 89 / 98 / 105).
+//   while what a call writes (all but the gradients) is at most kRtNtWritten,
+//   loads past the caches leave them to the writes: Adam, 384 MiB: 118 / 143 /
+//   145 (through them 140 / 142 / 151, 4-byte 139 / 144 / 152); Adagrad,
+//   448 MiB: 130 / 159 / 157 (4-byte 154 / 154 / 169).  SGD has one array of
+//   each and gains longer, up to kRtNtWrittenSgd: 640 MiB 165 / 174 / 189
+//   (4-byte 189 / 190 / 208).
+//   beyond, nothing stays and 4-byte accesses, four to a thread 1 KiB apart,
+//   keep the memory channels busiest: Adam, 1 GiB: 340 / 340 / 351 (16-byte
+//   past the caches 357 / 359 / 354, through them 355 / 362 / 363); Adagrad,
+//   2 GiB: 612 / 615 / 642 (678 / 679 / 670 and 659 / 661 / 671).
+constexpr size_t kRtCacheBytes = (size_t)336 << 20;
+constexpr size_t kRtNtWritten = (size_t)352 << 20;
+constexpr size_t kRtNtWrittenSgd = (size_t)512 << 20;
+template <int KIND, bool MOM, int ACC>
 __global__ void __launch_bounds__(kRtThreads) rt_apply_kernel(RtArgs a) {
   const int2 bt = a.blocks[blockIdx.x];
   const RtPtrs t = rt_ptrs(a, bt.x);
@@ -137,7 +163,9 @@ __global__ void __launch_bounds__(kRtThreads) rt_apply_kernel(RtArgs a) {
   float* const p0 = kS0 ? a.s0 + sh.off : nullptr;
   float* const p1 = kS1 ? a.s1 + sh.off : nullptr;
   const int64_t lo = (int64_t)bt.y * kRtChunk;
-  if (lo + kRtChunk <= sh.count && (((uintptr_t)t.p | (uintptr_t)t.g) & 15) == 0) {  // (the arenas are aligned)
+  constexpr bool NT = ACC == RT_QUADS_NT;
+  if (ACC != RT_WORDS && lo + kRtChunk <= sh.count &&
+      (((uintptr_t)t.p | (uintptr_t)t.g) & 15) == 0) {  // (the arenas are aligned)
     const int64_t i = lo + 4 * (int)threadIdx.x;
     floatx4 p = rt_load4<NT>(t.p + i);
     const floatx4 g = rt_load4<NT>(t.g + i);
@@ -194,13 +222,14 @@ __device__ __forceinline__ float2 block_sum2(float2 v, float2* sh) {
 }
 
 // LARS, stage 1: (sum p^2, sum g^2) of each chunk of a tensor with a gradient.
+template <bool TABLE>
 __global__ void __launch_bounds__(kRtThreads) rt_norm_partials(RtArgs a, float2* partials) {
   __shared__ float2 sh[kRtThreads];
   const int2 bt = a.blocks[blockIdx.x];
-  const RtPtrs t = rt_ptrs(a, bt.x);
+  const RtPtrs t = rt_ptrs_scalar<TABLE>(a, bt.x);
+  const int64_t last = a.shapes[bt.x].count - 1;
   if (!t.g) return;
   const int64_t base = (int64_t)bt.y * kRtChunk + threadIdx.x;
-  const int64_t last = a.shapes[bt.x].count - 1;
   float p[kRtPer], g[kRtPer];
 #pragma unroll
   for (int j = 0; j < kRtPer; ++j) {
@@ -221,11 +250,12 @@ __global__ void __launch_bounds__(kRtThreads) rt_norm_partials(RtArgs a, float2*
 
 // LARS, stage 2: one workgroup per tensor adds its chunks' partials (thread
 // t takes chunks t, t+256, ... in order, then the tree) and takes the roots.
+template <bool TABLE>
 __global__ void __launch_bounds__(kRtThreads) rt_norm_finish(RtArgs a, const int* first_block, const float2* partials,
                                                               float2* norms) {
   __shared__ float2 sh[kRtThreads];
   const int ti = blockIdx.x;
-  if (!rt_ptrs(a, ti).g) return;
+  if (!rt_ptrs_scalar<TABLE>(a, ti).g) return;
   const int b0 = first_block[ti], b1 = first_block[ti + 1];
   float2 s = make_float2(0.0f, 0.0f);
   for (int b = b0 + (int)threadIdx.x; b < b1; b += kRtThreads) {
@@ -397,11 +427,22 @@ int validate(VoltaRtOptimizer* h, const volta_rt_config& c, RtArgs& a) {
 
 template <int KIND, bool MOM>
 void launch_apply(VoltaRtOptimizer* h, const RtArgs& a) {
-  const int arrays = 2 + (a.s0 ? 1 : 0) + (a.s1 ? 1 : 0);
-  if ((size_t)h->total * arrays * sizeof(float) > kRtNtBytes)
-    hipLaunchKernelGGL((rt_apply_kernel<KIND, MOM, true>), dim3(h->nblocks), dim3(kRtThreads), 0, h->stream, a);
+  const size_t array = (size_t)h->total * sizeof(float);
+  const int arrays = 2 + (a.s0 ? 1 : 0) + (a.s1 ? 1 : 0);  // all but the gradient are written too
+  const dim3 grid(h->nblocks), block(kRtThreads);
+  if (arrays * array <= kRtCacheBytes)
+    hipLaunchKernelGGL((rt_apply_kernel<KIND, MOM, RT_QUADS>), grid, block, 0, h->stream, a);
+  else if ((arrays - 1) * array <= (a.s0 ? kRtNtWritten : kRtNtWrittenSgd))
+    hipLaunchKernelGGL((rt_apply_kernel<KIND, MOM, RT_QUADS_NT>), grid, block, 0, h->stream, a);
   else
-    hipLaunchKernelGGL((rt_apply_kernel<KIND, MOM, false>), dim3(h->nblocks), dim3(kRtThreads), 0, h->stream, a);
+    hipLaunchKernelGGL((rt_apply_kernel<KIND, MOM, RT_WORDS>), grid, block, 0, h->stream, a);
+}
+
+template <bool TABLE>
+void launch_norms(VoltaRtOptimizer* h, const RtArgs& a) {
+  hipLaunchKernelGGL(rt_norm_partials<TABLE>, dim3(h->nblocks), dim3(kRtThreads), 0, h->stream, a, h->partials);
+  hipLaunchKernelGGL(rt_norm_finish<TABLE>, dim3(h->n), dim3(kRtThreads), 0, h->stream, a, h->first_block, h->partials,
+                     h->norms);
 }
 
 }  // namespace
@@ -509,9 +550,8 @@ int32_t volta_rt_apply_gradients(VoltaRtOptimizer* h, const volta_rt_config* cfg
     if (!h->partials && (!ok(hipMalloc((void**)&h->partials, (size_t)h->nblocks * sizeof(float2)), "volta_rt: LARS") ||
                          !ok(hipMalloc((void**)&h->norms, (size_t)h->n * sizeof(float2)), "volta_rt: LARS")))
       return -1;
-    hipLaunchKernelGGL(rt_norm_partials, dim3(h->nblocks), dim3(kRtThreads), 0, h->stream, a, h->partials);
-    hipLaunchKernelGGL(rt_norm_finish, dim3(h->n), dim3(kRtThreads), 0, h->stream, a, h->first_block, h->partials,
-                       h->norms);
+    if (a.table) launch_norms<true>(h, a);
+    else launch_norms<false>(h, a);
     a.norms = h->norms;
   }
   switch (kind) {
