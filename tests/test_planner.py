@@ -121,6 +121,19 @@ def test_short_reduction_line():
         assert plan(layout, 1024, 512, 512)[0] == TILE_64  # K >= 512
 
 
+def test_smallm_max_m_bounds_every_small_m_product():
+    """VOLTA_SMALLM_MAX_M is the largest batch on the small-M tile, short
+    reductions included."""
+    limit = lambda m: {"VOLTA_SMALLM_MAX_M": str(m)}  # noqa: E731
+    for layout in (NN, NT):
+        assert plan(layout, 700, 200, 500)[0] == TILE_SMALLM
+        assert plan(layout, 700, 200, 500, env=limit(256))[0] == TILE_64
+        assert plan(layout, 700, 200, 500, env=limit(700))[0] == TILE_SMALLM
+        assert plan(layout, 64, 100, 100, env=limit(64))[0] == TILE_SMALLM
+        assert plan(layout, 65, 100, 100, env=limit(64))[0] == TILE_64
+        assert plan(layout, 1, 100, 100, env=limit(0))[0] == TILE_64
+
+
 def test_planner_rejects_bad_arguments():
     out = (C.c_int32 * 6)()
     lib = load_hip()

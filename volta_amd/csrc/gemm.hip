@@ -3356,6 +3356,8 @@ GemmPlan gemm_plan(int layout, int M, int N, int K, bool vec, int num_cus, bool 
   // 64 for every forward product split C4 B=1024's fwd3 (1024 x 256, K =
   // 512, 64 tiles) eight ways instead of four: 0.2398 -> 0.2380 ms/step with
   // 128, the reduce reading half the planes.
+  // VOLTA_SMALLM_MAX_M: largest batch on the small-M tile, 0 for none (unset:
+  // 256 for a product that would split K, any batch for a short reduction)
   const char* sm = std::getenv("VOLTA_SMALLM_MAX_M");
   const int small_max = sm && *sm ? std::atoi(sm) : 256;
   const char* mk = std::getenv("VOLTA_SPLITK_MIN_K");
@@ -3377,8 +3379,7 @@ GemmPlan gemm_plan(int layout, int M, int N, int K, bool vec, int num_cus, bool 
   p.k_per_split = kps;
   // A product the 64x64 plan would split over K runs on the small-M tile
   // instead when it has few rows: the reduction over K stays inside each
-  // workgroup, which saves the reduce launch (B <= 256 by default;
-  // VOLTA_SMALLM_MAX_M changes the limit, 0 turns the tile off).  Measured
+  // workgroup, which saves the reduce launch (B <= 256).  Measured
   // with the small-K dW tile below: C4 B=256 0.1624 -> 0.1415 ms/step; at
   // B=1024 both tiles are slower than the 64x64 family (0.45 vs 0.30 ms).
   // ... except a dX product (NT) with a long reduction: there the 16x16
@@ -3403,7 +3404,7 @@ GemmPlan gemm_plan(int layout, int M, int N, int K, bool vec, int num_cus, bool 
   // part of a tile across, 400 at B=1024 (112) 133.3 and 126.3, 300 at B=1500
   // (120) 125.2 and 124.0.
   const size_t tiles16 = (size_t)((M + 15) / 16) * ((N + 15) / 16);
-  const bool short_k = small_max > 0 && K < 512 && 2 * tiles <= num_cus && tiles16 * K <= (size_t)12 * 256 * num_cus &&
+  const bool short_k = !(sm && *sm && M > small_max) && K < 512 && 2 * tiles <= num_cus && tiles16 * K <= (size_t)12 * 256 * num_cus &&
                        (K < 256 || N % 64 != 0 || 8 * tiles <= 3 * num_cus);
   if (small_m && (layout == GEMM_NN || layout == GEMM_NT) && ((p.splits > 1 && M <= small_max && !nt_long) || short_k)) {
     p.tile = TILE_SMALLM;
