@@ -9,6 +9,7 @@ import pytest
 
 from tests.oracle_lib import load_oracle
 from tests.test_gpu_parity import _launch_labels, assert_params_close, close_enough, run_steps, say
+from tests.test_planner import forms
 from volta_amd import DeviceArray, data, load_hip
 from volta_amd.abi import STATUS_BAD_ARGUMENT, STATUS_NONFINITE_LOSS, MlpSpec, Trainer
 
@@ -245,23 +246,29 @@ def test_host_inference(L0, Ln, rows):
                                      ([63, 130, 1, 9, 2], 17), ([257, 18, 515, 3], 256), ([70, 1025, 34, 1], 130),
                                      ([13, 397, 250, 101, 7], 77), ([301, 703, 66, 2], 300), ([530, 1030, 67], 515),
                                      ([2, 771, 3, 770, 5], 641)])
-@pytest.mark.parametrize("opt", ["sgd", "adam"])
+@pytest.mark.parametrize("opt", ["sgd", "adam", "adamw", "adagrad"])
 def test_ragged_layers(sizes, B, opt):
-    """Adam divides each gradient by its own size, so a gradient of rounding
-    size moves a weight by up to lr either way: lr is small enough that three
-    such steps stay under the absolute tolerance."""
     say(f"ragged layers {sizes} B={B} {opt}")
-    against_oracle(MlpSpec(sizes, "tanh", opt), B, lr=0.02 if opt == "sgd" else 3e-6)
+    spec = MlpSpec(sizes, "tanh", opt)
+    if opt == "sgd":
+        against_oracle(spec, B, lr=0.02)
+    else:
+        resumed_against_oracle(spec, B)
 
 
 # The 128x64 direct-to-LDS tile (a grid of a tile per CU, sizes of any
 # multiple): integer operands are exact in every order; last stages of 1 to 32
 # k, 16- and 4-byte loads.
-@pytest.mark.parametrize("M,N,K", [(2048, 1024, 128), (1925, 1003, 131), (2044, 1020, 160), (1921, 961, 161),
-                                   (1001, 1985, 255)])
-@pytest.mark.parametrize("layout", [0, 1, 2])
+@pytest.mark.parametrize("layout,M,N,K", [(layout, *s) for layout in (0, 1) for s in (
+    (2048, 1024, 128), (1925, 1003, 131), (2044, 1020, 160), (1921, 961, 161), (1001, 1985, 255), (1900, 1050, 289))] +
+    # (a dW with K <= 256 is the small-K tile's)
+    [(2, *s) for s in ((2048, 1024, 288), (1925, 1003, 257), (2044, 1020, 321), (1921, 961, 319), (1001, 1985, 300),
+                       (1900, 1050, 289), (1896, 1048, 320))])
 def test_mid_tile_integer_exact(M, N, K, layout):
+    """Grids of 256 and of 255 tiles (the tile order over the XCDs with a remainder)."""
     say(f"mid tile {M}x{N}x{K} layout {layout}")
+    contig = (M if layout == 2 else K, K if layout == 1 else N)
+    assert forms(layout, M, N, K, vec=all(c % 4 == 0 for c in contig)) == (True, False)
     rng = np.random.default_rng(M + layout)
     A = rng.integers(-4, 5, (M, K)).astype(np.float32)
     B = rng.integers(-4, 5, (K, N)).astype(np.float32)
@@ -278,6 +285,15 @@ def test_mid_tile_step(sizes, B, act):
     """Its three epilogues in a training step (products of 256 and 512 tiles)."""
     say(f"mid tile step {sizes} B={B}")
     against_oracle(MlpSpec(sizes, act, "sgd"), B, lr=0.02, steps=2)
+
+
+@pytest.mark.parametrize("sizes,opt", [([132, 1992, 1004, 2], "adamw"), ([131, 1990, 1001, 3], "adam"),
+                                       ([131, 1990, 1001, 3], "adagrad")])
+def test_mid_tile_optimizers(sizes, opt):
+    """Its dW epilogue on a resumed optimizer state."""
+    say(f"mid tile optimizers {sizes} {opt}")
+    assert forms(2, *sizes[1:3], 2000, vec=sizes[1] % 4 == 0)[0]
+    resumed_against_oracle(MlpSpec(sizes, "tanh", opt), 2000, steps=2)
 
 
 # The codegen extras' backward launch (rows beside 64-column blocks) and the

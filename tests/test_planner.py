@@ -34,6 +34,13 @@ def plan(layout, M, N, K, vec=True, small_m=True, env=None):
                 os.environ[k] = v
 
 
+def forms(layout, M, N, K, vec=True, small_m=True):
+    """(mid, ragged) of the plan."""
+    out = (C.c_int32 * 2)()
+    assert load_hip().lib.volta_hip_gemm_plan_forms(layout, M, N, K, int(vec), CUS, int(small_m), out) == 0
+    return tuple(bool(x) for x in out)
+
+
 def test_big_tile_for_full_grids_of_256_multiples():
     """C5's 4096-wide products: 256x256 tiles, one per CU, whole K."""
     assert plan(NN, 4096, 4096, 4096) == (TILE_BIG, 1, 4096, 1, 0)
@@ -134,9 +141,35 @@ def test_smallm_max_m_bounds_every_small_m_product():
         assert plan(layout, 1, 100, 100, env=limit(0))[0] == TILE_64
 
 
+def test_mid_tile_rule():
+    """128x64 direct-to-LDS tiles for products of any multiple from about a
+    tile per CU on, where the last round of tiles is filled well enough; not
+    where another tile is exact, and never a dW of the small-K tile."""
+    assert forms(NN, 2000, 3000, 3000) == (True, False)  # 752 tiles
+    assert forms(TN, 1500, 3000, 2000) == (True, False)  # 564
+    assert forms(NT, 2000, 1000, 3000, vec=False) == (True, False)  # 256
+    assert not forms(TN, 3000, 1000, 2000)[0]  # 384 tiles: 0.75 against 64x64 tiles
+    assert not forms(NN, 2000, 1203, 801)[0]  # 304 tiles: 0.59
+    assert not forms(NN, 1024, 1024, 1024)[0]  # 128 tiles
+    assert not forms(NN, 2048, 1024, 127)[0]  # K < 128
+    assert not forms(NN, 4096, 4096, 4096)[0] and plan(NN, 4096, 4096, 4096)[0] == TILE_BIG
+    assert not forms(TN, 2048, 1024, 256)[0] and plan(TN, 2048, 1024, 256)[0] == TILE_DW_SMALLK
+    assert not forms(NN, 2000, 3000, 3000, small_m=False)[0]
+
+
+def test_ragged_small_k_dw():
+    """The small-K dW tile's rows that may not be 16-byte aligned."""
+    assert forms(TN, 512, 1024, 64) == (False, False)
+    for shape in ((511, 1024, 64), (512, 10, 64), (512, 1022, 64)):
+        assert forms(TN, *shape) == (False, True) and plan(TN, *shape)[0] == TILE_DW_SMALLK
+    assert forms(TN, 512, 1024, 64, vec=False) == (False, True)
+    assert plan(TN, 512, 1, 64)[0] == TILE_64  # one column: narrow_dw_kernel's
+
+
 def test_planner_rejects_bad_arguments():
     out = (C.c_int32 * 6)()
     lib = load_hip()
+    assert lib.lib.volta_hip_gemm_plan_forms(TN, 64, 0, 64, 1, CUS, 1, out) == -1
     assert lib.lib.volta_hip_gemm_plan(7, 64, 64, 64, 1, CUS, 1, out) == -1
     assert lib.lib.volta_hip_gemm_plan(NN, 0, 64, 64, 1, CUS, 1, out) == -1
     assert "volta_hip_gemm_plan" in lib.last_error()

@@ -33,10 +33,6 @@ int32_t volta_hip_calibration_copy(void* dst, const void* src, int64_t bytes, in
   return hipGetLastError() == hipSuccess && hipDeviceSynchronize() == hipSuccess ? 0 : -1;
 }
 
-// C[M x N] = op(A) op(B) for layout GEMM_NN / GEMM_NT / GEMM_TN (see gemm.h).
-// force_tile < 0 and force_splits == 0 select the runtime's own plan;
-// force_splits > 0 splits K over that many launch slices (reduced by a
-// second kernel), force_splits = -G over G groups of one workgroup's waves.
 // The planner's choice for one product (gemm_plan; host code only, no
 // device call): out[0..5] = tile (GemmTile), splits, k_per_split, kgroups,
 // waves, vec.  `small_m` as the step passes it (0 for the loss-head
@@ -57,6 +53,26 @@ int32_t volta_hip_gemm_plan(int32_t layout, int32_t M, int32_t N, int32_t K, int
   out[5] = p.vec ? 1 : 0;
   return 0;
 }
+
+// The same choice's forms: out[0] = mid (run as 128x64 direct-to-LDS tiles),
+// out[1] = ragged (TILE_DW_SMALLK: rows that may not be 16-byte aligned).
+int32_t volta_hip_gemm_plan_forms(int32_t layout, int32_t M, int32_t N, int32_t K, int32_t vec, int32_t num_cus,
+                                  int32_t small_m, int32_t* out) {
+  using namespace volta;
+  if (layout < GEMM_NN || layout > GEMM_TN || M <= 0 || N <= 0 || K <= 0 || num_cus <= 0 || !out) {
+    set_last_error("volta_hip_gemm_plan_forms: bad arguments");
+    return -1;
+  }
+  const GemmPlan p = gemm_plan(layout, M, N, K, vec != 0, num_cus, small_m != 0);
+  out[0] = p.mid ? 1 : 0;
+  out[1] = p.ragged ? 1 : 0;
+  return 0;
+}
+
+// C[M x N] = op(A) op(B) for layout GEMM_NN / GEMM_NT / GEMM_TN (see gemm.h).
+// force_tile < 0 and force_splits == 0 select the runtime's own plan;
+// force_splits > 0 splits K over that many launch slices (reduced by a
+// second kernel), force_splits = -G over G groups of one workgroup's waves.
 
 int32_t volta_hip_gemm(int32_t layout, const float* A, const float* B, float* Cm, int32_t M, int32_t N,
                        int32_t K, int32_t force_tile, int32_t force_splits) {
