@@ -21,7 +21,7 @@ batch.  Then (tests/grad_check.py, check_step_ext):
     gamma/beta equal, bit for bit, the oracle's optimizer (and LayerNorm's
     SGD step) applied to the HIP step's own gradients.
 The last pins the wiring only the extras path uses -- the bias update from
-the unclipped deltas under clipping (bias_update_kernel) and the phase-2
+the unclipped deltas under clipping (extras_tail_kernel) and the phase-2
 dW launches without a bias -- in magnitude, not only in sign.
 """
 import os
