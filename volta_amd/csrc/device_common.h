@@ -161,23 +161,10 @@ __device__ __forceinline__ void adagrad_elem(float* w, float* G, float g, float 
 // Once per step, after the loss: record it, raise the non-finite flag, and
 // advance the Adam step counter and its bias corrections 1 - beta^t, read
 // from a table the host filled with the same f32 powf the reference calls
-// (mlp_train_rust_codegen.rs:803-811).  Single thread.
-__device__ __forceinline__ void step_epilogue(DevScalars* sc, const float2* bc_table, int bc_len, float loss) {
-  sc->loss = loss;
-  if (!(fabsf(loss) <= 3.402823466e38f)) atomicOr(&sc->flags, (uint32_t)VOLTA_STATUS_NONFINITE_LOSS);
-  if (bc_table) {
-    const uint32_t t = sc->t + 1u;
-    sc->t = t;
-    const float2 bc = bc_table[t < (uint32_t)bc_len ? t : (uint32_t)(bc_len - 1)];
-    sc->bc1 = bc.x;
-    sc->bc2 = bc.y;
-  }
-}
-
-// step_epilogue split in two so its loads (step counter, then the table
-// entry) overlap the kernel's main work: step_prefetch at kernel start,
-// step_finish at the end (same stores as step_epilogue).  Single thread;
-// nothing else may change the counter in between.
+// (mlp_train_rust_codegen.rs:803-811).  In two parts, so its loads (step
+// counter, then the table entry) overlap the kernel's main work: step_prefetch
+// at kernel start, step_finish at the end.  Single thread; nothing else may
+// change the counter in between.
 struct StepNext {
   uint32_t t;
   float2 bc;

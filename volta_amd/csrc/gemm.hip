@@ -3052,7 +3052,7 @@ struct NarrowDwOp {  // staged delta in the launch's LDS
   using Args = NarrowDwArgs;
   static constexpr int kLds = 0;
   static __device__ __forceinline__ void run(const NarrowDwArgs& p, int blk, float* lds) {
-    narrow_dw_block<1>(p, blk, lds);
+    narrow_dw_block(p, blk, lds);
   }
 };
 
@@ -3138,7 +3138,7 @@ bool pair_supported(const PairOp& a, const PairOp& b) {
   if (a_dx && a.plan.tile != TILE_SMALLM && b_small) return false;
   if (a.kind == PAIR_GEMM && !a_dx && (a.plan.tile == TILE_DW_SMALLK) != b_small) return false;
   for (const PairOp* o : ops)  // the narrow dW stages its deltas and partial sums in the GEMM's LDS
-    if (o->kind == PAIR_NARROW_DW && narrow_lds_floats_n(o->nd.B, o->nd.N) > lds) return false;
+    if (o->kind == PAIR_NARROW_DW && narrow_lds_floats(o->nd.B) > lds) return false;
   // no split product in the pair may share the other's workspace
   if (a.kind == PAIR_GEMM && b.kind == PAIR_GEMM && a.plan.splits > 1 && b.plan.splits > 1 &&
       a.args.partial == b.args.partial)
@@ -3185,7 +3185,7 @@ dw_group_kernel(DwGroup d) {
   if (b == 0 && threadIdx.x == 0 && d.loss_partials)
     deferred_loss_finish(d.loss_scalars, d.loss_partials, d.loss_blocks, d.loss_denom);
   if (b < d.narrow_blocks) {
-    narrow_dw_block<1, true>(d.nd, b, lds);
+    narrow_dw_block<true>(d.nd, b, lds);
     return;
   }
   b -= d.narrow_blocks;
@@ -3254,7 +3254,7 @@ bool dw_group_supported(const DwGroup& d) {
   }
   if (d.narrow_blocks) {
     const NarrowDwArgs& p = d.nd;
-    if (p.N != 1 || p.B < 1 || p.B > kNarrowMaxB || narrow_lds_floats_n(p.B, p.N) > kDwLds) return false;
+    if (p.N != 1 || p.B < 1 || p.B > kNarrowMaxB || narrow_lds_floats(p.B) > kDwLds) return false;
     if (p.opt != VOLTA_OPT_SGD && p.opt != VOLTA_OPT_ADAM && p.opt != VOLTA_OPT_ADAGRAD) return false;
     if (d.narrow_blocks != (p.R + kNarrowRows - 1) / kNarrowRows) return false;
   }

@@ -429,7 +429,7 @@ outer_dx_kernel(const float* __restrict__ delta, const float* __restrict__ W, in
 // Stand-alone launch: 64 rows of W per block.
 __global__ void __launch_bounds__(kNarrowThreads) narrow_dw_kernel(NarrowDwArgs p) {
   extern __shared__ float lds[];
-  narrow_dw_block<1>(p, blockIdx.x, lds);
+  narrow_dw_block(p, blockIdx.x, lds);
 }
 
 // ---------------------------------------------------------------------------
@@ -468,7 +468,7 @@ hipError_t launch_narrow_dw(const NarrowDwArgs& p, hipStream_t st) {
   if (p.N != 1 || p.B < 1 || p.B > kNarrowMaxB) return hipErrorInvalidValue;
   if (p.opt != VOLTA_OPT_SGD && p.opt != VOLTA_OPT_ADAM && p.opt != VOLTA_OPT_ADAGRAD) return hipErrorInvalidValue;
   const int blocks = (p.R + kNarrowRows - 1) / kNarrowRows;
-  hipLaunchKernelGGL(narrow_dw_kernel, dim3(blocks), dim3(kNarrowThreads), narrow_lds_floats<1>(p.B, p.N) * 4, st, p);
+  hipLaunchKernelGGL(narrow_dw_kernel, dim3(blocks), dim3(kNarrowThreads), narrow_lds_floats(p.B) * 4, st, p);
   return hipGetLastError();
 }
 
