@@ -65,8 +65,9 @@ def test_dominant_launch_is_the_longest_measured():
 
 def test_per_launch_splits_whole_steps():
     """A primary workload of 3 launches and a secondary of 2 (its first a
-    large-tile kernel), each run for whole steps after a warm-up fragment:
-    values are grouped per step position from the end of each region."""
+    large-tile kernel), each run for whole steps after a warm-up fragment and
+    followed by host-fed steps, whose input launches are no launch of the
+    step: values are grouped per step position from the end of each region."""
     def row(i, name, v):
         return {"Dispatch_Id": str(i), "Kernel_Name": f"void volta::{name}(args)", "Grid_Size_X": "256",
                 "Workgroup_Size_X": "64", "Grid_Size_Y": "1", "v": v}
@@ -74,7 +75,9 @@ def test_per_launch_splits_whole_steps():
     seq = [("gemm_smallm<1>", 9.0)]  # a leftover fragment before the whole steps
     for s in range(3):
         seq += [("gemm_smallm<1>", 1.0 + s), ("out_layer_dx_kernel<1>", 2.0), ("dw_group_kernel<1>", 3.0)]
+        seq += [("input_copy_kernel<1>", 7.0)] if s else []
     for s in range(2):
+        seq += [("input_copy_kernel<4>", 8.0)] if s else []
         seq += [("gemm_big<true>", 10.0 + s), ("splitk_reduce<1>", 1.5)]
     rows = [row(i, n, v) for i, (n, v) in enumerate(seq)]
     labels = {"c2": ["fwd0", "fwd1+loss", "dw"], "c5": ["fwd0", "fwd0.splitk_reduce"]}
