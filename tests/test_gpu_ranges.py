@@ -173,6 +173,22 @@ def test_output_strips(loss, K, N, B, extras):
     against_oracle(MlpSpec([8, K, N], "tanh", "sgd", loss, **kw), B)
 
 
+# Its route: strips, or for 17 to 64 columns and a long K (more than 192 k a
+# wave up to 256 rows, from 512 on up to 1024) the product and a loss launch, at
+# both sides of each bound.
+@pytest.mark.parametrize("loss,K,N,B,strips", [
+    ("ce", 1543, 17, 33, True), ("ce", 1544, 17, 33, False), ("mse", 1545, 32, 1, False), ("ce", 771, 33, 256, True),
+    ("ce", 772, 33, 256, False), ("mse", 4096, 64, 16, False), ("ce", 2047, 33, 257, True), ("ce", 2048, 64, 257, False),
+    ("mse", 2049, 40, 1024, False), ("ce", 2049, 40, 1025, True), ("ce", 4096, 16, 64, True), ("mse", 2050, 16, 300, True)])
+def test_output_layer_route(loss, K, N, B, strips):
+    say(f"output layer route {loss} K={K} N={N} B={B}")
+    spec = MlpSpec([8, K, N], "tanh", "sgd", loss)
+    labels = _launch_labels({}, spec, B)
+    assert any(x.startswith("fwd1+loss") for x in labels) == strips, labels
+    assert ("loss" in labels) == (not strips), labels
+    against_oracle(spec, B, steps=2)
+
+
 # The runtime optimizer's two access widths (whole and partial chunks, aligned
 # and misaligned tensors) and its two ways of passing pointers (64 tensors in
 # the arguments, more in a table): bit for bit the oracle, as its other tests.

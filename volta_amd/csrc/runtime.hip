@@ -15,9 +15,10 @@
 //                               small-batch product on few CUs over two halves
 //                               of K into two planes, which the next forward
 //                               launch adds with the bias and activation
-//   fwd_{n-1} + loss            16-row MFMA strips with the loss head (L_n <= 64;
-//                               one column of a small batch as wave dot
-//                               products), or GEMM + loss kernel: delta_{n-1},
+//   fwd_{n-1} + loss            16-row MFMA strips with the loss head (L_n <= 64
+//                               unless K is long; one column of a small batch
+//                               as wave dot products), or GEMM + loss kernel:
+//                               delta_{n-1},
 //                               loss, Adam t
 //   dX_{n-1}                    outer product (L_n <= 16) or GEMM NT; merged
 //                               into the output launch where that is narrow
@@ -65,7 +66,7 @@ namespace volta {
 enum OutMode {
   OUT_COLUMN = 0,  // L[n] == 1, small batch: wave dot products + loss head
   OUT_STRIP = 1,   // L[n] <= 64: 16-row MFMA strips + loss head (out_strip_kernel)
-  OUT_GEMM = 2,    // wider: MFMA GEMM, then a stand-alone loss kernel
+  OUT_GEMM = 2,    // wider, or a long K: MFMA GEMM, then a stand-alone loss kernel
 };
 
 static std::string hip_msg(const char* what, hipError_t e) {
@@ -923,10 +924,20 @@ static bool build(Handle* h, bool infer_only) {
   // one block runs all rows, up to 32k activations (512-1024-1024-512-256-1
   // with LayerNorm at B=64: 111.3 us a step, 112.0 on strips).  Every other
   // layer of up to 64 columns runs on strips, whose loss and deltas take one
-  // launch (measured there).
+  // launch (measured there), but for more than 16 columns and a long K: a strip
+  // is one workgroup whatever K is, and its 16 waves divide K by 8 or 4 only.
+  // There the product on its own tiles and a loss launch are faster, from more
+  // than 192 k a wave on at a small batch (us a step of 64-K-N CE SGD, strips
+  // and that: K=1024 N=64 B=64 29.3 and 23.5, K=4096 N=64 B=64 64.0 and 37.0,
+  // K=4096 N=17 B=256 63.6 and 56.2, K=2000 N=20 B=100 34.9 and 33.4; K=1032
+  // N=20 B=16 24.0 and 26.2), from 512 on up to 64 strips (K=4096 N=64 B=512
+  // 89.9 and 71.0, K=2048 N=33 B=1024 85.3 and 80.4, N=32 60.2 and 63.9), and not
+  // with more strips (K=4096 N=33 B=4096 220.1 and 227.2).
   const bool column = Ln == 1 && B <= kNarrowMaxB && n > 1 &&
                       (!h->extras() || (int64_t)B * h->L[n - 1] <= 32768);
-  h->out_mode = column ? OUT_COLUMN : Ln <= kOutStripMaxN ? OUT_STRIP : OUT_GEMM;
+  const int wave_k = h->L[n - 1] * (Ln <= 32 ? 2 : 4) / 16;  // of a strip of 17 to 64 columns
+  const bool long_k = Ln > 16 && (B <= kNarrowMaxB ? wave_k > 192 : out_strip_blocks(B) <= 64 && wave_k >= 512);
+  h->out_mode = column ? OUT_COLUMN : Ln <= kOutStripMaxN && !long_k ? OUT_STRIP : OUT_GEMM;
   h->narrow_dx = Ln <= 16 && n > 1;
   const char* nod = std::getenv("VOLTA_NO_OUT_DX");
   h->out_dx_merged = h->narrow_dx && !h->extras() && !(nod && *nod && *nod != '0') && B <= kNarrowMaxB;
